@@ -1,5 +1,5 @@
 // Register-resident FP32 dX chain of the reference topology (W = 256 with the
-// rgb branch): the backward twin of mlp_fwd_f32r.h.
+// rgb branch), register-resident.
 //
 // A wave owns 16 samples and walks the layers top-down on
 // v_mfma_f32_16x16x4f32.  dh_{l-1} = W_l[:W] dz_l: the output blocks are the 16
@@ -16,9 +16,47 @@
 //   sigma = relu(z):   dz_sigma = d_sigma * [sigma > 0]
 //   dz = dh * [h > 0] for the ReLU layers; the bottleneck is linear.
 #pragma once
-#include "mlp_fwd_f32r.h"
+#include "mlp_kernels.h"
+#include "mlp_fwd_bf16ws.h"  // ws::packed_rsrc, ws::ldf4, ws::static_for
 
 namespace f32r {
+
+constexpr int kWaves = 4;  // waves per workgroup (64 samples)
+
+__device__ __forceinline__ floatx4 mfma16(float a, float b, floatx4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// acc[0 .. NBO) = sum over the NG k-step groups of A * act.  Step u runs group u / 2
+// on output blocks (u % 2) * NBO/2 .. + NBO/2 - 1; the weights of step u + 1 are loaded at the
+// start of step u.  The loads are unconditional, so every wait counts only the
+// loads of its own step.
+template <int NBO, int NG>
+__device__ __forceinline__ void layer(floatx4 (&acc)[16], const floatx4 (&act)[16], __amdgpu_buffer_rsrc_t rs,
+                                      uint32_t lane_off, int64_t p_layer) {
+  constexpr int HB = NBO / 2;
+  floatx4 w[2][HB];
+  auto load_step = [&](int u, floatx4 (&dst)[HB]) {
+    const int grp = u >> 1, h = u & 1;
+#pragma unroll
+    for (int i = 0; i < HB; ++i) dst[i] = ws::ldf4(rs, lane_off, p_layer + (int64_t)(grp * NBO + h * HB + i) * 1024);
+  };
+  load_step(0, w[0]);
+  const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+  ws::static_for<0, 2 * NG>([&](auto U) {
+    constexpr int u = decltype(U)::value;
+    constexpr int grp = u >> 1, h = u & 1;
+    if constexpr (u + 1 < 2 * NG) load_step(u + 1, w[(u + 1) & 1]);
+    const floatx4 bv = act[grp];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int i = 0; i < HB; ++i)
+        acc[h * HB + i] = mfma16(w[u & 1][i][r], bv[r], (grp == 0 && r == 0) ? zero : acc[h * HB + i]);
+    __builtin_amdgcn_sched_barrier(0);
+  });
+}
+
 
 __device__ __forceinline__ void store_f4(const floatx4& v, __amdgpu_buffer_rsrc_t r, uint32_t off) {
   __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_cvt, v), r, off, 0, 0);
@@ -104,14 +142,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
   mask_store<NR>(act, mr, rdz, row_z, P.dz_rbr);
   // dh_bott = W_{D+1}[:W] dz_rbr; the bottleneck is linear, so dz_bott = dh_bott
-  layer<16, 0, NR>(acc, act, nullptr, rs, lane_off, P.p_bwd4[D + 1]);
+  layer<16, NR>(acc, act, rs, lane_off, P.p_bwd4[D + 1]);
 #pragma unroll
   for (int nb = 0; nb < 16; ++nb) {
     act[nb] = acc[nb];
     store_f4(act[nb], rdz, row_z + (uint32_t)((P.dz_bott + 16 * nb) * 4));
   }
   // dh_{D-1} = W_D dz_bott + W_sigma dz_sigma
-  layer<16, 0, NH>(acc, act, nullptr, rs, lane_off, P.p_bwd4[D]);
+  layer<16, NH>(acc, act, rs, lane_off, P.p_bwd4[D]);
 #pragma unroll
   for (int nb = 0; nb < 16; ++nb) {
     const floatx4 w = ws::ldf4(rs, q_off, P.p_hs_nat + 64 * nb);
@@ -122,7 +160,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // trunk, top-down: dh_{l-1} = W_l[:W] dz_l, dz_{l-1} = dh_{l-1} [h_{l-1} > 0]
   ws::static_for<1, D>([&](auto Lc) {
     constexpr int l = D - decltype(Lc)::value;  // D-1 .. 1
-    layer<16, 0, NH>(acc, act, nullptr, rs, lane_off, P.p_bwd4[l]);
+    layer<16, NH>(acc, act, rs, lane_off, P.p_bwd4[l]);
 #pragma unroll
     for (int nb = 0; nb < 16; ++nb) act[nb] = acc[nb];
     mask_store<16>(act, mw[l - 1], rdz, row_z, P.dz_h[l - 1]);

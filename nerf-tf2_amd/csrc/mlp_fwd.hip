@@ -1,9 +1,10 @@
 // Fused positional-encoding + MLP forward (model.py:289-394) on MFMA.
 //
-// The reference topology (8 x 256 with the rgb branch) runs the register-
-// resident kernel of mlp_fwd_f32r.h in fp32 and the eight-wave weight-
-// stationary kernel of mlp_fwd_bf16ws8.h in bf16.  The fp32 kernel below serves the other topologies
-// (the proposal and finite-difference nets).  One wave owns 32 samples and
+// The reference topology (8 x 256 with the rgb branch) runs the kernel of
+// mlp_fwd_f32s.h in fp32 (split products on the FP16 matrix cores) and the
+// eight-wave weight-stationary kernel of mlp_fwd_bf16ws8.h in bf16.  The fp32
+// kernel below serves the other topologies (the proposal and finite-difference
+// nets).  One wave owns 32 samples and
 // carries them through every layer:
 //   * the encoding is computed in registers directly in B-operand slots;
 //   * each layer's output accumulates in registers (floatx16 per 32 features),
@@ -20,7 +21,7 @@
 
 #include "mlp_fwd_bf16.h"
 #include "mlp_fwd_bf16ws.h"
-#include "mlp_fwd_f32r.h"
+#include "mlp_fwd_f32s.h"
 #include "mlp_fwd_bf16ws8.h"
 
 namespace {
@@ -124,8 +125,7 @@ int launch_fwd_f32(const MlpPlan& P, const void* packed, int64_t M, const float*
                    const float* dirs, const float* ro, const float* rd, const float* tv, int spr,
                    float* rgb, float* sigma, void* stash, hipStream_t s) {
   if constexpr (W == 256 && LD > 0 && SKIP >= 0 && SKIP + 1 < D) {
-    // the reference topology: the register-resident kernel (16 samples per wave)
-    launch_fwd_f32r<W, D, SKIP, LX, LD>(P, packed, M, xyz, dirs, ro, rd, tv, spr, rgb, sigma, stash, s);
+    launch_fwd_f32s<W, D, SKIP, LX, LD>(P, packed, M, xyz, dirs, ro, rd, tv, spr, rgb, sigma, stash, s);
   } else {
     const int64_t nblk = (M + 31) / 32;
     const int64_t grid = (nblk + 3) / 4;

@@ -1,0 +1,344 @@
+// FP32 forward of the reference topology (W = 256 with the rgb branch), with or
+// without the training stash, on the FP16 matrix cores (mlp_f32s.h).
+//
+// A workgroup of eight waves carries 32 N samples through every layer.  Wave w
+// owns output block w (32 features); a layer's input sits in LDS as split B
+// operands (32 KB per sample block), the weights, split when they are packed,
+// stream from L2 as 1 KB loads two k-steps ahead.  A layer ends with the bias and
+// the ReLU, the exchange of each sample's largest value (its scale for the next
+// layer) and, behind that barrier, the split values' stores over the old tile.
+// With N = 2 the kernel keeps to 80 KB and 128 registers, so two workgroups share
+// a CU, four waves a SIMD: one workgroup's epilogues, encodings and barriers
+// overlap the other's MFMAs.  The encoding of the skip layer and of the rgb
+// branch is computed a second time into the tile once the hidden input has been
+// read, instead of holding 24 KB of it throughout.
+//
+// What bounds it: power.  The matrix cores are busy 0.69 of the time at a clock
+// that falls to 1.57 GHz; with random operands three FP16 products a step, their
+// LDS reads and 2 KB of weights per six MFMAs from L2, and nothing else, ran at
+// 1,139 TFLOP/s of FP16 work, this kernel at 1,190.  Measured at 6,291,456 samples:
+// 51.0 -> 18.7 ms (147 -> 399 TFLOP/s of FP32 work) against the register-resident
+// v_mfma_f32_16x16x4f32 kernel it replaced, which kept the FP32 matrix cores 0.94
+// busy; one workgroup of 128 samples per CU (half the weight traffic, but its
+// epilogues exposed) took 19.1 ms.  Three bf16 planes and six products, also
+// exact, took 31.6 ms.
+//
+// N = 1 halves a workgroup's serial time where the samples do not fill the chip:
+// M = 1,000 189 -> 34 us a call; N = 1 / 2: 28.7 / 45.0 us at M = 4,096, 34.5 / 45.0
+// at 8,192, 52.5 / 46.5 at 12,000, 62.5 / 54.6 at 16,384, so N = 1 up to 32 samples
+// per CU.
+#pragma once
+#include "mlp_f32s.h"
+
+// N sample blocks of 32 per workgroup.
+template <int W, int D, int SKIP, int LX, int LD, int N, bool STASH>
+__global__ __launch_bounds__(512, 4) void mlp_fwd_f32s_kernel(
+    MlpPlan P, const char* __restrict__ pk, int64_t M, const float* __restrict__ xyz,
+    const float* __restrict__ dirs, const float* __restrict__ ro, const float* __restrict__ rd,
+    const float* __restrict__ tv, int spr, float* __restrict__ rgb_out, float* __restrict__ sig_out,
+    float* __restrict__ stash) {
+  using namespace f32s;
+  using C = NetC<W, D, SKIP, LX, LD>;
+  static_assert(W == 256 && C::KX == 32 && C::KD == 16 && SKIP >= 0 && SKIP + 1 < D,
+                "split kernel is for the 8x256 NeRF MLP");
+  static_assert(N == 1 || N == 2, "the rgb branch's 4 N output blocks go to waves 0 .. 4 N - 1");
+  constexpr int TX = C::KX / 8, TD = C::KD / 8;
+  // weight units and k-steps of B operands in registers: one workgroup's two waves a SIMD
+  // (N = 1) wait for L2 and LDS themselves, two workgroups' four for each other
+  constexpr int AR = N == 1 ? 4 : 3, BR = N == 1 ? 2 : 1;
+  constexpr int NBIAS = (D + 1) * C::NB + C::NBR;
+  __shared__ half8 s_tile[N][kTH * 128];         // 32 KB per sample block: a layer's input
+  __shared__ floatx4 s_bias[NBIAS * 8];          // 9.5 KB: [block][lane half][16]
+  __shared__ float s_max[N][kWaves * 32];        // a layer's largest values per block and sample
+  __shared__ float s_sig[N][kWaves * 32];        // sigma-head partials per block and sample
+  __shared__ float s_pt[N][6][32];               // sample points and directions
+  const int lane = threadIdx.x & 63, j = lane & 31, g = lane >> 5;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t base = (int64_t)blockIdx.x * (32 * N);
+  const __amdgpu_buffer_rsrc_t rs = ws::packed_rsrc(pk + P.p_fs[0], P.fs_bytes);
+  const uint32_t lane_off = 16u * (uint32_t)lane;
+  const int* wexp = reinterpret_cast<const int*>(pk + P.p_fse);  // weight scales [layer][block]
+  // this wave's units of layer l start here (rgb branch: output block wv % 4)
+  auto unit0 = [&](int l) -> int64_t {
+    const int T = l == 0 ? TX : (l == SKIP + 1 ? kTH + TX : (l <= D ? kTH : kTH + TD));
+    return P.p_fs[l] - P.p_fs[0] + (int64_t)(l <= D ? wv : wv & 3) * T * kUnit;
+  };
+  Planes a[AR];
+#pragma unroll
+  for (int t = 0; t < AR - 1; ++t) a[t] = load_unit(rs, lane_off, unit0(0) + t * kUnit);
+
+  // the stash rows of this workgroup as a buffer resource (rows past M fall outside it)
+  const int64_t w_rows = M - base < 32 * N ? M - base : 32 * N;
+  const __amdgpu_buffer_rsrc_t rst =
+      STASH ? __builtin_amdgcn_make_buffer_rsrc(stash + base * P.stash_per_sample, 0,
+                                                (int)(w_rows * P.stash_per_sample * 4), 0x00020000)
+            : rs;
+  const uint32_t row = (uint32_t)(j * P.stash_per_sample * 4), blk_row = (uint32_t)(32 * P.stash_per_sample * 4);
+  auto st4 = [&](floatx4 v, int n, int64_t el) {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rst, row + n * blk_row + (uint32_t)(4 * el), 0, 0);
+  };
+
+  if (threadIdx.x < 32 * N) {
+    const int64_t m = base + threadIdx.x;
+    float x[3], d[3];
+    load_sample(m < M ? m : M - 1, xyz, dirs, ro, rd, tv, spr, x, d);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      s_pt[threadIdx.x >> 5][c][threadIdx.x & 31] = x[c];
+      s_pt[threadIdx.x >> 5][3 + c][threadIdx.x & 31] = d[c];
+    }
+  }
+  // Scale of this lane's sample in block n for an encoding (c0: 0 xyz, 3 direction): no value
+  // exceeds the largest component, or 1, the bound of the sines.
+  auto enc_scale = [&](int n, int c0) {
+    return scale_exp(fmaxf(fmaxf(fabsf(s_pt[n][c0][j]), fabsf(s_pt[n][c0 + 1][j])), fmaxf(fabsf(s_pt[n][c0 + 2][j]), 1.f)));
+  };
+  // Encoding of L frequencies (K slots per lane half) as the first K / 8 k-steps of the tile:
+  // unit u (wave u % 8) is k-step u % (K / 8) of sample block u / (K / 8).
+  auto encode = [&](auto Lc, int c0, int64_t st_off, bool first) {
+    constexpr int L = decltype(Lc)::value, K = L == LX ? C::KX : C::KD, T = K / 8;
+    for (int u = wv; u < T * N; u += kWaves) {
+      const int n = u / T, t = u % T;
+      const float x[3] = {s_pt[n][c0][j], s_pt[n][c0 + 1][j], s_pt[n][c0 + 2][j]};
+      float v[8];
+      encode_kstep<L>(x, g, t, v);
+      const Planes p = split8(v, pow2(enc_scale(n, c0)));
+      s_tile[n][t * 128 + lane] = p.h;
+      s_tile[n][t * 128 + 64 + lane] = p.l;
+      if (STASH && first) {
+        st4(floatx4{v[0], v[1], v[2], v[3]}, n, st_off + g * K + 8 * t);
+        st4(floatx4{v[4], v[5], v[6], v[7]}, n, st_off + g * K + 8 * t + 4);
+      }
+    }
+  };
+  // biases of every layer in accumulator order (element 4 a + r of half g: feature 8 a + 4 g + r)
+  {
+    const __amdgpu_buffer_rsrc_t rp = ws::packed_rsrc(pk, P.packed_bytes);
+    for (int e = threadIdx.x; e < NBIAS * 8; e += 64 * kWaves) {
+      const int blk = e >> 3, h = (e >> 2) & 1, q = e & 3;
+      const int l = blk / C::NB < D + 1 ? blk / C::NB : D + 1;
+      s_bias[e] = ws::ldf4(rp, 4u * (uint32_t)(32 * (blk - C::NB * l) + 8 * q + 4 * h) + (uint32_t)P.p_bias[l], 0);
+    }
+  }
+  lds_h8* tile[N];
+#pragma unroll
+  for (int n = 0; n < N; ++n) tile[n] = lds_lane(s_tile[n], lane);
+  const lds_f4* bias = (const lds_f4*)&s_bias[8 * wv + 4 * g];
+  floatx16 hi[N], lo[N];
+  int se[N];  // scale of this lane's sample in the tile
+  lds_barrier();
+  encode(std::integral_constant<int, LX>{}, 0, P.st_encx, true);
+#pragma unroll
+  for (int n = 0; n < N; ++n) se[n] = enc_scale(n, 0);
+  lds_barrier();
+
+  // ring position of layer l's first weight unit
+  constexpr auto ring0 = [](int l) {
+    int u = 0;
+    for (int i = 0; i < l; ++i) u += i == 0 ? TX : (i == SKIP + 1 ? kTH + TX : kTH);
+    return u % AR;
+  };
+  ws::static_for<0, D + 1>([&](auto Lc) {
+    constexpr int l = decltype(Lc)::value, R = ring0(l);
+    const int we = wexp[l * C::NB + wv];
+    zero(hi);
+    zero(lo);
+    if constexpr (l == 0) {
+      steps<N, TX, R, AR, BR>(a, hi, lo, tile, rs, lane_off, unit0(0), unit0(1));
+    } else if constexpr (l == SKIP + 1) {
+      steps<N, kTH, R, AR, BR>(a, hi, lo, tile, rs, lane_off, unit0(l), unit0(l) + kTH * kUnit);
+      lds_barrier();
+      encode(std::integral_constant<int, LX>{}, 0, 0, false);
+      // the sums so far go to the encoding's scale
+#pragma unroll
+      for (int n = 0; n < N; ++n) {
+        const int s1 = enc_scale(n, 0);
+        const float f = pow2(s1 - se[n]);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          hi[n][i] = hi[n][i] * f;
+          lo[n][i] = lo[n][i] * f;
+        }
+        se[n] = s1;
+      }
+      lds_barrier();
+      steps<N, TX, (R + kTH) % AR, AR, BR>(a, hi, lo, tile, rs, lane_off, unit0(l) + kTH * kUnit, unit0(l + 1));
+    } else {
+      steps<N, kTH, R, AR, BR>(a, hi, lo, tile, rs, lane_off, unit0(l), unit0(l + 1));
+    }
+    const int64_t st_off = (l < D ? P.st_h[l] : P.st_bott) + 32 * wv;
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      const float f = inv_scale(se[n], we);
+      float mx = 0.f;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const floatx4 b = bias[8 * C::NB * l + q];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = 4 * q + r;
+          float v = __builtin_fmaf(hi[n][i] + lo[n][i], f, b[r]);
+          if constexpr (l < D) v = v > 0.f ? v : 0.f;
+          hi[n][i] = v;
+          mx = fmaxf(mx, l < D ? v : fabsf(v));
+        }
+      }
+      put_max((lds_f*)s_max[n], wv, j, g, mx);
+      if constexpr (STASH) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          st4(floatx4{hi[n][4 * q], hi[n][4 * q + 1], hi[n][4 * q + 2], hi[n][4 * q + 3]}, n, st_off + 8 * q + 4 * g);
+      }
+      if constexpr (STASH && l < D) {
+        // ReLU bits of this block: lane half g holds features 8 q + 4 g + r, quarter 2 (q % 2) + g of
+        // 16-feature block 2 wv + q / 2; 8 bits (one byte) per quarter and layer word
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          uint32_t w = 0u;
+#pragma unroll
+          for (int i = 0; i < 8; ++i) w |= (hi[n][4 * (k + 2 * (i >> 2)) + (i & 3)] > 0.f ? 1u : 0u) << i;
+          __builtin_amdgcn_raw_buffer_store_b8((unsigned char)w, rst,
+                                               row + n * blk_row + (uint32_t)(4 * (P.st_mask + 8 * l + 2 * (2 * k + g)) + wv),
+                                               0, 0);
+        }
+      }
+      if constexpr (l == D - 1) {
+        // sigma head on h_{D-1} (model.py:374-375): this block's part of the dot product
+        const floatx4* hs = reinterpret_cast<const floatx4*>(pk + P.p_head_sigma) + (g * C::KH + 16 * wv) / 4;
+        float z = 0.f;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const floatx4 w = hs[q];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) z = z + hi[n][4 * q + r] * w[r];
+        }
+        z = z + shfl_xor(z, 32);
+        if (g == 0) s_sig[n][wv * 32 + j] = z;
+      }
+    }
+    lds_barrier();  // every wave has read the tile; the largest values are there
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      se[n] = scale_exp(get_max((const lds_f*)s_max[n], j));
+      const float sc = pow2(se[n]);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = hi[n][8 * h + i];
+        const Planes p = split8(v, sc);
+        lds_h8* o = tile[n] + (2 * wv + h) * 128;
+        o[0] = p.h;
+        o[64] = p.l;
+      }
+    }
+    lds_barrier();
+  });
+
+  // ---- dense_{D+1} on concat(bottleneck, direction encoding) (model.py:380-384): wave w
+  // does output block w % 4 of sample block w / 4
+  constexpr int RR = ring0(D + 1);
+  const bool own = wv < 4 * N;
+  const int n = N == 1 ? 0 : wv >> 2, nb = wv & 3;
+  floatx16 h1[1], l1[1];
+  lds_h8* t1[1];
+  t1[0] = n ? tile[N - 1] : tile[0];
+  zero(h1);
+  zero(l1);
+  if (own) steps<1, kTH, RR, AR, BR>(a, h1, l1, t1, rs, lane_off, unit0(D + 1), unit0(D + 1) + kTH * kUnit);
+  lds_barrier();
+  encode(std::integral_constant<int, LD>{}, 3, P.st_encd, true);
+  lds_barrier();
+  float p0 = 0.f, p1 = 0.f, p2 = 0.f;
+  if (own) {
+    const int s1 = enc_scale(n, 3);
+    const float f1 = pow2(s1 - (n ? se[N - 1] : se[0]));
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      h1[0][i] = h1[0][i] * f1;
+      l1[0][i] = l1[0][i] * f1;
+    }
+    steps<1, TD, (RR + kTH) % AR, AR, BR>(a, h1, l1, t1, rs, lane_off, unit0(D + 1) + kTH * kUnit, unit0(D + 1));
+    const float f = inv_scale(s1, wexp[(D + 1) * C::NB + nb]);
+    const floatx4* hr4 = reinterpret_cast<const floatx4*>(pk + P.p_head_rgb) + g * 16 * C::NBR + 16 * nb;
+    const lds_f4* br = (const lds_f4*)&s_bias[8 * (C::NB * (D + 1) + nb) + 4 * g];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const floatx4 b = br[q];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = 4 * q + r;
+        const float v = __builtin_fmaf(h1[0][i] + l1[0][i], f, b[r]);
+        h1[0][i] = v > 0.f ? v : 0.f;
+        const floatx4 w = hr4[i];  // rgb head (model.py:386-387)
+        p0 = p0 + h1[0][i] * w[0];
+        p1 = p1 + h1[0][i] * w[1];
+        p2 = p2 + h1[0][i] * w[2];
+      }
+      if constexpr (STASH)
+        st4(floatx4{h1[0][4 * q], h1[0][4 * q + 1], h1[0][4 * q + 2], h1[0][4 * q + 3]}, n,
+            P.st_rbr + 32 * nb + 8 * q + 4 * g);
+    }
+    if constexpr (STASH) {
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        uint32_t w = 0u;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) w |= (h1[0][4 * (k + 2 * (i >> 2)) + (i & 3)] > 0.f ? 1u : 0u) << i;
+        __builtin_amdgcn_raw_buffer_store_b8(
+            (unsigned char)w, rst, row + n * blk_row + (uint32_t)(4 * (P.st_mask + 8 * D + 2 * k + g) + nb), 0, 0);
+      }
+    }
+    p0 = p0 + shfl_xor(p0, 32);
+    p1 = p1 + shfl_xor(p1, 32);
+    p2 = p2 + shfl_xor(p2, 32);
+  }
+  lds_barrier();  // the tile is free: rgb-head partials per output block and sample
+  float* s_red = reinterpret_cast<float*>(s_tile);  // [nb][n][3][32]
+  if (own && g == 0) {
+    float* o = s_red + (nb * N + n) * 96 + j;
+    o[0] = p0;
+    o[32] = p1;
+    o[64] = p2;
+  }
+  lds_barrier();
+  // outputs: thread 4 q + c of the first 128 N finishes colour c (c < 3) or sigma of sample q
+  if (threadIdx.x < 128 * N) {
+    const int q = threadIdx.x >> 2, c = threadIdx.x & 3, nn = q >> 5, jj = q & 31;
+    const int64_t m = base + q;
+    if (m < M) {
+      if (c < 3) {
+        const float* r = s_red + nn * 96 + c * 32 + jj;
+        const float z = ((r[0] + r[N * 96]) + (r[2 * N * 96] + r[3 * N * 96])) +
+                        reinterpret_cast<const float*>(pk + P.p_head_rgb)[2 * 16 * C::NBR * 4 + c];
+        rgb_out[3 * m + c] = sigmoidf(z);
+      } else {
+        float z = 0.f;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) z = z + s_sig[nn][w * 32 + jj];
+        sig_out[m] = relu(z + reinterpret_cast<const float*>(pk + P.p_head_sigma)[2 * C::KH]);
+      }
+    }
+  }
+}
+
+template <int W, int D, int SKIP, int LX, int LD>
+void launch_fwd_f32s(const MlpPlan& P, const void* packed, int64_t M, const float* xyz, const float* dirs,
+                     const float* ro, const float* rd, const float* tv, int spr, float* rgb, float* sigma,
+                     void* stash, hipStream_t s) {
+  auto go = [&](auto Nc, auto St) {
+    constexpr int N = decltype(Nc)::value;
+    mlp_fwd_f32s_kernel<W, D, SKIP, LX, LD, N, decltype(St)::value>
+        <<<(unsigned)((M + 32 * N - 1) / (32 * N)), 64 * f32s::kWaves, 0, s>>>(
+            P, reinterpret_cast<const char*>(packed), M, xyz, dirs, ro, rd, tv, spr, rgb, sigma,
+            reinterpret_cast<float*>(stash));
+  };
+  const bool small = M <= (int64_t)32 * nerf_num_cus();  // (figures at the top)
+  if (stash) {
+    if (small) go(std::integral_constant<int, 1>{}, std::true_type{});
+    else go(std::integral_constant<int, 2>{}, std::true_type{});
+  } else {
+    if (small) go(std::integral_constant<int, 1>{}, std::false_type{});
+    else go(std::integral_constant<int, 2>{}, std::false_type{});
+  }
+}

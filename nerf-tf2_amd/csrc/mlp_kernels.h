@@ -115,6 +115,34 @@ __device__ __forceinline__ void encode_slots(const float (&x)[3], int g, float (
   }
 }
 
+// Slots 8 t .. 8 t + 7 of encode_slots (t wave-uniform at run time), the same values.
+template <int L>
+__device__ __forceinline__ void encode_kstep(const float (&x)[3], int g, int t, float (&out)[8]) {
+  constexpr int P0 = (3 * L - 2) / 2;
+  constexpr float kPi = 3.14159265358979323846f;
+  float x0 = x[0], x1 = x[1], x2 = x[2];
+  asm volatile("" : "+v"(x0), "+v"(x1), "+v"(x2));
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int k = 4 * t + i;
+    const int p = g ? P0 + k : k - 2;
+    const bool is_pair = g ? (P0 + k < 3 * L) : (k >= 2 && k - 2 < P0);
+    float s = 0.f, c = 0.f;
+    if (is_pair) {
+      const int comp = p / L, l = p - comp * L;
+      const float xc = comp == 0 ? x0 : (comp == 1 ? x1 : x2);
+      const float arg = fmul(xc, ldexpf(kPi, l));
+      sincosf(arg, &s, &c);
+    }
+    if (!is_pair) {
+      s = (g == 0 && k == 0) ? x0 : ((g == 0 && k == 1) ? x2 : 0.f);
+      c = (g == 0 && k == 0) ? x1 : 0.f;
+    }
+    out[2 * i] = s;
+    out[2 * i + 1] = c;
+  }
+}
+
 template <int K>
 __device__ __forceinline__ void store_slots_f32(const float (&v)[K], float* dst) {
 #pragma unroll

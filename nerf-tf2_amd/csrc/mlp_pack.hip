@@ -2,8 +2,13 @@
 // and the size queries of the MLP entry points.
 #include "common.h"
 #include "mlp_plan.h"
+#include "mlp_f32s.h"
 
 namespace {
+
+typedef float floatx4_a4 __attribute__((ext_vector_type(4), aligned(4)));  // the caller's weights: any float alignment
+
+constexpr int kSplitRows = 320;  // rows of the widest split layer (the skip layer's 256 + 63 inputs), padded
 
 // Input row (of the Keras kernel) fed by fp32 k-step s on lane half g of MFMA layer m.
 __device__ int fwd_row_f32(const MlpPlan& P, int m, int s, int g) {
@@ -25,165 +30,195 @@ __device__ int fwd_row_bf16(const MlpPlan& P, int m, int t, int r, int g) {
   return (m == 0 ? 0 : P.W) + ef;
 }
 
-// Input row fed by k-step s (0 .. ke4 + kh4 - 1: the encoding's first) on lane
-// quarter q of MFMA layer m in the register-resident fp32 forward.
-__device__ int fwd_row_f32x4(const MlpPlan& P, int m, int s, int q) {
-  const int ke4 = P.ks_enc[m] == 0 ? 0 : (P.enc_L[m] == P.LX ? P.S4X : P.S4D);
-  if (s < ke4) {
-    const int ef = enc_feat4(q, s, P.enc_L[m]);
-    return ef < 0 ? -1 : (m == 0 ? 0 : P.W) + ef;
-  }
-  const int t = s - ke4;  // hidden k-step 4 nb + r reads G(nb, r, q)
-  return 16 * (t / 4) + 4 * q + t % 4;
-}
-
 __device__ float kernel_at(const MlpPlan& P, const float* flat, int kl, int row, int col) {
   if (row < 0 || row >= P.fan_in[kl] || col < 0 || col >= P.fan_out[kl]) return 0.f;
   return flat[P.k_off[kl] + (int64_t)row * P.fan_out[kl] + col];
 }
 
-// One launch packs everything: blockIdx.y selects the segment.
-//   y in [0, n_mfma)            forward A operands of MFMA layer y
-//   y in [n_mfma, 2 n_mfma)     backward (transposed) A operands
-//   y in [2 n_mfma, 3 n_mfma)   biases
-//   y == 3 n_mfma               sigma head, y == 3 n_mfma + 1 rgb head
-//   y in [3 n_mfma + 2, 4 n_mfma + 2)  register-resident fp32 forward A operands
-//   y == 4 n_mfma + 2           both heads in natural feature order (fp32)
-//   y in [4 n_mfma + 3, 5 n_mfma + 3)  register-resident fp32 dX chain A operands
-__global__ void pack_kernel(MlpPlan P, const float* __restrict__ flat, char* __restrict__ out) {
-  const int seg = blockIdx.y;
-  const int nm = P.n_mfma;
-  const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t nthr = (int64_t)gridDim.x * blockDim.x;
-  if (seg >= 4 * nm + 3) {
-    // e = ((grp * NBi + nb) * 64 + lane) * 4 + r: A[n = input feature 16 nb + i][k = output
-    // feature 16 grp + 4 q + r] of layer m (lane = i + 16 q)
-    const int m = seg - (4 * nm + 3);
-    if (P.prec != 0 || m == 0) return;
-    const int kl = P.keras_of[m], NBi = P.W / 16, G = 2 * P.nb_out[m];
-    float* o = reinterpret_cast<float*>(out + P.p_bwd4[m]);
-    const int64_t n = (int64_t)G * NBi * 64 * 4;
-    for (int64_t e = tid; e < n; e += nthr) {
-      const int r = (int)(e % 4), lane = (int)((e / 4) % 64);
-      const int nb = (int)((e / 256) % NBi), grp = (int)(e / (256 * NBi));
-      const int i = lane & 15, q = lane >> 4;
-      o[e] = kernel_at(P, flat, kl, 16 * nb + i, 16 * grp + 4 * q + r);
-    }
-    return;
+// One launch packs everything: a list of segments, each a run of workgroups.
+enum PackKind : int { kFwd, kBwd, kBias, kHeads, kNatHeads, kBwd4, kSplitFwd };
+constexpr int kMaxSegs = 4 * NERF_MAX_LAYERS + 2;
+struct PackSegs {
+  int n;
+  int first[kMaxSegs + 1];  // first workgroup of each segment; [n]: their number
+  unsigned char kind[kMaxSegs], layer[kMaxSegs];
+};
+
+// Forward A operands of MFMA layer m: thread u writes the 16 bytes of lane u % 64 of
+// (k-step or k-step group, output block) u / 64.
+__device__ void pack_fwd(const MlpPlan& P, const float* __restrict__ flat, char* __restrict__ out, int m, int u) {
+  const int kl = P.keras_of[m], NBo = P.nb_out[m];
+  const int lane = u & 63, j = lane & 31, g = lane >> 5, nb = (u >> 6) % NBo, t = (u >> 6) / NBo;
+  if (P.prec == 0) {
+    if (t >= (P.ks_hid[m] + P.ks_enc[m]) / 4) return;
+    floatx4 v;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = kernel_at(P, flat, kl, fwd_row_f32(P, m, 4 * t + r, g), 32 * nb + j);
+    reinterpret_cast<floatx4*>(out + P.p_fwd[m])[u] = v;
+  } else {
+    const int ke16 = P.ks_enc[m] == 0 ? 0 : (P.enc_L[m] == P.LX ? P.KX16 : P.KD16);
+    if (t >= P.ks_hid[m] / 8 + ke16) return;
+    ushortx8 v;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) v[r] = f2bf(kernel_at(P, flat, kl, fwd_row_bf16(P, m, t, r, g), 32 * nb + j));
+    reinterpret_cast<ushortx8*>(out + P.p_fwd[m])[u] = v;
   }
-  if (seg >= 3 * nm + 2) {
-    if (P.prec != 0) return;
-    if (seg < 4 * nm + 2) {
-      // e = ((grp * NBo4 + nb) * 64 + lane) * 4 + r; k-step 4 grp + r; lane = i + 16 q
-      const int m = seg - (3 * nm + 2), kl = P.keras_of[m], NBo4 = 2 * P.nb_out[m];
-      const int ke4 = P.ks_enc[m] == 0 ? 0 : (P.enc_L[m] == P.LX ? P.S4X : P.S4D);
-      const int kh4 = P.ks_hid[m] == 0 ? 0 : P.W / 4;
-      float* o = reinterpret_cast<float*>(out + P.p_fwd4[m]);
-      const int64_t n = (int64_t)(ke4 + kh4) * NBo4 * 64;
-      for (int64_t e = tid; e < n; e += nthr) {
-        const int r = (int)(e % 4), lane = (int)((e / 4) % 64);
-        const int nb = (int)((e / 256) % NBo4), grp = (int)(e / (256 * NBo4));
-        const int i = lane & 15, q = lane >> 4;
-        o[e] = kernel_at(P, flat, kl, fwd_row_f32x4(P, m, 4 * grp + r, q), 16 * nb + i);
-      }
+}
+
+// Backward (transposed) A operands: A[n = input hidden feature 32 nb + j][k = output feature].
+__device__ void pack_bwd(const MlpPlan& P, const float* __restrict__ flat, char* __restrict__ out, int m, int u) {
+  const int kl = P.keras_of[m], lane = u & 63, j = lane & 31, g = lane >> 5, nb = (u >> 6) % P.NB, t = (u >> 6) / P.NB;
+  if (P.prec == 0) {
+    if (t >= 4 * P.nb_out[m]) return;
+    floatx4 v;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = kernel_at(P, flat, kl, 32 * nb + j, cfeat((4 * t + r) / 16, (4 * t + r) % 16, g));
+    reinterpret_cast<floatx4*>(out + P.p_bwd[m])[u] = v;
+  } else {
+    if (t >= 2 * P.nb_out[m]) return;
+    ushortx8 v;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) v[r] = f2bf(kernel_at(P, flat, kl, 32 * nb + j, cfeat(t / 2, 8 * (t % 2) + r, g)));
+    reinterpret_cast<ushortx8*>(out + P.p_bwd[m])[u] = v;
+  }
+}
+
+// Register-resident fp32 dX chain, thread u: A[n = input feature 16 nb + i][k = output feature
+// 16 grp + 4 q + r] of layer m (lane = i + 16 q).
+__device__ void pack_bwd4(const MlpPlan& P, const float* __restrict__ flat, char* __restrict__ out, int m, int u) {
+  const int kl = P.keras_of[m], NBi = P.W / 16, i = u & 15, q = (u >> 4) & 3, nb = (u >> 6) % NBi, grp = (u >> 6) / NBi;
+  if (grp >= 2 * P.nb_out[m]) return;
+  floatx4 v;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) v[r] = kernel_at(P, flat, kl, 16 * nb + i, 16 * grp + 4 * q + r);
+  reinterpret_cast<floatx4*>(out + P.p_bwd4[m])[u] = v;
+}
+
+__device__ void pack_heads(const MlpPlan& P, const float* __restrict__ flat, char* __restrict__ out) {
+  float* hs = reinterpret_cast<float*>(out + P.p_head_sigma);
+  const int KH = P.W / 2, KS = 16 * P.NBR;
+  for (int e = threadIdx.x; e < 2 * KH + 4; e += 256) {
+    const int g = e / KH, s = e % KH;
+    hs[e] = e < 2 * KH ? kernel_at(P, flat, P.kl_sigma, cfeat(s / 16, s % 16, g), 0)
+                       : (e == 2 * KH ? flat[P.b_off[P.kl_sigma]] : 0.f);
+  }
+  if (!P.rgb) return;
+  float* hr = reinterpret_cast<float*>(out + P.p_head_rgb);
+  for (int e = threadIdx.x; e < 2 * KS * 4 + 4; e += 256) {
+    const int c = e % 4, s = (e / 4) % KS, g = e / (4 * KS);
+    if (e < 2 * KS * 4)
+      hr[e] = c < 3 ? kernel_at(P, flat, P.kl_rgb, cfeat(s / 16, s % 16, g), c) : 0.f;
+    else
+      hr[e] = c < 3 ? flat[P.b_off[P.kl_rgb] + c] : 0.f;
+  }
+}
+
+// Both heads in natural feature order (fp32).
+__device__ void pack_nat_heads(const MlpPlan& P, const float* __restrict__ flat, char* __restrict__ out) {
+  float* hs = reinterpret_cast<float*>(out + P.p_hs_nat);
+  for (int e = threadIdx.x; e < P.W + 4; e += 256)
+    hs[e] = e < P.W ? kernel_at(P, flat, P.kl_sigma, e, 0) : (e == P.W ? flat[P.b_off[P.kl_sigma]] : 0.f);
+  if (!P.rgb) return;
+  float* hr = reinterpret_cast<float*>(out + P.p_hr_nat);
+  for (int e = threadIdx.x; e < P.WR * 4 + 4; e += 256) {
+    const int c = e % 4;
+    if (e < P.WR * 4)
+      hr[e] = c < 3 ? kernel_at(P, flat, P.kl_rgb, e / 4, c) : 0.f;
+    else
+      hr[e] = c < 3 ? flat[P.b_off[P.kl_rgb] + c] : 0.f;
+  }
+}
+
+// Split forward operands of layer m, one workgroup per output block nb: its 32 columns go to
+// LDS (one read of the weights, all loads in flight together), the largest gives the block's
+// scale, and each thread writes 16-byte chunks: the 8 slots of lane (j, g) of k-step t in unit
+// nb T + t, planes 1 KB apart.
+__device__ void pack_split(const MlpPlan& P, const float* __restrict__ flat, char* __restrict__ out, int m, int nb,
+                           float* s_w, float* s_m) {
+  const int kl = P.keras_of[m], T = (P.ks_hid[m] + P.ks_enc[m]) / 8, rows = P.fan_in[kl];
+  const float* w = flat + P.k_off[kl] + 32 * nb + 4 * (threadIdx.x & 7);
+  floatx4 v4[kSplitRows / 32];
+#pragma unroll
+  for (int i = 0; i < kSplitRows / 32; ++i) {
+    const int row = 32 * i + (threadIdx.x >> 3);
+    v4[i] = row < rows ? (floatx4)*reinterpret_cast<const floatx4_a4*>(w + (int64_t)row * P.fan_out[kl]) : floatx4{0.f, 0.f, 0.f, 0.f};
+  }
+  float mx = 0.f;
+#pragma unroll
+  for (int i = 0; i < kSplitRows / 32; ++i) {
+    reinterpret_cast<floatx4*>(s_w)[i * 256 + threadIdx.x] = v4[i];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) mx = fmaxf(mx, fabsf(v4[i][r]));
+  }
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) mx = fmaxf(mx, shfl_xor(mx, d));
+  if ((threadIdx.x & 63) == 0) s_m[threadIdx.x >> 6] = mx;
+  __syncthreads();
+  const int s = f32s::scale_exp(fmaxf(fmaxf(s_m[0], s_m[1]), fmaxf(s_m[2], s_m[3])), 60);
+  if (threadIdx.x == 0) reinterpret_cast<int*>(out + P.p_fse)[m * P.NB + nb] = s;
+  const float sc = f32s::pow2(s);
+  const int j = threadIdx.x & 31, g = (threadIdx.x >> 5) & 1;
+  f32s::half8* o = reinterpret_cast<f32s::half8*>(out + P.p_fs[m]) + (int64_t)nb * T * 128 + (threadIdx.x & 63);
+  for (int t = threadIdx.x >> 6; t < T; t += 4) {
+    float v[8];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const int row = fwd_row_bf16(P, m, t, r, g);
+      v[r] = row < 0 ? 0.f : s_w[row * 32 + j];
+    }
+    const f32s::Planes p = f32s::split8(v, sc);
+    o[t * 128] = p.h;
+    o[t * 128 + 64] = p.l;
+  }
+}
+
+__global__ __launch_bounds__(256) void pack_kernel(MlpPlan P, PackSegs S, const float* __restrict__ flat,
+                                                   char* __restrict__ out) {
+  __shared__ floatx4 s_w[kSplitRows * 8];
+  __shared__ float s_m[4];
+  int seg = 0;
+  while (seg + 1 < S.n && (int)blockIdx.x >= S.first[seg + 1]) ++seg;
+  const int blk = blockIdx.x - S.first[seg], m = S.layer[seg], u = 256 * blk + threadIdx.x;
+  switch (S.kind[seg]) {
+    case kFwd: return pack_fwd(P, flat, out, m, u);
+    case kBwd: return pack_bwd(P, flat, out, m, u);
+    case kBias: {
+      const int kl = P.keras_of[m];
+      if (u < 32 * P.nb_out[m])
+        reinterpret_cast<float*>(out + P.p_bias[m])[u] = u < P.fan_out[kl] ? flat[P.b_off[kl] + u] : 0.f;
       return;
     }
-    float* hs = reinterpret_cast<float*>(out + P.p_hs_nat);
-    for (int64_t e = tid; e < P.W + 4; e += nthr)
-      hs[e] = e < P.W ? kernel_at(P, flat, P.kl_sigma, (int)e, 0) : (e == P.W ? flat[P.b_off[P.kl_sigma]] : 0.f);
-    if (!P.rgb) return;
-    float* hr = reinterpret_cast<float*>(out + P.p_hr_nat);
-    for (int64_t e = tid; e < (int64_t)P.WR * 4 + 4; e += nthr) {
-      const int c = (int)(e % 4);
-      if (e < (int64_t)P.WR * 4)
-        hr[e] = c < 3 ? kernel_at(P, flat, P.kl_rgb, (int)(e / 4), c) : 0.f;
-      else
-        hr[e] = c < 3 ? flat[P.b_off[P.kl_rgb] + c] : 0.f;
-    }
-    return;
+    case kHeads: return pack_heads(P, flat, out);
+    case kNatHeads: return pack_nat_heads(P, flat, out);
+    case kBwd4: return pack_bwd4(P, flat, out, m, u);
+    case kSplitFwd: return pack_split(P, flat, out, m, blk, reinterpret_cast<float*>(s_w), s_m);
   }
-  if (seg < nm) {
-    const int m = seg, kl = P.keras_of[m], NBo = P.nb_out[m];
-    if (P.prec == 0) {
-      const int KS = P.ks_hid[m] + P.ks_enc[m];
-      float* o = reinterpret_cast<float*>(out + P.p_fwd[m]);
-      const int64_t n = (int64_t)KS * NBo * 64;
-      for (int64_t e = tid; e < n; e += nthr) {  // e = ((q*NBo + nb)*64 + lane)*4 + r
-        const int r = (int)(e % 4), lane = (int)((e / 4) % 64);
-        const int nb = (int)((e / 256) % NBo), q = (int)(e / (256 * NBo));
-        const int s = 4 * q + r, j = lane & 31, g = lane >> 5;
-        o[e] = kernel_at(P, flat, kl, fwd_row_f32(P, m, s, g), 32 * nb + j);
-      }
-    } else {
-      const int ke16 = P.ks_enc[m] == 0 ? 0 : (P.enc_L[m] == P.LX ? P.KX16 : P.KD16);
-      const int KS = P.ks_hid[m] / 8 + ke16;
-      unsigned short* o = reinterpret_cast<unsigned short*>(out + P.p_fwd[m]);
-      const int64_t n = (int64_t)KS * NBo * 64 * 8;
-      for (int64_t e = tid; e < n; e += nthr) {  // e = ((t*NBo + nb)*64 + lane)*8 + r
-        const int r = (int)(e % 8), lane = (int)((e / 8) % 64);
-        const int nb = (int)((e / 512) % NBo), t = (int)(e / (512 * NBo));
-        const int j = lane & 31, g = lane >> 5;
-        o[e] = f2bf(kernel_at(P, flat, kl, fwd_row_bf16(P, m, t, r, g), 32 * nb + j));
-      }
-    }
-  } else if (seg < 2 * nm) {
-    const int m = seg - nm;
-    if (m == 0) return;
-    const int kl = P.keras_of[m], NBo = P.nb_out[m];
-    if (P.prec == 0) {
-      const int KS = NBo * 16;  // k-steps over the layer's outputs
-      float* o = reinterpret_cast<float*>(out + P.p_bwd[m]);
-      const int64_t n = (int64_t)KS * P.NB * 64;
-      for (int64_t e = tid; e < n; e += nthr) {
-        const int r = (int)(e % 4), lane = (int)((e / 4) % 64);
-        const int nb = (int)((e / 256) % P.NB), q = (int)(e / (256 * P.NB));
-        const int s = 4 * q + r, j = lane & 31, g = lane >> 5;
-        // A[n = input hidden feature 32nb+j][k = output feature cfeat(s)]
-        o[e] = kernel_at(P, flat, kl, 32 * nb + j, cfeat(s / 16, s % 16, g));
-      }
-    } else {
-      const int KS = NBo * 2;
-      unsigned short* o = reinterpret_cast<unsigned short*>(out + P.p_bwd[m]);
-      const int64_t n = (int64_t)KS * P.NB * 64 * 8;
-      for (int64_t e = tid; e < n; e += nthr) {
-        const int r = (int)(e % 8), lane = (int)((e / 8) % 64);
-        const int nb = (int)((e / 512) % P.NB), t = (int)(e / (512 * P.NB));
-        const int j = lane & 31, g = lane >> 5;
-        o[e] = f2bf(kernel_at(P, flat, kl, 32 * nb + j, cfeat(t / 2, 8 * (t % 2) + r, g)));
-      }
-    }
-  } else if (seg < 3 * nm) {
-    const int m = seg - 2 * nm, kl = P.keras_of[m];
-    float* o = reinterpret_cast<float*>(out + P.p_bias[m]);
-    const int n = 32 * P.nb_out[m];
-    for (int64_t e = tid; e < n; e += nthr)
-      o[e] = e < P.fan_out[kl] ? flat[P.b_off[kl] + e] : 0.f;
-  } else if (seg == 3 * nm) {
-    const int kl = P.kl_sigma;
-    float* o = reinterpret_cast<float*>(out + P.p_head_sigma);
-    const int KH = P.W / 2;
-    for (int64_t e = tid; e < 2 * KH + 4; e += nthr) {
-      if (e < 2 * KH) {
-        const int g = (int)(e / KH), s = (int)(e % KH);
-        o[e] = kernel_at(P, flat, kl, cfeat(s / 16, s % 16, g), 0);
-      } else {
-        o[e] = e == 2 * KH ? flat[P.b_off[kl]] : 0.f;
-      }
-    }
-  } else if (P.rgb) {
-    const int kl = P.kl_rgb;
-    float* o = reinterpret_cast<float*>(out + P.p_head_rgb);
-    const int KS = 16 * P.NBR;
-    for (int64_t e = tid; e < 2 * KS * 4 + 4; e += nthr) {
-      if (e < 2 * KS * 4) {
-        const int c = (int)(e % 4), s = (int)((e / 4) % KS), g = (int)(e / (4 * KS));
-        o[e] = c < 3 ? kernel_at(P, flat, kl, cfeat(s / 16, s % 16, g), c) : 0.f;
-      } else {
-        const int c = (int)(e - 2 * KS * 4);
-        o[e] = c < 3 ? flat[P.b_off[kl] + c] : 0.f;
-      }
-    }
+}
+
+// The segments of a plan, the longest-running first.
+PackSegs pack_segs(const MlpPlan& P) {
+  PackSegs S{};
+  auto add = [&](PackKind k, int m, int64_t blocks) {
+    S.kind[S.n] = (unsigned char)k;
+    S.layer[S.n] = (unsigned char)m;
+    S.first[S.n + 1] = S.first[S.n] + (int)blocks;
+    ++S.n;
+  };
+  auto blocks16 = [](int64_t bytes) { return (bytes + 4095) / 4096; };  // 16 bytes per thread
+  for (int m = 0; m < P.n_mfma; ++m)
+    if (P.p_fs[m] >= 0) add(kSplitFwd, m, P.nb_out[m]);
+  for (int m = 0; m < P.n_mfma; ++m) {
+    const int ks = P.ks_hid[m] + P.ks_enc[m];
+    const int ke16 = P.ks_enc[m] == 0 ? 0 : (P.enc_L[m] == P.LX ? P.KX16 : P.KD16);
+    if (P.p_fwd[m] >= 0)
+      add(kFwd, m, blocks16((int64_t)P.nb_out[m] * 64 * 16 * (P.prec == 0 ? ks / 4 : P.ks_hid[m] / 8 + ke16)));
+    if (P.p_bwd[m] >= 0) add(kBwd, m, blocks16((int64_t)P.nb_out[m] * (P.prec == 0 ? 4 : 2) * P.NB * 64 * 16));
+    if (P.p_bwd4[m] >= 0) add(kBwd4, m, blocks16((int64_t)2 * P.nb_out[m] * (P.W / 16) * 64 * 16));
   }
+  for (int m = 0; m < P.n_mfma; ++m) add(kBias, m, (32 * P.nb_out[m] + 255) / 256);
+  add(kHeads, 0, 1);
+  if (P.p_hs_nat >= 0) add(kNatHeads, 0, 1);
+  return S;
 }
 
 }  // namespace
@@ -228,8 +263,8 @@ extern "C" int32_t nerf_mlp_pack(const nerf_mlp_desc* desc, int32_t precision, c
                                  void* packed, void* stream) {
   NERF_PLAN_OR_FAIL(desc, precision, P, "nerf_mlp_pack");
   NERF_CHECK_ARG(flat && packed, "nerf_mlp_pack: null pointer");
-  dim3 grid(64, 5 * P.n_mfma + 3), block(256);
-  pack_kernel<<<grid, block, 0, as_stream(stream)>>>(P, flat, reinterpret_cast<char*>(packed));
+  const PackSegs S = pack_segs(P);
+  pack_kernel<<<(unsigned)S.first[S.n], 256, 0, as_stream(stream)>>>(P, S, flat, reinterpret_cast<char*>(packed));
   NERF_LAUNCH_CHECK("nerf_mlp_pack");
   return NERF_OK;
 }

@@ -45,40 +45,12 @@ __host__ __device__ inline int enc_feat(int g, int e, int L) {
 // Hidden feature held by accumulator i of output block nb on lane half g.
 __host__ __device__ inline int cfeat(int nb, int i, int g) { return 32 * nb + 8 * (i / 4) + 4 * g + (i % 4); }
 
-// Register-resident fp32 forward (v_mfma_f32_16x16x4f32): one wave owns 16
+// Register-resident fp32 dX chain (v_mfma_f32_16x16x4f32): one wave owns 16
 // samples, lane l = j + 16 q (j = sample, q = lane quarter).  Output block nb
 // (16 features) holds in accumulator r of lane (j, q) the feature
 //   G(nb, r, q) = 16 nb + 4 q + r
 // which is also what k-step 4 nb + r of the next layer reads on quarter q, so
-// a layer's output is the next layer's B operand in place.  An encoding of L
-// frequencies takes S4(L) slots per quarter (a multiple of 4): quarter 0 holds
-// x, y, z, pad, then (sin, cos) pairs 0 .. S4/2 - 3; quarter q >= 1 holds
-// pairs S4/2 - 2 + (q - 1) S4/2 + e/2; pairs >= 3L are pads.
-// Inverse of enc_feat: lane-half slot index g * K + e (K slots per half) of
-// reference encoding feature f of an encoding with L frequencies.
-__host__ __device__ inline int enc_slot_of(int f, int L, int K) {
-  if (f < 3) return f;
-  const int P0 = (3 * L - 2) / 2, p = (f - 3) / 2, sc = (f - 3) % 2;
-  return p < P0 ? 4 + 2 * p + sc : K + 2 * (p - P0) + sc;
-}
-
-__host__ __device__ constexpr int enc_slots4(int L) { return ((3 * L + 3) / 2 + 3) / 4 * 4; }
-__host__ __device__ inline int enc_feat4(int q, int e, int L) {
-  const int S = enc_slots4(L), P0 = S / 2 - 2;
-  if (e < 0 || e >= S) return -1;
-  int p;
-  if (q == 0) {
-    if (e < 3) return e;
-    if (e == 3) return -1;
-    p = (e - 4) / 2;
-  } else {
-    p = P0 + (q - 1) * (S / 2) + e / 2;
-  }
-  if (p >= 3 * L) return -1;
-  const int c = p / L, l = p % L;
-  return 3 + c * 2 * L + 2 * l + e % 2;
-}
-
+// a layer's output is the next layer's B operand in place.
 struct MlpPlan {
   int D, W, skip, LX, LD, rgb;
   int NB, NBR, WR;      // hidden blocks, rgb-branch blocks, rgb-branch width
@@ -102,16 +74,20 @@ struct MlpPlan {
   // packed byte offsets
   int64_t p_fwd[NERF_MAX_LAYERS], p_bwd[NERF_MAX_LAYERS], p_bias[NERF_MAX_LAYERS];
   int64_t p_head_sigma, p_head_rgb, packed_bytes;
-  // fp32 only: A operands of the register-resident forward (per layer: the
-  // encoding's k-step groups first, then the hidden input's; a group is 4
-  // k-steps of every output block of 16), and both heads in natural feature
-  // order (sigma: W weights + bias; rgb: [W/2][4] + bias[4]); -1 for bf16
-  int64_t p_fwd4[NERF_MAX_LAYERS], p_hs_nat, p_hr_nat;
+  // fp32 only: both heads in natural feature order (sigma: W weights + bias; rgb:
+  // [W/2][4] + bias[4]); -1 for bf16
+  int64_t p_hs_nat, p_hr_nat;
   // fp32 only: transposed A operands of the register-resident dX chain, layers
   // m >= 1 (k-step groups of 16 output features of layer m, each over the W/16
   // blocks of its hidden input; -1 otherwise)
   int64_t p_bwd4[NERF_MAX_LAYERS];
-  int S4X, S4D;  // encoding slots per lane quarter in that forward
+  // fp32, W = 256 with an rgb branch only (-1 otherwise): A operands of the forward
+  // on the FP16 matrix cores, each weight split into two fp16 planes.  Per layer
+  // units [output block of 32][k-step of 16][plane][lane][8], the k-steps and their
+  // order as in the bf16 form; the layers follow each other without gaps (fs_bytes
+  // from p_fs[0] on).  p_fse: int32 per layer and output block (NB apart), the
+  // power of two its weights are scaled by
+  int64_t p_fs[NERF_MAX_LAYERS], fs_bytes, p_fse;
   int prec;
   // stash (elements per sample; fp32 or bf16 elements) and dz (floats per sample)
   int64_t st_encx, st_h[NERF_MAX_LAYERS], st_bott, st_rbr, st_encd, stash_per_sample;
@@ -222,10 +198,13 @@ inline int mlp_make_plan(int D, int W, int skip, int LX, int LD, int prec, MlpPl
     ++m;
   }
   P.n_mfma = m;
-  // packed layout
+  // packed layout (p_fwd, p_bwd: not for the split form, whose kernels read p_fs and p_bwd4)
+  const bool split = prec == 0 && W == 256 && P.rgb && P.NBR == 4;
   int64_t b = 0;
   auto align = [&](int64_t a) { b = (b + a - 1) / a * a; };
   for (int i = 0; i < P.n_mfma; ++i) {
+    P.p_fwd[i] = -1;
+    if (split) continue;
     align(256);
     P.p_fwd[i] = b;
     if (prec == 0)
@@ -237,7 +216,7 @@ inline int mlp_make_plan(int D, int W, int skip, int LX, int LD, int prec, MlpPl
   }
   for (int i = 0; i < P.n_mfma; ++i) {
     P.p_bwd[i] = -1;
-    if (i == 0) continue;  // no dX for the encoding input
+    if (i == 0 || split) continue;  // no dX for the encoding input
     align(256);
     P.p_bwd[i] = b;
     // A[n = input hidden feature][k = output feature]: k-steps over the outputs
@@ -258,18 +237,7 @@ inline int mlp_make_plan(int D, int W, int skip, int LX, int LD, int prec, MlpPl
   align(256);
   P.p_head_rgb = b;  // [2][16*NBR][4] fp32 + bias[4]
   if (P.rgb) b += (int64_t)2 * 16 * P.NBR * 16 + 16;
-  P.S4X = enc_slots4(LX);
-  P.S4D = LD ? enc_slots4(LD) : 0;
   P.p_hs_nat = P.p_hr_nat = -1;
-  for (int i = 0; i < P.n_mfma; ++i) {
-    P.p_fwd4[i] = -1;
-    if (prec != 0) continue;
-    align(256);
-    P.p_fwd4[i] = b;
-    const int ke4 = P.ks_enc[i] == 0 ? 0 : (P.enc_L[i] == LX ? P.S4X : P.S4D);
-    const int kh4 = P.ks_hid[i] == 0 ? 0 : W / 4;
-    b += (int64_t)(ke4 + kh4) * (2 * P.nb_out[i]) * 64 * 4;
-  }
   for (int i = 0; i < P.n_mfma; ++i) {
     P.p_bwd4[i] = -1;
     if (prec != 0 || i == 0) continue;
@@ -277,6 +245,16 @@ inline int mlp_make_plan(int D, int W, int skip, int LX, int LD, int prec, MlpPl
     P.p_bwd4[i] = b;
     b += (int64_t)(2 * P.nb_out[i]) * (W / 16) * 64 * 4 * 4;
   }
+  align(4096);
+  const int64_t fs0 = b;
+  for (int i = 0; i < P.n_mfma; ++i) {
+    P.p_fs[i] = split ? b : -1;
+    if (split) b += (int64_t)((P.ks_hid[i] + P.ks_enc[i]) / 8) * P.nb_out[i] * 2 * 1024;
+  }
+  P.fs_bytes = b - fs0;
+  align(256);
+  P.p_fse = split ? b : -1;
+  if (split) b += (int64_t)P.n_mfma * P.NB * 4;
   if (prec == 0) {
     align(256);
     P.p_hs_nat = b;

@@ -1,0 +1,94 @@
+"""FP32 forward of the 8x256 net on split FP16 products: batch sizes around the workgroup and
+dispatch edges against 64 bits, and power-of-two scales that leave the result's bits alone."""
+import importlib
+
+import numpy as np
+import pytest
+import torch
+
+oracle = importlib.import_module("oracle.restatement")
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.fixture(scope="module")
+def nerf():
+    return importlib.import_module("nerf-tf2_amd")
+
+
+def _net(nerf, seed=3, scale=None):
+    mlp = nerf.NerfMLP("fine", seed=seed, device=DEV)
+    w = mlp.get_weights()
+    rng = np.random.default_rng(seed)
+    w = [a if a.ndim == 2 else rng.normal(0.0, 0.05, a.shape).astype(np.float32) for a in w]
+    w[-1] = w[-1] + np.float32(0.3)
+    if scale is not None:
+        w = scale(w)
+    mlp.set_weights(w)
+    return mlp, w
+
+
+def _points(m, seed, size=1.2):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    x = size * (2 * torch.rand((m, 3), generator=g, device=DEV) - 1)
+    d = torch.randn((m, 3), generator=g, device=DEV)
+    return x, d / d.norm(dim=1, keepdim=True)
+
+
+def _encode64(x, L):
+    """Arguments in float32, as the encoding defines them; sines and cosines in 64 bits."""
+    mult = 2.0 ** torch.arange(L, dtype=torch.float32) * torch.tensor(np.float32(np.pi))
+    a = (x.cpu()[..., None] * mult).double()
+    return torch.cat([x.cpu().double(), torch.stack([a.sin(), a.cos()], -1).reshape(x.shape[0], -1)], -1)
+
+
+def _forward64(w, x, d):
+    w = [torch.from_numpy(a).double() for a in w]
+    e = _encode64(x, 10)
+    h = e
+    for i in range(8):
+        h = torch.relu(h @ w[2 * i] + w[2 * i + 1])
+        if i == 4:
+            h = torch.cat([h, e], -1)
+    r = torch.relu(torch.cat([h @ w[16] + w[17], _encode64(d, 4)], -1) @ w[18] + w[19])
+    return torch.sigmoid(r @ w[20] + w[21]), torch.relu(h @ w[22] + w[23])
+
+
+# One FP32 rounding per term of a K-term sum is off by about sqrt(K) 2^-25 of the sum's norm, 5e-7 at
+# K = 256, and ReLU layers pass a relative error on as it is: 1e-6 holds for FP32 sums.
+TOL = 1e-6
+
+
+@pytest.mark.parametrize("m", [1, 31, 33, 65, 8191, 8193, 16411])
+@pytest.mark.parametrize("size", [1.2, 300.0])
+def test_forward_against_64_bits(nerf, m, size):
+    mlp, w = _net(nerf)
+    x, d = _points(m, m, size)
+    with torch.no_grad():
+        rgb, sigma = mlp((x, d))
+    stash = mlp._alloc_stash(m)
+    rgb2, sigma2 = torch.empty_like(rgb), torch.empty_like(sigma)
+    mlp._launch_forward(m, x, d, None, None, None, rgb2, sigma2, stash)
+    assert torch.equal(rgb, rgb2) and torch.equal(sigma, sigma2)
+    pick = torch.unique(torch.cat([torch.arange(min(m, 300)), torch.arange(max(0, m - 300), m)]))
+    rgb64, sigma64 = _forward64(w, x[pick], d[pick])
+    for got, want in ((rgb, rgb64), (sigma, sigma64)):
+        err = (got[pick].cpu().double() - want).norm()
+        assert float(err) <= TOL * float(want.norm()), float(err)     # (0 <= 0 where a single density is 0)
+
+
+@pytest.mark.parametrize("e", [40, -40])
+def test_power_of_two_scales(nerf, e):
+    """Layer 2 times 2^e (its ReLU output with it) and layer 3's kernel times 2^-e: the same bits."""
+    def scale(w):
+        w = list(w)
+        w[4], w[5] = np.ldexp(w[4], e), np.ldexp(w[5], e)
+        w[6] = np.ldexp(w[6], -e)
+        return w
+    x, d = _points(777, 5)
+    a, _ = _net(nerf)
+    b, _ = _net(nerf, scale=scale)
+    with torch.no_grad():
+        ra, sa = a((x, d))
+        rb, sb = b((x, d))
+    assert torch.equal(ra, rb) and torch.equal(sa, sb)
