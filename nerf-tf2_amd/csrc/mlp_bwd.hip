@@ -21,6 +21,7 @@
 #include "mlp_bwd_bf16ws.h"
 #include "mlp_bwd_bf16ws8.h"
 #include "mlp_bwd_f32r.h"
+#include "mlp_wgrad_f32s.h"
 
 namespace {
 
@@ -241,141 +242,6 @@ __global__ __launch_bounds__(256) void mlp_bwd_bf16_kernel(
     mfma_lds_bf16<C::NB, TH>(acc, reinterpret_cast<const bf16x8*>(pk + P.p_bwd[l]), act, lane);
     relu_mask_rows_bf16(acc, srow, P.st_h[l - 1], g);
     if (valid) store_rows_bf16(acc, zrow, P.dz_h[l - 1], g);
-  }
-}
-
-// ---------------------------------------------------------------------------
-// fp32 weight-gradient GEMM: part[split][k][n] = sum over the split's samples of
-// X[m][xoff + k] * Z[m][zoff + n], for k < K, n < N.  128x128 tile per block,
-// 4 waves of 64x64 (2x2 blocks of v_mfma_f32_32x32x2_f32), 32-sample LDS chunks.
-// The block with tile_k == 0 also sums the columns of Z (bias gradient).
-// ---------------------------------------------------------------------------
-constexpr int kTile = 128, kChunk = 32, kPad = 4;
-
-struct GemmArgs {
-  const float* X;
-  int64_t ldx, xoff;
-  const float* Z;
-  int64_t ldz, zoff;
-  int64_t M, m_per_split;
-  int K, N, tiles_k, tiles_n, splits;
-  float* part;   // [splits][K][N]
-  float* bpart;  // [splits][N] or null
-};
-
-__global__ __launch_bounds__(256) void wgrad_gemm_kernel(GemmArgs a) {
-  __shared__ float Xs[kChunk][kTile + kPad];
-  __shared__ float Zs[kChunk][kTile + kPad];
-  // XCD-aware order: workgroup b runs on XCD b % 8, so all tiles of one sample
-  // split (which read the same X / dz rows) share b % 8 and hence one L2.
-  const int T = a.tiles_k * a.tiles_n;
-  const int xcd = blockIdx.x % 8, yy = blockIdx.x / 8;
-  const int tile = yy % T;
-  const int split = (yy / T) * 8 + xcd;
-  if (split >= a.splits) return;  // padding of the split count to a multiple of 8
-  const int tk = tile / a.tiles_n, tn = tile % a.tiles_n;
-  const int k0 = tk * kTile, n0 = tn * kTile;
-  const int64_t mb = (int64_t)split * a.m_per_split;
-  const int64_t me = mb + a.m_per_split < a.M ? mb + a.m_per_split : a.M;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int wk = (wv >> 1) * 64, wn = (wv & 1) * 64;  // wave quadrant
-  const int r = lane & 31, q = lane >> 5;
-  floatx16 acc[2][2];
-#pragma unroll
-  for (int x = 0; x < 2; ++x)
-#pragma unroll
-    for (int y = 0; y < 2; ++y)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[x][y][i] = 0.f;
-  // bias sums from the loaded dz values: thread t adds its 16 columns of every
-  // row it loads; the 32 threads of a column group meet at the end
-  float bs[16];
-#pragma unroll
-  for (int e = 0; e < 16; ++e) bs[e] = 0.f;
-  const bool do_bias = a.bpart && tk == 0;
-  // loader mapping: 256 threads x 16 floats = 32 rows x 128 cols; the next chunk is
-  // loaded into registers while the current one is multiplied
-  const int lr = tid >> 3, lc = (tid & 7) * 16;
-  floatx4 xv[4], zv[4];
-  auto load = [&](int64_t c0) {
-    const int64_t mrow = c0 + lr;
-    const bool rok = mrow < me;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int col = lc + 4 * v;
-      xv[v] = floatx4{0.f, 0.f, 0.f, 0.f};
-      zv[v] = floatx4{0.f, 0.f, 0.f, 0.f};
-      if (rok) {
-        const int64_t xo = mrow * a.ldx + a.xoff + k0 + col;
-        if (k0 + col + 3 < a.K) {
-          xv[v] = *reinterpret_cast<const floatx4*>(a.X + xo);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (k0 + col + e < a.K) xv[v][e] = a.X[xo + e];
-        }
-        if (n0 + col + 3 < a.N) {
-          zv[v] = *reinterpret_cast<const floatx4*>(a.Z + mrow * a.ldz + a.zoff + n0 + col);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (n0 + col + e < a.N) zv[v][e] = a.Z[mrow * a.ldz + a.zoff + n0 + col + e];
-        }
-      }
-    }
-  };
-  if (mb < me) load(mb);
-  for (int64_t c0 = mb; c0 < me; c0 += kChunk) {
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int col = lc + 4 * v;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        Xs[lr][col + e] = xv[v][e];
-        Zs[lr][col + e] = zv[v][e];
-        bs[4 * v + e] += zv[v][e];
-      }
-    }
-    __syncthreads();
-    if (c0 + kChunk < me) load(c0 + kChunk);  // wave-uniform
-#pragma unroll 4
-    for (int s = 0; s < kChunk / 2; ++s) {
-      const int row = 2 * s + q;
-      float av[2], bv[2];
-#pragma unroll
-      for (int x = 0; x < 2; ++x) av[x] = Xs[row][wk + 32 * x + r];
-#pragma unroll
-      for (int y = 0; y < 2; ++y) bv[y] = Zs[row][wn + 32 * y + r];
-#pragma unroll
-      for (int x = 0; x < 2; ++x)
-#pragma unroll
-        for (int y = 0; y < 2; ++y) acc[x][y] = mfma_f32(av[x], bv[y], acc[x][y]);
-    }
-    __syncthreads();
-  }
-  float* out = a.part + (int64_t)split * a.K * a.N;
-#pragma unroll
-  for (int x = 0; x < 2; ++x)
-#pragma unroll
-    for (int y = 0; y < 2; ++y)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int kk = k0 + wk + 32 * x + 8 * (i / 4) + 4 * q + (i % 4);
-        const int nn = n0 + wn + 32 * y + r;
-        if (kk < a.K && nn < a.N) out[(int64_t)kk * a.N + nn] = acc[x][y][i];
-      }
-  if (do_bias) {
-    // threads lr = 0..31 of column group t & 7 hold partial sums: through LDS, fixed order
-    float* red = &Xs[0][0];  // [32 rows][128 columns] fits the 32 x 132 tile
-#pragma unroll
-    for (int e = 0; e < 16; ++e) red[lr * 128 + lc + e] = bs[e];
-    __syncthreads();
-    if (tid < kTile) {
-      float v = 0.f;
-#pragma unroll 8
-      for (int rr = 0; rr < kChunk; ++rr) v += red[rr * 128 + tid];
-      if (n0 + tid < a.N) a.bpart[(int64_t)split * a.N + n0 + tid] = v;
-    }
   }
 }
 
@@ -945,8 +811,38 @@ __device__ __forceinline__ float sum_splits(const float* __restrict__ p, int64_t
   return s;
 }
 
+// The same sum with 64 (then 16) partials at a time added as a tree: the sum over the
+// splits is rounded a few times instead of once per split (192 splits of the proposal
+// net's layers: error against 64 bits 2.1e-7 -> 0.4e-7 of the gradient's norm).
+template <int N>
+__device__ __forceinline__ float tree_sum(float (&v)[N]) {
+#pragma unroll
+  for (int d = N / 2; d >= 1; d >>= 1)
+#pragma unroll
+    for (int j = 0; j < d; ++j) v[j] += v[j + d];
+  return v[0];
+}
+__device__ __forceinline__ float sum_splits_tree(const float* __restrict__ p, int64_t stride, int n) {
+  float s = 0.f;
+  int sp = 0;
+  for (; sp + 64 <= n; sp += 64) {
+    float v[64];
+#pragma unroll
+    for (int j = 0; j < 64; ++j) v[j] = p[(int64_t)(sp + j) * stride];
+    s += tree_sum(v);
+  }
+  for (; sp < n; sp += 16) {
+    float v[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) v[j] = sp + j < n ? p[(int64_t)(sp + j) * stride] : 0.f;
+    s += tree_sum(v);
+  }
+  return s;
+}
+
 // Blocks blk (of nblk) of the reduction of one job: element e of the K x N tile
 // (and of the bias row) summed over the splits into the flat gradient.
+template <bool TREE>
 __device__ __forceinline__ void reduce_job(const ReduceArgs& a, int64_t blk, int64_t nblk) {
   const int64_t n_el = (int64_t)a.K * a.N;
   for (int64_t e = blk * blockDim.x + threadIdx.x; e < n_el + a.N; e += nblk * blockDim.x) {
@@ -959,20 +855,18 @@ __device__ __forceinline__ void reduce_job(const ReduceArgs& a, int64_t blk, int
         row = enc_feat(g, s, a.enc_L);
         if (row < 0) continue;
       }
-      const float s = sum_splits(a.part + e, n_el, a.splits);
+      const float s = TREE ? sum_splits_tree(a.part + e, n_el, a.splits) : sum_splits(a.part + e, n_el, a.splits);
       float* dst = a.grad + a.k_off + (int64_t)(a.row_base + row) * a.fan_out + n;
       *dst = a.accumulate ? *dst + s : s;
     } else if (a.bpart) {
       const int n = (int)(e - n_el);
       if (n >= a.n_real) continue;
-      const float s = sum_splits(a.bpart + n, a.N, a.splits);
+      const float s = TREE ? sum_splits_tree(a.bpart + n, a.N, a.splits) : sum_splits(a.bpart + n, a.N, a.splits);
       float* dst = a.grad + a.b_off + n;
       *dst = a.accumulate ? *dst + s : s;
     }
   }
 }
-
-__global__ void wgrad_reduce_kernel(ReduceArgs a) { reduce_job(a, blockIdx.x, gridDim.x); }
 
 // The reductions of several jobs (a group, or every job of the call) in one
 // launch: job j owns blocks [first[j], first[j + 1]).
@@ -982,10 +876,11 @@ struct ReduceBatch {
   int njobs;
 };
 
+template <bool TREE>  // fp32: TREE
 __global__ void wgrad_reduce_batch_kernel(ReduceBatch b) {
   int j = 0;
   while (j + 1 < b.njobs && (int)blockIdx.x >= b.first[j + 1]) ++j;
-  reduce_job(b.job[j], (int64_t)blockIdx.x - b.first[j], b.first[j + 1] - b.first[j]);
+  reduce_job<TREE>(b.job[j], (int64_t)blockIdx.x - b.first[j], b.first[j + 1] - b.first[j]);
 }
 
 // One (X-segment, Z) GEMM + reduction into the flat gradient.
@@ -1127,6 +1022,118 @@ extern "C" int32_t nerf_mlp_backward(const nerf_mlp_desc* desc, int32_t precisio
   return NERF_OK;
 }
 
+// The fp32 launches: jobs by tile shape (mlp_wgrad_f32s.h), one launch per shape;
+// the heads (at most 4 columns) by VALU.
+enum { kWg8x4, kWg2x8, kWg1x4, kWg2x2, kWgHead, kWg32Classes };
+static int wg32_class(const WgradJob& J) {
+  if (J.N <= 4) return kWgHead;
+  if (J.K > 64) return kWg8x4;
+  if (J.N > 128 || (J.N > 64 && J.K > 32)) return kWg2x8;
+  return J.N > 64 ? kWg1x4 : kWg2x2;
+}
+static int64_t wg32_job_floats(const WgradJob& J) { return (int64_t)J.K * J.N + (J.bias ? J.N : 0); }
+static int wg32_tiles(const WgradJob& J, int cls) { return cls == kWg8x4 ? (J.N + 127) / 128 : 1; }
+
+// Splits per job of a class: one round of workgroups (a CU holds 1, 1, 2 or 3 of the
+// shapes by their LDS), but at least 256 samples per split, and more rounds so that no
+// split sums over more than 8,192 samples (the rounding of one long sum: 192,064 samples
+// of the 8x256 net 1.6e-7 of the gradient's norm in 15 splits, 0.9e-7 in 30), as far as the class's partial tiles stay within the allocation-free entry
+// point's static scratch; never so few that a split's rows pass 2^31 bytes.  Heads: 512.
+static int64_t wg32_splits(const MlpPlan& P, int64_t M, const WgradJob* jobs, int nj, int cls) {
+  static const int per_cu[kWg32Classes] = {1, 1, 2, 3, 0};
+  int64_t tiles = 0, floats = 0;
+  for (int t = 0; t < nj; ++t)
+    if (wg32_class(jobs[t]) == cls) {
+      tiles += wg32_tiles(jobs[t], cls);
+      floats += wg32_job_floats(jobs[t]);
+    }
+  if (!tiles) return 1;
+  const int64_t cap = (M + 255) / 256;
+  if (cls == kWgHead) return cap < 512 ? cap : 512;
+  int64_t s = 256 * per_cu[cls] / tiles;
+  if (s < 1) s = 1;
+  const int64_t rounds = (M + s * 8192 - 1) / (s * 8192);
+  if (rounds > 1) s = 256 * per_cu[cls] * rounds / tiles;
+  const int64_t most = (int64_t)NERF_WGRAD_STATIC_SCRATCH_BYTES / 4 / floats;
+  if (s > most) s = most;
+  if (s > cap) s = cap;
+  const int64_t least = wg16_min_splits(M, 4 * (P.stash_per_sample > P.dz_per_sample ? P.stash_per_sample : P.dz_per_sample));
+  if (s < least) s = least;
+  return s < 1 ? 1 : s;
+}
+
+static int64_t wg32_floats(const MlpPlan& P, int64_t M, const WgradJob* jobs, int nj) {
+  int64_t f = 0;
+  for (int cls = 0; cls < kWg32Classes; ++cls) {
+    const int64_t sp = wg32_splits(P, M, jobs, nj, cls);
+    for (int t = 0; t < nj; ++t)
+      if (wg32_class(jobs[t]) == cls) f += sp * wg32_job_floats(jobs[t]);
+  }
+  return f;
+}
+
+// One launch of n jobs of class cls with sp splits, partial tiles job after job from `part` on.
+static void wg32_launch(const MlpPlan& P, int64_t M, const void* stash, const void* dz, const WgradJob* jobs,
+                        const int* members, int n, int cls, int64_t sp, float* part, hipStream_t s) {
+  const float* X = reinterpret_cast<const float*>(stash);
+  const float* Z = reinterpret_cast<const float*>(dz);
+  auto tile = [&](const WgradJob& J, int n0, float* p) {
+    wg32::Tile T;
+    T.xoff = (int)J.xoff;
+    T.zoff = (int)J.zoff;
+    T.K = J.K;
+    T.N = J.N;
+    T.n0 = n0;
+    T.part = p;
+    T.bpart = J.bias ? p + sp * J.K * J.N : nullptr;
+    return T;
+  };
+  if (cls == kWgHead) {
+    wg32::HeadArgs h;
+    h.X = X;
+    h.Z = Z;
+    h.ldx = P.stash_per_sample;
+    h.ldz = P.dz_per_sample;
+    h.M = M;
+    h.m_per_split = (int)((M + sp - 1) / sp);
+    h.splits = (int)sp;
+    h.njobs = n;
+    for (int i = 0; i < n; ++i) {
+      h.tile[i] = tile(jobs[members[i]], 0, part);
+      part += sp * wg32_job_floats(jobs[members[i]]);
+    }
+    wg32::wgrad_head_kernel<<<(unsigned)(sp * n), 256, 0, s>>>(h);
+    return;
+  }
+  wg32::Args a;
+  a.X = X;
+  a.Z = Z;
+  a.ldx = P.stash_per_sample;
+  a.ldz = P.dz_per_sample;
+  a.M = M;
+  a.m_per_split = (int)(((M + sp - 1) / sp + wg32::kChunk - 1) / wg32::kChunk * wg32::kChunk);
+  a.splits = (int)sp;
+  a.pairs = a.singles = 0;
+  wg32::Tile single[2 * NERF_MAX_LAYERS];
+  for (int i = 0; i < n; ++i) {
+    const WgradJob& J = jobs[members[i]];
+    if (wg32_tiles(J, cls) == 2) {
+      a.tile[2 * a.pairs] = tile(J, 0, part);
+      a.tile[2 * a.pairs + 1] = tile(J, 128, part);
+      ++a.pairs;
+    } else {
+      single[a.singles++] = tile(J, 0, part);
+    }
+    part += sp * wg32_job_floats(J);
+  }
+  for (int i = 0; i < a.singles; ++i) a.tile[2 * a.pairs + i] = single[i];
+  const unsigned grid = (unsigned)(16 * ((a.pairs * sp + 7) / 8) + a.singles * sp);
+  if (cls == kWg8x4) wg32::wgrad_f32s_kernel<8, 4, 2, 2><<<grid, 512, 0, s>>>(a);
+  else if (cls == kWg2x8) wg32::wgrad_f32s_kernel<2, 8, 2, 1><<<grid, 512, 0, s>>>(a);
+  else if (cls == kWg1x4) wg32::wgrad_f32s_kernel<1, 4, 1, 1><<<grid, 256, 0, s>>>(a);
+  else wg32::wgrad_f32s_kernel<2, 2, 1, 1><<<grid, 256, 0, s>>>(a);
+}
+
 // Partial-tile floats of the weight-gradient workspace: room for `s` tiles of the
 // widest layer (kmax x W) and their bias rows, s = the larger of the float32
 // split count and the bf16 bound: a group of n <= kMaxJobs same-shape jobs uses
@@ -1252,6 +1259,12 @@ static int64_t wgrad_workspace_bytes_for(const nerf_mlp_desc* desc, int64_t M) {
   MlpPlan P, P16;
   if (nerf_plan_from_desc(desc, NERF_PREC_F32, &P) || M < 0) return -1;
   int64_t f = wgrad_workspace_floats(P, M);
+  {
+    WgradJob jobs[2 * NERF_MAX_LAYERS];
+    const int nj = wgrad_jobs(P, jobs);
+    const int64_t st = wg32_floats(P, M, jobs, nj);
+    if (st > f) f = st;
+  }
   if (nerf_plan_from_desc(desc, NERF_PREC_BF16, &P16) == 0) {
     const int64_t st = wg16_stacked_floats(P16, M, true);
     if (st > f) f = st;
@@ -1270,7 +1283,6 @@ static int32_t wgrad_run(const MlpPlan& P, int32_t precision, int64_t M, const v
                          int64_t part_floats, hipStream_t s) {
   WgradJob jobs[2 * NERF_MAX_LAYERS];
   const int nj = wgrad_jobs(P, jobs);
-  const int64_t splits = splits_for(M);
   auto reduce_args = [&](const WgradJob& J, const float* jp, const float* jb, int nsplit) {
     ReduceArgs r;
     r.part = jp;
@@ -1346,37 +1358,52 @@ static int32_t wgrad_run(const MlpPlan& P, int32_t precision, int64_t M, const v
         rbt.job[k] = reduce_args(jobs[G.members[i]], b.job[i].part, b.job[i].bpart, (int)sg);
         rbt.first[k + 1] = rbt.first[k] + reduce_blocks(jobs[G.members[i]]);
       }
-      if (!stack) wgrad_reduce_batch_kernel<<<(unsigned)rbt.first[rbt.njobs], 256, 0, s>>>(rbt);
+      if (!stack) wgrad_reduce_batch_kernel<false><<<(unsigned)rbt.first[rbt.njobs], 256, 0, s>>>(rbt);
     }
-    if (stack) wgrad_reduce_batch_kernel<<<(unsigned)all.first[all.njobs], 256, 0, s>>>(all);
+    if (stack) wgrad_reduce_batch_kernel<false><<<(unsigned)all.first[all.njobs], 256, 0, s>>>(all);
   } else {
-    for (int t = 0; t < nj; ++t) {
-      const WgradJob& J = jobs[t];
-      const int64_t kmax = (P.W > 2 * P.KX ? P.W : 2 * P.KX);
-      float* bpart = J.bias ? part + splits * kmax * P.W : nullptr;
-      GemmArgs a;
-      a.X = reinterpret_cast<const float*>(stash);
-      a.ldx = P.stash_per_sample;
-      a.xoff = J.xoff;
-      a.Z = reinterpret_cast<const float*>(dz);
-      a.ldz = P.dz_per_sample;
-      a.zoff = J.zoff;
-      a.M = M;
-      a.K = J.K;
-      a.N = J.N;
-      a.tiles_k = (J.K + kTile - 1) / kTile;
-      a.tiles_n = (J.N + kTile - 1) / kTile;
-      // three workgroups fit per CU: a four-tile layer takes 3/4 of the splits, so that
-      // its 4 x 192 workgroups run as one round on 256 CUs
-      const int64_t sj = a.tiles_k * a.tiles_n >= 4 && splits >= 4 ? splits * 3 / 4 : splits;
-      a.m_per_split = (M + sj - 1) / sj;
-      a.splits = (int)sj;
-      a.part = part;
-      a.bpart = bpart;
-      const int64_t nb = (int64_t)a.tiles_k * a.tiles_n * ((sj + 7) / 8) * 8;
-      wgrad_gemm_kernel<<<(unsigned)nb, 256, 0, s>>>(a);
-      wgrad_reduce_kernel<<<(unsigned)reduce_blocks(J), 256, 0, s>>>(reduce_args(J, part, bpart, (int)sj));
+    const bool stack = wg32_floats(P, M, jobs, nj) <= part_floats;  // every job's tiles side by side
+    ReduceBatch rb;
+    rb.njobs = rb.first[0] = 0;
+    float* base = part;
+    auto flush = [&]() {
+      if (rb.njobs) wgrad_reduce_batch_kernel<true><<<(unsigned)rb.first[rb.njobs], 256, 0, s>>>(rb);
+      rb.njobs = 0;
+      base = part;
+    };
+    for (int cls = 0; cls < kWg32Classes; ++cls) {
+      const int64_t sp0 = wg32_splits(P, M, jobs, nj, cls);
+      int t = 0;
+      while (t < nj) {
+        // the jobs of this class that fit the partial-tile buffer together
+        int members[2 * NERF_MAX_LAYERS], n = 0;
+        int64_t sp = sp0, used = base - part;
+        for (; t < nj; ++t) {
+          if (wg32_class(jobs[t]) != cls) continue;
+          const int64_t f = wg32_job_floats(jobs[t]);
+          if (used + sp * f > part_floats) {
+            if (n || used) break;
+            sp = part_floats / f;  // a job that does not fit by itself: fewer splits
+          }
+          used += sp * f;
+          members[n++] = t;
+        }
+        if (!n) {
+          if (t < nj) flush();
+          continue;
+        }
+        wg32_launch(P, M, stash, dz, jobs, members, n, cls, sp, base, s);
+        for (int i = 0; i < n; ++i) {
+          const WgradJob& J = jobs[members[i]];
+          const int k = rb.njobs++;
+          rb.job[k] = reduce_args(J, base, J.bias ? base + sp * J.K * J.N : nullptr, (int)sp);
+          rb.first[k + 1] = rb.first[k] + reduce_blocks(J);
+          base += sp * wg32_job_floats(J);
+        }
+        if (!stack) flush();
+      }
     }
+    flush();
   }
   NERF_LAUNCH_CHECK("nerf_mlp_weight_grads");
   return NERF_OK;

@@ -92,3 +92,52 @@ def test_power_of_two_scales(nerf, e):
         ra, sa = a((x, d))
         rb, sb = b((x, d))
     assert torch.equal(ra, rb) and torch.equal(sa, sb)
+
+
+NETS = {"nerf": dict(), "proposal": dict(depth=4, width=64, skip=-1, l_xyz=8, l_dir=0),
+        "narrow": dict(depth=4, width=32, skip=1)}
+
+
+@pytest.mark.parametrize("m", [1, 31, 33, 257, 8209, 30011])
+@pytest.mark.parametrize("net", list(NETS))
+@pytest.mark.parametrize("least", [False, True])
+def test_weight_grads_against_64_bits(nerf, net, m, least):
+    """FP32 weight gradients of the hidden layers and the density head from a random stash and dz
+    whose rows differ by powers of two, against 64 bits: chunk and split edges, every tile shape,
+    with the workspace that is asked for and with the least that is taken (least)."""
+    import ctypes
+    L = nerf._lib
+    cfg = nerf.MLPConfig(**NETS[net])
+    mlp = nerf.NerfMLP("fine", cfg, "fp32", seed=1, device=DEV)
+    d = ctypes.byref(mlp._desc)
+    g = torch.Generator(device=DEV).manual_seed(m)
+    stash = torch.randn((m, mlp.stash_per_sample), generator=g, device=DEV).relu()
+    dz = torch.randn((m, mlp.dz_per_sample), generator=g, device=DEV)
+    dz *= 2.0 ** torch.randint(-12, 13, (m, 1), generator=g, device=DEV)
+    ws = int(L.load().nerf_mlp_wgrad_workspace_bytes(d, m))
+    if least:
+        rc = L.load().nerf_mlp_weight_grads(d, 0, m, stash.data_ptr(), dz.data_ptr(), dz.data_ptr(), 0,
+                                            stash.data_ptr(), 0, L.stream())
+        assert rc == L.NERF_ERR_INVALID_ARG
+        ws = int(L.load().nerf_last_error().decode().split("needs ")[1].split()[0])
+    work = torch.empty(ws, dtype=torch.uint8, device=DEV)
+    grad = torch.full((mlp.n_params,), float("nan"), device=DEV)
+    L.call("nerf_mlp_weight_grads", d, 0, m, L.ptr(stash), L.ptr(dz), L.ptr(grad), 0, L.ptr(work), ws, L.stream())
+    assert bool(torch.isfinite(grad).all())
+    W, D = cfg.width, cfg.depth
+    enc = 2 * ((2 + 3 * cfg.l_xyz + 7) // 8 * 8)
+    z_sigma = D * W + (W + (W // 2 + 31) // 32 * 32 if cfg.l_dir else 0)
+    off = 0
+    for i, (name, fi, fo) in enumerate(cfg.layer_shapes()):
+        k, b = grad[off:off + fi * fo].view(fi, fo), grad[off + fi * fo:off + fi * fo + fo]
+        off += fi * fo + fo
+        if name == "sigma":
+            x0, z0 = enc + (D - 1) * W, z_sigma
+        elif 1 <= i < D:
+            x0, z0 = enc + (i - 1) * W, i * W
+        else:
+            continue
+        x, z = stash[:, x0:x0 + W].cpu().double(), dz[:, z0:z0 + fo].cpu().double()
+        for got, want in ((k[:W], x.T @ z), (b, z.sum(0))):
+            err = (got.cpu().double() - want).norm()
+            assert float(err) <= TOL * float(want.norm()), (name, float(err / want.norm()))
