@@ -2,8 +2,8 @@
 // takes through model.py:355-392) and its weight gradients.
 //
 // nerf_mlp_backward: one wave per 32 samples walks the layers top-down (the
-// reference topology runs the register-resident twin of mlp_bwd_f32r.h in fp32
-// and the eight-wave kernel of mlp_bwd_bf16ws8.h in bf16, same rows in and out).
+// reference topology runs the eight-wave kernels of mlp_bwd_f32s.h in fp32 and of
+// mlp_bwd_bf16ws8.h in bf16, same rows in and out).
 //   rgb = sigmoid(z):  dz_rgb = d_rgb * rgb (1 - rgb)
 //   sigma = relu(z):   dz_sigma = d_sigma * [sigma > 0]      (softplus: * (1 - e^-sigma))
 //   dh = W dz (MFMA with the transposed packed weights; the accumulators of one
@@ -20,7 +20,7 @@
 #include "mlp_kernels.h"
 #include "mlp_bwd_bf16ws.h"
 #include "mlp_bwd_bf16ws8.h"
-#include "mlp_bwd_f32r.h"
+#include "mlp_bwd_f32s.h"
 #include "mlp_wgrad_f32s.h"
 
 namespace {
@@ -950,7 +950,7 @@ int launch_bwd_f32(const MlpPlan& P, const void* packed, int64_t M, const float*
                    void* dz, hipStream_t s) {
   if constexpr (W == 256 && LD > 0 && SKIP >= 0 && SKIP + 1 < D) {
     // the reference topology: the register-resident chain (16 samples per wave)
-    launch_bwd_f32r<W, D, SKIP, LX, LD>(P, packed, M, d_rgb, d_sigma, rgb, sigma, stash, dz, s);
+    launch_bwd_f32s<W, D, SKIP, LX, LD>(P, packed, M, d_rgb, d_sigma, rgb, sigma, stash, dz, s);
   } else {
     const int64_t nblk = (M + 31) / 32;
     mlp_bwd_f32_kernel<W, D, SKIP, LX, LD><<<(unsigned)((nblk + 3) / 4), 256, 0, s>>>(

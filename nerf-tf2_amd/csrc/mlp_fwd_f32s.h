@@ -20,8 +20,8 @@
 // 51.0 -> 18.7 ms (147 -> 399 TFLOP/s of FP32 work) against the register-resident
 // v_mfma_f32_16x16x4f32 kernel it replaced, which kept the FP32 matrix cores 0.94
 // busy; one workgroup of 128 samples per CU (half the weight traffic, but its
-// epilogues exposed) took 19.1 ms.  Three bf16 planes and six products, also
-// exact, took 31.6 ms.
+// epilogues exposed) took 19.1 ms.  Three exact bf16 planes and six products
+// took 31.6 ms.
 //
 // N = 1 halves a workgroup's serial time where the samples do not fill the chip:
 // M = 1,000 189 -> 34 us a call; N = 1 / 2: 28.7 / 45.0 us at M = 4,096, 34.5 / 45.0
@@ -190,17 +190,12 @@ __global__ __launch_bounds__(512, 4) void mlp_fwd_f32s_kernel(
           st4(floatx4{hi[n][4 * q], hi[n][4 * q + 1], hi[n][4 * q + 2], hi[n][4 * q + 3]}, n, st_off + 8 * q + 4 * g);
       }
       if constexpr (STASH && l < D) {
-        // ReLU bits of this block: lane half g holds features 8 q + 4 g + r, quarter 2 (q % 2) + g of
-        // 16-feature block 2 wv + q / 2; 8 bits (one byte) per quarter and layer word
+        // ReLU word of this block, lane half and layer
+        uint32_t w = 0u;
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-          uint32_t w = 0u;
-#pragma unroll
-          for (int i = 0; i < 8; ++i) w |= (hi[n][4 * (k + 2 * (i >> 2)) + (i & 3)] > 0.f ? 1u : 0u) << i;
-          __builtin_amdgcn_raw_buffer_store_b8((unsigned char)w, rst,
-                                               row + n * blk_row + (uint32_t)(4 * (P.st_mask + 8 * l + 2 * (2 * k + g)) + wv),
-                                               0, 0);
-        }
+        for (int i = 0; i < 16; ++i) w |= (hi[n][i] > 0.f ? 1u : 0u) << i;
+        __builtin_amdgcn_raw_buffer_store_b16((unsigned short)w, rst,
+                                              row + n * blk_row + (uint32_t)(4 * P.st_mask + 2 * ((2 * wv + g) * D + l)), 0, 0);
       }
       if constexpr (l == D - 1) {
         // sigma head on h_{D-1} (model.py:374-375): this block's part of the dot product
@@ -280,14 +275,11 @@ __global__ __launch_bounds__(512, 4) void mlp_fwd_f32s_kernel(
             P.st_rbr + 32 * nb + 8 * q + 4 * g);
     }
     if constexpr (STASH) {
+      uint32_t w = 0u;
 #pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        uint32_t w = 0u;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) w |= (h1[0][4 * (k + 2 * (i >> 2)) + (i & 3)] > 0.f ? 1u : 0u) << i;
-        __builtin_amdgcn_raw_buffer_store_b8(
-            (unsigned char)w, rst, row + n * blk_row + (uint32_t)(4 * (P.st_mask + 8 * D + 2 * k + g) + nb), 0, 0);
-      }
+      for (int i = 0; i < 16; ++i) w |= (h1[0][i] > 0.f ? 1u : 0u) << i;
+      __builtin_amdgcn_raw_buffer_store_b16((unsigned short)w, rst,
+                                            row + n * blk_row + (uint32_t)(4 * P.st_mask + 2 * (16 * D + 2 * nb + g)), 0, 0);
     }
     p0 = p0 + shfl_xor(p0, 32);
     p1 = p1 + shfl_xor(p1, 32);

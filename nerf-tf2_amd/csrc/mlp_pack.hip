@@ -36,8 +36,8 @@ __device__ float kernel_at(const MlpPlan& P, const float* flat, int kl, int row,
 }
 
 // One launch packs everything: a list of segments, each a run of workgroups.
-enum PackKind : int { kFwd, kBwd, kBias, kHeads, kNatHeads, kBwd4, kSplitFwd };
-constexpr int kMaxSegs = 4 * NERF_MAX_LAYERS + 2;
+enum PackKind : int { kFwd, kBwd, kBias, kHeads, kSplitFwd, kSplitBwd };
+constexpr int kMaxSegs = 3 * NERF_MAX_LAYERS + 1;
 struct PackSegs {
   int n;
   int first[kMaxSegs + 1];  // first workgroup of each segment; [n]: their number
@@ -83,17 +83,6 @@ __device__ void pack_bwd(const MlpPlan& P, const float* __restrict__ flat, char*
   }
 }
 
-// Register-resident fp32 dX chain, thread u: A[n = input feature 16 nb + i][k = output feature
-// 16 grp + 4 q + r] of layer m (lane = i + 16 q).
-__device__ void pack_bwd4(const MlpPlan& P, const float* __restrict__ flat, char* __restrict__ out, int m, int u) {
-  const int kl = P.keras_of[m], NBi = P.W / 16, i = u & 15, q = (u >> 4) & 3, nb = (u >> 6) % NBi, grp = (u >> 6) / NBi;
-  if (grp >= 2 * P.nb_out[m]) return;
-  floatx4 v;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) v[r] = kernel_at(P, flat, kl, 16 * nb + i, 16 * grp + 4 * q + r);
-  reinterpret_cast<floatx4*>(out + P.p_bwd4[m])[u] = v;
-}
-
 __device__ void pack_heads(const MlpPlan& P, const float* __restrict__ flat, char* __restrict__ out) {
   float* hs = reinterpret_cast<float*>(out + P.p_head_sigma);
   const int KH = P.W / 2, KS = 16 * P.NBR;
@@ -113,20 +102,13 @@ __device__ void pack_heads(const MlpPlan& P, const float* __restrict__ flat, cha
   }
 }
 
-// Both heads in natural feature order (fp32).
-__device__ void pack_nat_heads(const MlpPlan& P, const float* __restrict__ flat, char* __restrict__ out) {
-  float* hs = reinterpret_cast<float*>(out + P.p_hs_nat);
-  for (int e = threadIdx.x; e < P.W + 4; e += 256)
-    hs[e] = e < P.W ? kernel_at(P, flat, P.kl_sigma, e, 0) : (e == P.W ? flat[P.b_off[P.kl_sigma]] : 0.f);
-  if (!P.rgb) return;
-  float* hr = reinterpret_cast<float*>(out + P.p_hr_nat);
-  for (int e = threadIdx.x; e < P.WR * 4 + 4; e += 256) {
-    const int c = e % 4;
-    if (e < P.WR * 4)
-      hr[e] = c < 3 ? kernel_at(P, flat, P.kl_rgb, e / 4, c) : 0.f;
-    else
-      hr[e] = c < 3 ? flat[P.b_off[P.kl_rgb] + c] : 0.f;
-  }
+// The scale exponent of a workgroup's weights, mx each thread's largest; orders its LDS writes.
+__device__ int split_scale(float mx, float* s_m) {
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) mx = fmaxf(mx, shfl_xor(mx, d));
+  if ((threadIdx.x & 63) == 0) s_m[threadIdx.x >> 6] = mx;
+  __syncthreads();
+  return f32s::scale_exp(fmaxf(fmaxf(s_m[0], s_m[1]), fmaxf(s_m[2], s_m[3])), 60);
 }
 
 // Split forward operands of layer m, one workgroup per output block nb: its 32 columns go to
@@ -150,11 +132,7 @@ __device__ void pack_split(const MlpPlan& P, const float* __restrict__ flat, cha
 #pragma unroll
     for (int r = 0; r < 4; ++r) mx = fmaxf(mx, fabsf(v4[i][r]));
   }
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) mx = fmaxf(mx, shfl_xor(mx, d));
-  if ((threadIdx.x & 63) == 0) s_m[threadIdx.x >> 6] = mx;
-  __syncthreads();
-  const int s = f32s::scale_exp(fmaxf(fmaxf(s_m[0], s_m[1]), fmaxf(s_m[2], s_m[3])), 60);
+  const int s = split_scale(mx, s_m);
   if (threadIdx.x == 0) reinterpret_cast<int*>(out + P.p_fse)[m * P.NB + nb] = s;
   const float sc = f32s::pow2(s);
   const int j = threadIdx.x & 31, g = (threadIdx.x >> 5) & 1;
@@ -166,6 +144,42 @@ __device__ void pack_split(const MlpPlan& P, const float* __restrict__ flat, cha
       const int row = fwd_row_bf16(P, m, t, r, g);
       v[r] = row < 0 ? 0.f : s_w[row * 32 + j];
     }
+    const f32s::Planes p = f32s::split8(v, sc);
+    o[t * 128] = p.h;
+    o[t * 128 + 64] = p.l;
+  }
+}
+
+// The same for the dX chain: input block nb, 32 rows of fan_out (128 or 256) weights each, kept
+// in LDS one float apart so that 32 lanes read 32 rows without bank conflicts.
+__device__ void pack_split_bwd(const MlpPlan& P, const float* __restrict__ flat, char* __restrict__ out, int m,
+                               int nb, float* s_w, float* s_m) {
+  const int kl = P.keras_of[m], T = 2 * P.nb_out[m], FO = P.fan_out[kl], V = FO / 128;  // float4s per thread and 4 rows
+  const float* w = flat + P.k_off[kl] + (int64_t)32 * nb * FO;
+  floatx4 v4[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    v4[i] = i < 4 * V ? (floatx4)*reinterpret_cast<const floatx4_a4*>(w + 4 * (i * 256 + threadIdx.x)) : floatx4{0.f, 0.f, 0.f, 0.f};
+  float mx = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    if (i >= 4 * V) break;
+    const int e = 4 * (i * 256 + threadIdx.x);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      s_w[(e / FO) * (FO + 1) + e % FO + r] = v4[i][r];
+      mx = fmaxf(mx, fabsf(v4[i][r]));
+    }
+  }
+  const int s = split_scale(mx, s_m);
+  if (threadIdx.x == 0) reinterpret_cast<int*>(out + P.p_bse)[m * P.NB + nb] = s;
+  const float sc = f32s::pow2(s);
+  const int j = threadIdx.x & 31, g = (threadIdx.x >> 5) & 1;
+  f32s::half8* o = reinterpret_cast<f32s::half8*>(out + P.p_bs[m]) + (int64_t)nb * T * 128 + (threadIdx.x & 63);
+  for (int t = threadIdx.x >> 6; t < T; t += 4) {
+    float v[8];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) v[r] = s_w[j * (FO + 1) + cfeat(t / 2, 8 * (t % 2) + r, g)];
     const f32s::Planes p = f32s::split8(v, sc);
     o[t * 128] = p.h;
     o[t * 128 + 64] = p.l;
@@ -189,9 +203,8 @@ __global__ __launch_bounds__(256) void pack_kernel(MlpPlan P, PackSegs S, const 
       return;
     }
     case kHeads: return pack_heads(P, flat, out);
-    case kNatHeads: return pack_nat_heads(P, flat, out);
-    case kBwd4: return pack_bwd4(P, flat, out, m, u);
     case kSplitFwd: return pack_split(P, flat, out, m, blk, reinterpret_cast<float*>(s_w), s_m);
+    case kSplitBwd: return pack_split_bwd(P, flat, out, m, blk, reinterpret_cast<float*>(s_w), s_m);
   }
 }
 
@@ -205,19 +218,19 @@ PackSegs pack_segs(const MlpPlan& P) {
     ++S.n;
   };
   auto blocks16 = [](int64_t bytes) { return (bytes + 4095) / 4096; };  // 16 bytes per thread
-  for (int m = 0; m < P.n_mfma; ++m)
+  for (int m = 0; m < P.n_mfma; ++m) {
     if (P.p_fs[m] >= 0) add(kSplitFwd, m, P.nb_out[m]);
+    if (P.p_bs[m] >= 0) add(kSplitBwd, m, P.NB);
+  }
   for (int m = 0; m < P.n_mfma; ++m) {
     const int ks = P.ks_hid[m] + P.ks_enc[m];
     const int ke16 = P.ks_enc[m] == 0 ? 0 : (P.enc_L[m] == P.LX ? P.KX16 : P.KD16);
     if (P.p_fwd[m] >= 0)
       add(kFwd, m, blocks16((int64_t)P.nb_out[m] * 64 * 16 * (P.prec == 0 ? ks / 4 : P.ks_hid[m] / 8 + ke16)));
     if (P.p_bwd[m] >= 0) add(kBwd, m, blocks16((int64_t)P.nb_out[m] * (P.prec == 0 ? 4 : 2) * P.NB * 64 * 16));
-    if (P.p_bwd4[m] >= 0) add(kBwd4, m, blocks16((int64_t)2 * P.nb_out[m] * (P.W / 16) * 64 * 16));
   }
   for (int m = 0; m < P.n_mfma; ++m) add(kBias, m, (32 * P.nb_out[m] + 255) / 256);
   add(kHeads, 0, 1);
-  if (P.p_hs_nat >= 0) add(kNatHeads, 0, 1);
   return S;
 }
 

@@ -45,12 +45,6 @@ __host__ __device__ inline int enc_feat(int g, int e, int L) {
 // Hidden feature held by accumulator i of output block nb on lane half g.
 __host__ __device__ inline int cfeat(int nb, int i, int g) { return 32 * nb + 8 * (i / 4) + 4 * g + (i % 4); }
 
-// Register-resident fp32 dX chain (v_mfma_f32_16x16x4f32): one wave owns 16
-// samples, lane l = j + 16 q (j = sample, q = lane quarter).  Output block nb
-// (16 features) holds in accumulator r of lane (j, q) the feature
-//   G(nb, r, q) = 16 nb + 4 q + r
-// which is also what k-step 4 nb + r of the next layer reads on quarter q, so
-// a layer's output is the next layer's B operand in place.
 struct MlpPlan {
   int D, W, skip, LX, LD, rgb;
   int NB, NBR, WR;      // hidden blocks, rgb-branch blocks, rgb-branch width
@@ -74,13 +68,6 @@ struct MlpPlan {
   // packed byte offsets
   int64_t p_fwd[NERF_MAX_LAYERS], p_bwd[NERF_MAX_LAYERS], p_bias[NERF_MAX_LAYERS];
   int64_t p_head_sigma, p_head_rgb, packed_bytes;
-  // fp32 only: both heads in natural feature order (sigma: W weights + bias; rgb:
-  // [W/2][4] + bias[4]); -1 for bf16
-  int64_t p_hs_nat, p_hr_nat;
-  // fp32 only: transposed A operands of the register-resident dX chain, layers
-  // m >= 1 (k-step groups of 16 output features of layer m, each over the W/16
-  // blocks of its hidden input; -1 otherwise)
-  int64_t p_bwd4[NERF_MAX_LAYERS];
   // fp32, W = 256 with an rgb branch only (-1 otherwise): A operands of the forward
   // on the FP16 matrix cores, each weight split into two fp16 planes.  Per layer
   // units [output block of 32][k-step of 16][plane][lane][8], the k-steps and their
@@ -88,17 +75,17 @@ struct MlpPlan {
   // from p_fs[0] on).  p_fse: int32 per layer and output block (NB apart), the
   // power of two its weights are scaled by
   int64_t p_fs[NERF_MAX_LAYERS], fs_bytes, p_fse;
+  // the same for the dX chain, layers m >= 1: A[n = input hidden feature][k = output
+  // feature], units [input block of 32][k-step of 16], bs_bytes from p_bs[1] on
+  int64_t p_bs[NERF_MAX_LAYERS], bs_bytes, p_bse;
   int prec;
   // stash (elements per sample; fp32 or bf16 elements) and dz (floats per sample)
   int64_t st_encx, st_h[NERF_MAX_LAYERS], st_bott, st_rbr, st_encd, stash_per_sample;
   // ReLU bit masks (W = 256 with an rgb branch; -1 otherwise), written by the
-  // forward for the dX chain.  bf16: per 32-feature block nb and lane half g, D
-  // uint16 words, one per trunk layer (element (2 nb + g) D + l), 16 D elements
-  // in all; then 8 elements for the rgb branch (one uint16 per block and lane
-  // half).  fp32 (register-resident kernels, lane quarter q holding features
-  // 16 nb + 4 q + r): per trunk layer l and quarter q two uint32 words (element
-  // 8 l + 2 q + h, bit 4 (nb - 8 h) + r for nb = 8 h .. 8 h + 7), 8 D elements;
-  // then one word per quarter for the rgb branch's 8 blocks (element 8 D + q)
+  // forward for the dX chain: per 32-feature block nb and lane half g, D uint16
+  // words, one per trunk layer (word (2 nb + g) D + l, bit i = accumulator i; in
+  // bf16 the bit order of ws::nz_bits), then 8 words for the rgb branch (word 16 D +
+  // 2 nb + g).  16 D + 8 elements of the bf16 stash, half as many of the fp32 one.
   int64_t st_mask;
   int64_t dz_h[NERF_MAX_LAYERS], dz_bott, dz_rbr, dz_sigma, dz_rgb, dz_per_sample;
   // Samples per block of the stash and dz buffers.  A buffer of M samples with S
@@ -198,7 +185,7 @@ inline int mlp_make_plan(int D, int W, int skip, int LX, int LD, int prec, MlpPl
     ++m;
   }
   P.n_mfma = m;
-  // packed layout (p_fwd, p_bwd: not for the split form, whose kernels read p_fs and p_bwd4)
+  // packed layout (p_fwd, p_bwd: not for the split form, whose kernels read p_fs and p_bs)
   const bool split = prec == 0 && W == 256 && P.rgb && P.NBR == 4;
   int64_t b = 0;
   auto align = [&](int64_t a) { b = (b + a - 1) / a * a; };
@@ -237,14 +224,6 @@ inline int mlp_make_plan(int D, int W, int skip, int LX, int LD, int prec, MlpPl
   align(256);
   P.p_head_rgb = b;  // [2][16*NBR][4] fp32 + bias[4]
   if (P.rgb) b += (int64_t)2 * 16 * P.NBR * 16 + 16;
-  P.p_hs_nat = P.p_hr_nat = -1;
-  for (int i = 0; i < P.n_mfma; ++i) {
-    P.p_bwd4[i] = -1;
-    if (prec != 0 || i == 0) continue;
-    align(256);
-    P.p_bwd4[i] = b;
-    b += (int64_t)(2 * P.nb_out[i]) * (W / 16) * 64 * 4 * 4;
-  }
   align(4096);
   const int64_t fs0 = b;
   for (int i = 0; i < P.n_mfma; ++i) {
@@ -255,14 +234,16 @@ inline int mlp_make_plan(int D, int W, int skip, int LX, int LD, int prec, MlpPl
   align(256);
   P.p_fse = split ? b : -1;
   if (split) b += (int64_t)P.n_mfma * P.NB * 4;
-  if (prec == 0) {
-    align(256);
-    P.p_hs_nat = b;
-    b += (int64_t)W * 4 + 16;
-    align(256);
-    P.p_hr_nat = b;
-    if (P.rgb) b += (int64_t)P.WR * 16 + 16;
+  align(4096);
+  const int64_t bs0 = b;
+  for (int i = 0; i < P.n_mfma; ++i) {
+    P.p_bs[i] = split && i > 0 ? b : -1;
+    if (split && i > 0) b += (int64_t)P.nb_out[i] * 2 * P.NB * 2 * 1024;
   }
+  P.bs_bytes = b - bs0;
+  align(256);
+  P.p_bse = split ? b : -1;
+  if (split) b += (int64_t)P.n_mfma * P.NB * 4;
   align(256);
   P.packed_bytes = b;
   // stash (elements per sample)

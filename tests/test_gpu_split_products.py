@@ -141,3 +141,41 @@ def test_weight_grads_against_64_bits(nerf, net, m, least):
         for got, want in ((k[:W], x.T @ z), (b, z.sum(0))):
             err = (got.cpu().double() - want).norm()
             assert float(err) <= TOL * float(want.norm()), (name, float(err / want.norm()))
+
+
+@pytest.mark.parametrize("m", [1, 33, 8191, 8193])
+def test_dx_rows_against_64_bits(nerf, m):
+    """Every sample's dz rows of the 8x256 net against 64 bits on the GPU's ReLU branches, sample
+    by sample, with cotangents from 2^-40 to 2^40 (each sample has its own scale) and some zero."""
+    import ctypes
+    L = nerf._lib
+    mlp, w = _net(nerf)
+    x, d = _points(m, m)
+    rgb, sigma, stash = torch.empty((m, 3), device=DEV), torch.empty((m, 1), device=DEV), mlp._alloc_stash(m)
+    mlp._launch_forward(m, x, d, None, None, None, rgb, sigma, stash)
+    g = torch.Generator(device=DEV).manual_seed(m)
+    scale = 2.0 ** torch.randint(-40, 41, (m, 1), generator=g, device=DEV)
+    scale[torch.rand((m, 1), generator=g, device=DEV) < 0.1] = 0.0
+    g_rgb = scale * torch.randn((m, 3), generator=g, device=DEV)
+    g_sigma = scale * torch.randn((m, 1), generator=g, device=DEV)
+    dz = torch.full((m, mlp.dz_per_sample), float("nan"), device=DEV)
+    L.call("nerf_mlp_backward", ctypes.byref(mlp._desc), mlp.prec, L.ptr(mlp.packed), m, L.ptr(g_rgb), L.ptr(g_sigma),
+           L.ptr(rgb), L.ptr(sigma), L.ptr(stash), L.ptr(dz), L.stream())
+    pick = torch.unique(torch.cat([torch.arange(min(m, 200)), torch.arange(max(0, m - 200), m)]))
+    st, z = stash[pick].cpu().double(), dz[pick].cpu().double()
+    w = [torch.from_numpy(a).double() for a in w]
+    y = rgb[pick].cpu().double()
+    d_rgb = g_rgb[pick].cpu().double() * y * (1 - y)
+    d_sig = g_sigma[pick].cpu().double() * (sigma[pick].cpu() > 0)
+    h = lambda i: st[:, 64 + 256 * i:64 + 256 * (i + 1)]
+    dr = (d_rgb @ w[20].T) * (st[:, 64 + 9 * 256:64 + 9 * 256 + 128] > 0)
+    db = dr @ w[18][:256].T
+    want = {"rbr": (9 * 256, dr), "bottleneck": (8 * 256, db)}
+    cur = (db @ w[16].T + d_sig @ w[22].T) * (h(7) > 0)
+    want["h7"] = (7 * 256, cur)
+    for i in range(7, 0, -1):
+        cur = (cur @ w[2 * i][:256].T) * (h(i - 1) > 0)
+        want[f"h{i - 1}"] = ((i - 1) * 256, cur)
+    for name, (z0, v) in want.items():
+        err = (z[:, z0:z0 + v.shape[1]] - v).norm(dim=1)
+        assert bool((err <= TOL * v.norm(dim=1)).all()), (name, float((err / v.norm(dim=1)).nan_to_num().max()))
