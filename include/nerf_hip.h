@@ -308,6 +308,25 @@ int32_t nerf_adam_tf_state(int64_t n, float* var, float* m, float* v, const floa
 int32_t nerf_step_end(nerf_step_state* state, int32_t interval, float factor, float min_scale,
                       void* stream);
 
+/* One optimizer step over any number of models: nerf_step_begin, with `check` nerf_check_finite of every
+ * gradient's grad_n values (of the scaled loss), nerf_adam_tf_state and nerf_mlp_pack of every
+ * model, nerf_step_end, in a few launches (8 models per launch) with the same results.  `models` is a host
+ * array; reserved[0] of the state belongs to it between its launches. */
+typedef struct nerf_opt_model {
+  const nerf_mlp_desc* desc; /* host */
+  int32_t precision;
+  float* params; /* flat parameters and Adam's m and v, nerf_mlp_param_count values each */
+  float* m;
+  float* v;
+  const float* grad;
+  int64_t grad_n;
+  void* packed; /* nerf_mlp_packed_bytes */
+} nerf_opt_model;
+int32_t nerf_optimizer_step(int32_t n_models, const nerf_opt_model* models, float lr0,
+                            int32_t decay_steps, float decay_rate, float b1, float b2, float eps,
+                            nerf_step_state* state, int32_t check, int32_t interval, float factor,
+                            float min_scale, void* stream);
+
 /* ------------------------------------------------------------------------
  * Float64 layer kernels for the finite-difference check of the hand-written
  * backward (the FP64 gradient check; no counterpart in the reference, whose

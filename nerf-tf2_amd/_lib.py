@@ -29,6 +29,12 @@ class NerfMlpDesc(ctypes.Structure):
                 ("l_xyz", ctypes.c_int32), ("l_dir", ctypes.c_int32)]
 
 
+class NerfOptModel(ctypes.Structure):
+    _fields_ = [("desc", ctypes.POINTER(NerfMlpDesc)), ("precision", ctypes.c_int32), ("params", ctypes.c_void_p),
+                ("m", ctypes.c_void_p), ("v", ctypes.c_void_p), ("grad", ctypes.c_void_p),
+                ("grad_n", ctypes.c_int64), ("packed", ctypes.c_void_p)]
+
+
 _i32, _i64, _f32, _vp = ctypes.c_int32, ctypes.c_int64, ctypes.c_float, ctypes.c_void_p
 _dp = ctypes.POINTER(ctypes.c_double)
 _fp = ctypes.POINTER(ctypes.c_float)
@@ -65,6 +71,8 @@ _SIGS = {
     "nerf_step_begin": (_i32, [_vp, _f32, _i32, _f32, _f32, _f32, _vp]),
     "nerf_adam_tf_state": (_i32, [_i64, _vp, _vp, _vp, _vp, _f32, _vp, _vp]),
     "nerf_step_end": (_i32, [_vp, _i32, _f32, _f32, _vp]),
+    "nerf_optimizer_step": (_i32, [_i32, ctypes.POINTER(NerfOptModel), _f32, _i32, _f32, _f32, _f32, _f32, _vp, _i32,
+                                   _i32, _f32, _f32, _vp]),
     "nerf_proposal_interlevel": (_i32, [_i64, _i32, _i32] + [_vp] * 8 + [_f32, _i32, _vp]),
     "nerf_f64_encode": (_i32, [_i64, _i32, _vp, _vp, _vp]),
     "nerf_f64_dense_forward": (_i32, [_i64, _i32, _vp, _i32, _vp, _i32, _vp, _vp, _i32, _vp, _vp]),

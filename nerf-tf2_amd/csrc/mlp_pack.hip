@@ -3,6 +3,7 @@
 #include "common.h"
 #include "mlp_plan.h"
 #include "mlp_f32s.h"
+#include "optim.h"
 
 namespace {
 
@@ -36,6 +37,10 @@ __device__ float kernel_at(const MlpPlan& P, const float* flat, int kl, int row,
 }
 
 // One launch packs everything: a list of segments, each a run of workgroups.
+struct PackModels {
+  const float* flat[kOptModels];
+  char* packed[kOptModels];
+};
 enum PackKind : int { kFwd, kBwd, kBias, kHeads, kSplitFwd, kSplitBwd };
 constexpr int kMaxSegs = 3 * NERF_MAX_LAYERS + 1;
 struct PackSegs {
@@ -186,8 +191,13 @@ __device__ void pack_split_bwd(const MlpPlan& P, const float* __restrict__ flat,
   }
 }
 
-__global__ __launch_bounds__(256) void pack_kernel(MlpPlan P, PackSegs S, const float* __restrict__ flat,
-                                                   char* __restrict__ out) {
+// blockIdx.y: the model (all of one plan).  The first thread of the last launch of an optimizer
+// step also closes the step (state; null otherwise).
+__global__ __launch_bounds__(256) void pack_kernel(MlpPlan P, PackSegs S, PackModels A, StepState* state,
+                                                   StepEnd end) {
+  const float* __restrict__ flat = A.flat[blockIdx.y];
+  char* __restrict__ out = A.packed[blockIdx.y];
+  if (state && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) step_end(state, end);
   __shared__ floatx4 s_w[kSplitRows * 8];
   __shared__ float s_m[4];
   int seg = 0;
@@ -236,6 +246,18 @@ PackSegs pack_segs(const MlpPlan& P) {
 
 }  // namespace
 
+// Packs n <= kOptModels models of one plan in one launch; state: also close the step.
+void pack_models(const MlpPlan& P, int n, const float* const* flat, void* const* packed, StepState* state,
+                 const StepEnd& end, hipStream_t s) {
+  const PackSegs S = pack_segs(P);
+  PackModels A{};
+  for (int i = 0; i < n; ++i) {
+    A.flat[i] = flat[i];
+    A.packed[i] = reinterpret_cast<char*>(packed[i]);
+  }
+  pack_kernel<<<dim3((unsigned)S.first[S.n], (unsigned)n), 256, 0, s>>>(P, S, A, state, end);
+}
+
 int nerf_plan_from_desc(const nerf_mlp_desc* d, int prec, MlpPlan* p) {
   if (!d) return -1;
   return mlp_make_plan(d->depth, d->width, d->skip, d->l_xyz, d->l_dir, prec, p);
@@ -276,8 +298,7 @@ extern "C" int32_t nerf_mlp_pack(const nerf_mlp_desc* desc, int32_t precision, c
                                  void* packed, void* stream) {
   NERF_PLAN_OR_FAIL(desc, precision, P, "nerf_mlp_pack");
   NERF_CHECK_ARG(flat && packed, "nerf_mlp_pack: null pointer");
-  const PackSegs S = pack_segs(P);
-  pack_kernel<<<(unsigned)S.first[S.n], 256, 0, as_stream(stream)>>>(P, S, flat, reinterpret_cast<char*>(packed));
+  pack_models(P, 1, &flat, &packed, nullptr, StepEnd{}, as_stream(stream));
   NERF_LAUNCH_CHECK("nerf_mlp_pack");
   return NERF_OK;
 }

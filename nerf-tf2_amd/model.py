@@ -13,6 +13,7 @@ the autograd tape.
 """
 from __future__ import annotations
 
+import ctypes
 import math
 from dataclasses import dataclass
 from typing import Dict, List, Optional, Sequence, Tuple
@@ -309,7 +310,6 @@ class NerfMLP:
 
 
 def ctypes_ref(d):
-    import ctypes
     return ctypes.byref(d)
 
 
@@ -381,21 +381,20 @@ class AdamTF:
     def apply_gradients(self, grads: Sequence[Tensor], scaler: Optional["DynamicLossScaler"] = None) -> None:
         """One Adam step.  With a scaler the gradients are those of the scaled loss:
         they are checked for inf/NaN and unscaled, the step is skipped on overflow
-        and the scale is updated, all on the device."""
-        st, dev = ptr(self.state), stream(self.state.device)
-        call("nerf_step_begin", st, self.initial_lr, self.decay_steps, self.decay_rate, float(self.b1),
-             float(self.b2), dev)
-        if scaler is not None:
-            for g in grads:
-                call("nerf_check_finite", g.numel(), ptr(g), st + 8, dev)   # &state->overflow
-        for mm, m, v, g in zip(self.models, self.m, self.v, grads):
-            call("nerf_adam_tf_state", mm.n_params, ptr(mm.params), ptr(m), ptr(v), ptr(g.contiguous()),
-                 float(self.eps), st, stream(mm.device))
-            mm.repack()
-        if scaler is None:
-            call("nerf_step_end", st, self._NEVER, 1.0, 1.0, dev)
-        else:
-            call("nerf_step_end", st, scaler.interval, scaler.factor, scaler.min_scale, dev)
+        and the scale is updated, all on the device, in one call of the library."""
+        models = (_lib.NerfOptModel * len(self.models))()
+        keep = []                                              # contiguous copies live until the launches are queued
+        for o, mm, m, v, g in zip(models, self.models, self.m, self.v, grads):
+            if scaler is None:
+                g = g.contiguous()
+                keep.append(g)
+            o.desc, o.precision = ctypes.pointer(mm._desc), mm.prec
+            o.params, o.m, o.v, o.packed = ptr(mm.params), ptr(m), ptr(v), ptr(mm.packed)
+            o.grad, o.grad_n = ptr(g), g.numel()
+        end = (self._NEVER, 1.0, 1.0) if scaler is None else (scaler.interval, scaler.factor, scaler.min_scale)
+        call("nerf_optimizer_step", len(keep) if scaler is None else min(len(models), len(grads)), models,
+             self.initial_lr, self.decay_steps, self.decay_rate, float(self.b1), float(self.b2), float(self.eps),
+             ptr(self.state), int(scaler is not None), *end, stream(self.state.device))
 
 
 # ---------------------------------------------------------------------------
