@@ -11,9 +11,9 @@
 // workgroups share a CU (N = 2); N = 1 where the samples do not fill the chip, the
 // forward's rule.
 //
-// Bound by power and by the dz stores (9.9 KB a sample, 2.5 TB/s of them at the time
+// Bound by power and by the dz stores (9.9 KB a sample, 2.7 TB/s of them at the time
 // below).  Against the register-resident v_mfma_f32_16x16x4f32 kernel it replaced:
-// 6,570 -> 3,180 us at 786,432 samples, 1,665 -> 777 at 192,064, 188 -> 41 at 8,192, 142
+// 6,570 -> 2,850 us at 786,432 samples, 1,665 -> 680 at 192,064, 188 -> 40 at 8,192, 142
 // -> 31 at 1,000; the dz rows' error against 64 bits 6.3e-7 -> 3.9e-7 of their norm at
 // the last layer (h0), 3.1e-7 -> 1.7e-7 at the first of 256 inputs.
 //   rgb = sigmoid(z):  dz_rgb = d_rgb * rgb (1 - rgb)
@@ -50,7 +50,7 @@ __global__ __launch_bounds__(512, 4) void mlp_bwd_f32s_kernel(
       const_cast<float*>(stash) + base * P.stash_per_sample, 0, (int)(w_rows * P.stash_per_sample * 4), 0x00020000);
   const __amdgpu_buffer_rsrc_t rdz =
       __builtin_amdgcn_make_buffer_rsrc(dz + base * P.dz_per_sample, 0, (int)(w_rows * P.dz_per_sample * 4), 0x00020000);
-  const uint32_t row_z = (uint32_t)(j * P.dz_per_sample * 4), blk_z = (uint32_t)(32 * P.dz_per_sample * 4);
+  const uint32_t row_bytes = (uint32_t)(P.dz_per_sample * 4), row_z = j * row_bytes, blk_z = 32 * row_bytes;
   auto store_block = [&](const floatx16& v, int n, int64_t el) {  // features 8 q + 4 g + r of a block
 #pragma unroll
     for (int q = 0; q < 4; ++q)
@@ -175,11 +175,13 @@ __global__ __launch_bounds__(512, 4) void mlp_bwd_f32s_kernel(
 #pragma unroll
         for (int i = 0; i < 16; ++i) hi[n][i] = (w >> (16 * ((l - 1) & 1) + i)) & 1u ? hi[n][i] : 0.f;
       }
-      store_block(hi[n], n, el);
       if constexpr (l > 1) put_max((lds_f*)s_max[n], wv, j, g, max_abs(hi[n]));
     }
+    lds_barrier();  // every wave has read the tile; the largest values are there
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+      store_rows(hi[n], tile[n] + 2 * wv * 128, lane, rdz, n * blk_z + (uint32_t)(4 * el), row_bytes);
     if constexpr (l > 1) {
-      lds_barrier();  // every wave has read the tile; the largest values are there
 #pragma unroll
       for (int n = 0; n < N; ++n) {
         se[n] = scale_exp(get_max((const lds_f*)s_max[n], j));

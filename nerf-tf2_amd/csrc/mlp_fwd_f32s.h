@@ -39,7 +39,7 @@ __global__ __launch_bounds__(512, 4) void mlp_fwd_f32s_kernel(
     float* __restrict__ stash) {
   using namespace f32s;
   using C = NetC<W, D, SKIP, LX, LD>;
-  static_assert(W == 256 && C::KX == 32 && C::KD == 16 && SKIP >= 0 && SKIP + 1 < D,
+  static_assert(W == 256 && C::KX == 32 && C::KD == 16 && D % 2 == 0 && SKIP >= 0 && SKIP + 1 < D,
                 "split kernel is for the 8x256 NeRF MLP");
   static_assert(N == 1 || N == 2, "the rgb branch's 4 N output blocks go to waves 0 .. 4 N - 1");
   constexpr int TX = C::KX / 8, TD = C::KD / 8;
@@ -73,7 +73,7 @@ __global__ __launch_bounds__(512, 4) void mlp_fwd_f32s_kernel(
       STASH ? __builtin_amdgcn_make_buffer_rsrc(stash + base * P.stash_per_sample, 0,
                                                 (int)(w_rows * P.stash_per_sample * 4), 0x00020000)
             : rs;
-  const uint32_t row = (uint32_t)(j * P.stash_per_sample * 4), blk_row = (uint32_t)(32 * P.stash_per_sample * 4);
+  const uint32_t row_bytes = (uint32_t)(P.stash_per_sample * 4), row = j * row_bytes, blk_row = 32 * row_bytes;
   auto st4 = [&](floatx4 v, int n, int64_t el) {
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rst, row + n * blk_row + (uint32_t)(4 * el), 0, 0);
   };
@@ -126,6 +126,7 @@ __global__ __launch_bounds__(512, 4) void mlp_fwd_f32s_kernel(
   const lds_f4* bias = (const lds_f4*)&s_bias[8 * wv + 4 * g];
   floatx16 hi[N], lo[N];
   int se[N];  // scale of this lane's sample in the tile
+  uint32_t mw[N];
   lds_barrier();
   encode(std::integral_constant<int, LX>{}, 0, P.st_encx, true);
 #pragma unroll
@@ -184,18 +185,16 @@ __global__ __launch_bounds__(512, 4) void mlp_fwd_f32s_kernel(
         }
       }
       put_max((lds_f*)s_max[n], wv, j, g, mx);
-      if constexpr (STASH) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          st4(floatx4{hi[n][4 * q], hi[n][4 * q + 1], hi[n][4 * q + 2], hi[n][4 * q + 3]}, n, st_off + 8 * q + 4 * g);
-      }
       if constexpr (STASH && l < D) {
-        // ReLU word of this block, lane half and layer
+        // ReLU words of this block and lane half, two layers per store
         uint32_t w = 0u;
 #pragma unroll
         for (int i = 0; i < 16; ++i) w |= (hi[n][i] > 0.f ? 1u : 0u) << i;
-        __builtin_amdgcn_raw_buffer_store_b16((unsigned short)w, rst,
-                                              row + n * blk_row + (uint32_t)(4 * P.st_mask + 2 * ((2 * wv + g) * D + l)), 0, 0);
+        if constexpr ((l & 1) == 0)
+          mw[n] = w;
+        else
+          __builtin_amdgcn_raw_buffer_store_b32(mw[n] | (w << 16), rst,
+                                                row + n * blk_row + (uint32_t)(4 * P.st_mask + 2 * ((2 * wv + g) * D + l - 1)), 0, 0);
       }
       if constexpr (l == D - 1) {
         // sigma head on h_{D-1} (model.py:374-375): this block's part of the dot product
@@ -216,6 +215,8 @@ __global__ __launch_bounds__(512, 4) void mlp_fwd_f32s_kernel(
     for (int n = 0; n < N; ++n) {
       se[n] = scale_exp(get_max((const lds_f*)s_max[n], j));
       const float sc = pow2(se[n]);
+      if constexpr (STASH)
+        store_rows(hi[n], tile[n] + 2 * wv * 128, lane, rst, n * blk_row + (uint32_t)(4 * st_off), row_bytes);
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         float v[8];
