@@ -143,6 +143,41 @@ def test_weight_grads_against_64_bits(nerf, net, m, least):
             assert float(err) <= TOL * float(want.norm()), (name, float(err / want.norm()))
 
 
+@pytest.mark.parametrize("m", [129, 4099])
+@pytest.mark.parametrize("width", [32, 64, 128, 160, 256])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_weight_grads_of_growing_rows(nerf, width, m, shift):
+    """dz grows by 2^30 over every 128 rows, and every second feature is zero in the larger half of
+    them: its gradients are sums of small terms only.  Rows on 16 bytes and 4 bytes off them
+    (shift); every tile shape, whole and in part."""
+    import ctypes
+    L = nerf._lib
+    cfg = nerf.MLPConfig(depth=3, width=width, skip=1)
+    mlp = nerf.NerfMLP("fine", cfg, "fp32", seed=1, device=DEV)
+    d = ctypes.byref(mlp._desc)
+    g = torch.Generator(device=DEV).manual_seed(m)
+    stash = torch.randn(m * mlp.stash_per_sample + shift, generator=g, device=DEV)[shift:].view(m, -1).relu_()
+    dz = torch.randn(m * mlp.dz_per_sample + shift, generator=g, device=DEV)[shift:].view(m, -1)
+    i = torch.arange(m, device=DEV)[:, None] % 128
+    dz *= 2.0 ** (i * 30 // 128)
+    stash[:, ::2] *= i < 64
+    work = torch.empty(int(L.load().nerf_mlp_wgrad_workspace_bytes(d, m)), dtype=torch.uint8, device=DEV)
+    grad = torch.full((mlp.n_params,), float("nan"), device=DEV)
+    L.call("nerf_mlp_weight_grads", d, 0, m, stash.data_ptr(), dz.data_ptr(), L.ptr(grad), 0, L.ptr(work), work.numel(),
+           L.stream())
+    enc, off = 2 * ((2 + 3 * cfg.l_xyz + 7) // 8 * 8), 0
+    for j, (name, fi, fo) in enumerate(cfg.layer_shapes()[:3]):
+        k = grad[off:off + fi * fo].view(fi, fo)[:width].cpu().double()
+        off += fi * fo + fo
+        if j == 0:
+            continue
+        x = stash[:, enc + (j - 1) * width:enc + j * width].cpu().double()
+        want = x.T @ dz[:, j * width:(j + 1) * width].cpu().double()
+        for half in (0, 1):
+            err = (k[half::2] - want[half::2]).norm()
+            assert float(err) <= TOL * float(want[half::2].norm()), (name, half, float(err / want[half::2].norm()))
+
+
 @pytest.mark.parametrize("m", [1, 33, 8191, 8193])
 def test_dx_rows_against_64_bits(nerf, m):
     """Every sample's dz rows of the 8x256 net against 64 bits on the GPU's ReLU branches, sample
