@@ -191,72 +191,154 @@ __device__ __forceinline__ float lane_shift_up(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x138, 0xF, 0xF, true));
 }
 
-// Lane i ^ J's value (J < 64): DPP quad_perm for 1 and 2, row_ror:8 for 8,
-// ds_swizzle (bit mode, within 32 lanes) for 4 and 16, ds_bpermute for 32.
+// Lane i ^ J's value for J = 1, 2, 3, 4, 7, 8, 15, 16, 31, 63: DPP moves (quad_perm,
+// row_half_mirror = ^7, row_ror:8 = ^8, row_mirror = ^15) and their products; across
+// rows of 16 and halves of 32, a lane swap and a select.
 template <int J>
-__device__ __forceinline__ float lane_xor(float v) {
-  const int x = __builtin_bit_cast(int, v);
-  int r;
-  if constexpr (J == 1) r = __builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, false);
-  else if constexpr (J == 2) r = __builtin_amdgcn_mov_dpp(x, 0x4E, 0xF, 0xF, false);
-  else if constexpr (J == 8) r = __builtin_amdgcn_mov_dpp(x, 0x128, 0xF, 0xF, false);
-  else if constexpr (J == 4 || J == 16) r = __builtin_amdgcn_ds_swizzle(x, 0x1F | (J << 10));
-  else r = __builtin_bit_cast(int, shfl_xor(v, J));
-  return __builtin_bit_cast(float, r);
+__device__ __forceinline__ int lane_xor(int x, int lane) {
+  if constexpr (J == 1) return __builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, false);
+  else if constexpr (J == 2) return __builtin_amdgcn_mov_dpp(x, 0x4E, 0xF, 0xF, false);
+  else if constexpr (J == 3) return __builtin_amdgcn_mov_dpp(x, 0x1B, 0xF, 0xF, false);
+  else if constexpr (J == 7) return __builtin_amdgcn_mov_dpp(x, 0x141, 0xF, 0xF, false);
+  else if constexpr (J == 8) return __builtin_amdgcn_mov_dpp(x, 0x128, 0xF, 0xF, false);
+  else if constexpr (J == 15) return __builtin_amdgcn_mov_dpp(x, 0x140, 0xF, 0xF, false);
+  else if constexpr (J == 4) return lane_xor<3>(lane_xor<7>(x, lane), lane);
+  else if constexpr (J == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);  // rows (0, 0, 2, 2) and (1, 1, 3, 3)
+    return lane & 16 ? r[0] : r[1];
+  } else if constexpr (J == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);  // halves (0, 0) and (1, 1)
+    return lane & 32 ? r[0] : r[1];
+  } else if constexpr (J == 31) return lane_xor<15>(lane_xor<16>(x, lane), lane);
+  else {
+    static_assert(J == 63, "");
+    return lane_xor<31>(lane_xor<32>(x, lane), lane);
+  }
 }
 
-// Count of the first n entries of the ascending row a that are <= x (LE) or
-// < x (!LE): a branch-free binary search with a fixed trip count.
+template <int J>
+__device__ __forceinline__ float lane_xor_f(float x, int lane) {
+  return __builtin_bit_cast(float, lane_xor<J>(__builtin_bit_cast(int, x), lane));
+}
+
+// The smaller of a and b where lim is INT_MIN, the larger where it is INT_MAX (v_med3_i32).
+__device__ __forceinline__ int med3(int a, int b, int lim) {
+  const int lo = a < b ? a : b, hi = a < b ? b : a;
+  const int c = hi < lim ? hi : lim;
+  return lo > c ? lo : c;
+}
+
+// Ascending sort of the wave's 64 R integers; element e = R lane + r.  Bitonic merges
+// whose first step pairs e with e ^ (2 k - 1), so that every comparison puts the smaller
+// value at the smaller index: which of the two a lane keeps depends on one bit of its
+// number, one v_med3_i32 against that bit's limit (lim).  With two elements a lane the
+// steps between neighbours stay inside the lane.
+template <int R>
+__device__ __forceinline__ void wave_sort(int (&v)[R], int lane) {
+  static_assert(R == 1 || R == 2, "");
+  int lim[6];
+#pragma unroll
+  for (int b = 0; b < 6; ++b) lim[b] = (int)(0x80000000u + (uint32_t)((lane << (31 - b)) >> 31));  // INT_MIN or INT_MAX
+  auto in_lane = [&]() {
+    if constexpr (R == 2) {
+      const int a = v[0], b = v[1];
+      v[0] = a < b ? a : b;
+      v[1] = a < b ? b : a;
+    }
+  };
+  auto step = [&](auto jc, auto mirror_c, int b) {
+    constexpr int J = decltype(jc)::value;
+    constexpr bool kMirror = decltype(mirror_c)::value;
+    int o[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) o[r] = lane_xor<J>(v[kMirror ? R - 1 - r : r], lane);
+#pragma unroll
+    for (int r = 0; r < R; ++r) v[r] = med3(v[r], o[r], lim[b]);
+  };
+  auto merge = [&](auto bc) {  // sorted runs of 2^b lanes -> of 2^(b + 1) lanes
+    constexpr int B = decltype(bc)::value;
+    step(std::integral_constant<int, (2 << B) - 1>{}, std::true_type{}, B);
+    if constexpr (B >= 5) step(std::integral_constant<int, 16>{}, std::false_type{}, 4);
+    if constexpr (B >= 4) step(std::integral_constant<int, 8>{}, std::false_type{}, 3);
+    if constexpr (B >= 3) step(std::integral_constant<int, 4>{}, std::false_type{}, 2);
+    if constexpr (B >= 2) step(std::integral_constant<int, 2>{}, std::false_type{}, 1);
+    if constexpr (B >= 1) step(std::integral_constant<int, 1>{}, std::false_type{}, 0);
+    in_lane();
+  };
+  in_lane();
+  merge(std::integral_constant<int, 0>{});
+  merge(std::integral_constant<int, 1>{});
+  merge(std::integral_constant<int, 2>{});
+  merge(std::integral_constant<int, 3>{});
+  merge(std::integral_constant<int, 4>{});
+  merge(std::integral_constant<int, 5>{});
+}
+
+// Integers in the order of the floats (its own inverse); NaNs lie beyond the infinities.
+__device__ __forceinline__ int order_key(int x) { return x ^ ((x >> 31) & 0x7FFFFFFF); }
+
+// Count of the first N entries of the ascending row a that are <= x (LE) or < x (!LE),
+// in steps of falling powers of two without a branch.  N = 2^k - 1 needs nothing more;
+// N = 2^k ends with one more comparison; for any other N the row has to be continued
+// to the next 2^k - 1 entries with +infinity, and the count is held to N.
 template <int N, bool LE>
 __device__ __forceinline__ int count_below(const float* a, float x) {
-  int c = 0;
+  constexpr bool kPow2 = (N & (N - 1)) == 0, kFull = (N & (N + 1)) == 0;
+  constexpr int kTop = 1 << (31 - __builtin_clz(N));
+  const float* p = a;  // a + the count so far
 #pragma unroll
-  for (int step = 1 << (31 - __builtin_clz(N)); step > 0; step >>= 1) {
-    if (c + step <= N) {
-      const float e = a[c + step - 1];
-      if (LE ? (e <= x) : (e < x)) c += step;
-    }
+  for (int step = kPow2 ? N / 2 : kTop; step > 0; step >>= 1) {
+    const float e = p[step - 1];
+    p += (LE ? (e <= x) : (e < x)) ? step : 0;
   }
-  return c;
+  if (kPow2) p += (LE ? (*p <= x) : (*p < x)) ? 1 : 0;
+  const int c = (int)(p - a);
+  return kPow2 || kFull ? c : (c < N ? c : N);
 }
 
-// The same computation for the shapes of the reference configuration and the
-// learned proposal (n_fine = 128, n_coarse <= 64, each a multiple of 8 or with
-// its Eigen tail), organised for throughput: every cross-lane read of the pdf /
-// cdf passes is a v_readlane of an unrolled, compile-time lane; the searchsorted
-// is a fixed-trip binary search; the merge sorts the 128 fine values with a
-// bitonic network in the wave (2 per lane), places each value by rank (its sorted
-// index + the number of coarse values <= it; a coarse value: its index + the
-// number of fine values < it — coarse first on ties, as the rank merge above), and
-// writes the row from LDS with coalesced stores.  Equal floats are
-// indistinguishable, so the output equals the sorted set bit for bit.
-template <int NC, bool COMP>
-__global__ __launch_bounds__(256) void fine128_kernel(
+// The same computation for the shapes in use (32, 48 or 64 coarse bins, 64 or 128 fine
+// samples), organised for throughput.  Instruction issue bounds it: the first form of
+// this kernel issued 738 vector instructions a ray, 2,950 of the 2,900 cycles a ray took
+// on its SIMD.  So: row addresses are scalar (the wave's number is made uniform); every
+// cross-lane read of the cdf passes is a DPP move or a v_readlane; the sort works on
+// integers (no canonicalising), two instructions a step and value; the searches have
+// neither a branch nor a remainder test; and only the coarse values look up their place
+// (index + the number of fine values below it, coarse first on ties): they are put down
+// in a cleared row, and each remaining place takes the next fine value, found by
+// counting the coarse values before it (a ballot) instead of by a search per fine value.
+// Equal floats are indistinguishable, so the output equals the sorted set bit for bit.
+// 32,768 rays, kernel trace: 64 + 128 samples 41.9 -> 27.7 us (84 MB with the coarse
+// kernel's: 2.3 TB/s here); as calls one after another, 32 + 128, by fine_kernel before:
+// 98 -> 23 us, 64 + 64: 45 -> 19 us.
+template <int NC, int NF, bool COMP>
+__global__ __launch_bounds__(256) void fine_wave_kernel(
     int64_t n_rays, const float* __restrict__ ro, const float* __restrict__ rd,
     const float* __restrict__ bin_weights, const float* __restrict__ bin_edges,
     const float* __restrict__ bin_widths, const float* __restrict__ t_c,
     const float* __restrict__ u_vals, float* __restrict__ t_out, int32_t* __restrict__ idx_out,
     float* __restrict__ tf_out, float* __restrict__ xyz, float* __restrict__ dirs,
     float* __restrict__ cdf_out) {
-  constexpr int NF = 128, S = NC + NF;
-  static_assert(NC >= 2 && NC <= 64, "one coarse bin per lane");
-  __shared__ float s_agg[kWaves][NC + 1];
-  __shared__ float s_pdf[kWaves][NC];
-  __shared__ float s_left[kWaves][NC];
-  __shared__ float s_tc[kWaves][NC];
+  constexpr int S = NC + NF, R = NF / 64, Q = (S + 63) / 64;
+  static_assert(NC >= 2 && NC <= 64 && NC % 8 == 0 && NF == 64 * R, "one coarse bin per lane, R fine samples");
+  constexpr int kFree = 0x7FC0A5A5;  // a place no coarse value has taken
+  __shared__ float s_agg[kWaves][65];
+  __shared__ float2 s_bin[kWaves][64];  // pdf, left edge
   __shared__ float s_sorted[kWaves][NF];
-  __shared__ float s_row[kWaves][S];
+  __shared__ int s_row[kWaves][64 * Q];
   const int lane = threadIdx.x & 63;
-  const int w = threadIdx.x >> 6;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t ray = (int64_t)blockIdx.x * kWaves + w;
   if (ray >= n_rays) return;  // wave-uniform; no block-level barriers below
 
   // ---- pdf and cdf over the coarse bins (ray_utils.py:335-345)
-  const bool on = lane < NC;
-  const float wv = on ? bin_weights[ray * NC + lane] : 0.f;
-  const float width = on ? bin_widths[ray * NC + lane] : 0.f;
-  const float left = on ? bin_edges[ray * (NC + 1) + lane] : 0.f;
-  const float tc = on ? t_c[ray * NC + lane] : 0.f;
+  const bool on = NC == 64 || lane < NC;
+  const float wv = on ? (bin_weights + ray * NC)[lane] : 0.f;
+  const float width = on ? (bin_widths + ray * NC)[lane] : 0.f;
+  const float left = on ? (bin_edges + ray * (NC + 1))[lane] : 0.f;
+  const float tc = on ? (t_c + ray * NC)[lane] : 0.f;
+  float u[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) u[r] = (u_vals + ray * NF)[lane + 64 * r];
   const float wp = fadd(wv, 1e-5f);
   const float prod = fmul(wp, width);
   float pdf, agg;
@@ -267,19 +349,18 @@ __global__ __launch_bounds__(256) void fine128_kernel(
     pdf = fdiv(wp, denom);
     agg = comp_ratio(sh, sl, denom);
   } else {
-    constexpr int NV = (NC / 8) * 8;
-    // lane j < 8: packet sum P_j = prod_j + prod_{j+8} + ... in that order
+    // lane j < 8: packet sum P_j = prod_j + prod_{j+8} + ... in that order (the other
+    // lanes' sums wrap round and are not used)
     float pj = prod;
 #pragma unroll
-    for (int i = 1; 8 * i < NV; ++i) pj = fadd(pj, shfl_down(prod, 8 * i));
-    float P[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) P[j] = lane_value(pj, j);
-    float tail = 0.f;
-#pragma unroll
-    for (int i = NV; i < NC; ++i) tail = fadd(tail, lane_value(prod, i));
-    const float denom =
-        fadd(tail, fadd(fadd(fadd(P[0], P[4]), fadd(P[2], P[6])), fadd(fadd(P[1], P[5]), fadd(P[3], P[7]))));
+    for (int i = 1; 8 * i < NC; ++i)
+      pj = fadd(pj, __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(4 * lane + 32 * i, __builtin_bit_cast(int, prod))));
+    // lane 0: ((P0 + P4) + (P2 + P6)) + ((P1 + P5) + (P3 + P7)); the 8-wide reduction's
+    // tail is empty
+    pj = fadd(pj, lane_xor_f<4>(pj, lane));
+    pj = fadd(pj, lane_xor_f<2>(pj, lane));
+    pj = fadd(pj, lane_xor_f<1>(pj, lane));
+    const float denom = fadd(0.f, lane_value(pj, 0));
     pdf = fdiv(wp, denom);
     const float cw = fmul(pdf, width);
     // sequential inclusive prefix: after step s lane i holds cw_{i-s} + ... + cw_i added
@@ -294,77 +375,39 @@ __global__ __launch_bounds__(256) void fine128_kernel(
     if (on) cdf_out[ray * (NC + 1) + 1 + lane] = agg;
   }
   if (lane == 0) s_agg[w][0] = 0.f;
-  if (on) {
-    s_agg[w][lane + 1] = agg;
-    s_pdf[w][lane] = pdf;
-    s_left[w][lane] = left;
-    s_tc[w][lane] = tc;
-  }
+  // the last bin's cdf is no inner edge: +infinity from there on (count_below)
+  s_agg[w][lane + 1] = lane < NC - 1 ? agg : __builtin_inff();
+  s_bin[w][lane] = make_float2(pdf, left);
+#pragma unroll
+  for (int i = 0; i < Q; ++i) s_row[w][lane + 64 * i] = kFree;
   wave_sync();
 
-  // ---- inverse transform (ray_utils.py:355-377), fine samples lane and lane + 64
-  float v[2];
+  // ---- inverse transform (ray_utils.py:355-377), fine samples lane + 64 r
+  int key[R], idx[R];
 #pragma unroll
-  for (int r = 0; r < 2; ++r) {
-    const int q = lane + 64 * r;
-    const float u = u_vals[ray * NF + q];
-    const int idx = count_below<NC - 1, true>(&s_agg[w][1], u);  // searchsorted(agg[1:-1], u, 'right')
-    const float agg_ = s_agg[w][idx];
-    float pdf_ = s_pdf[w][idx];
-    const float left_ = s_left[w][idx];
-    const float mask = pdf_ < 1e-8f ? 0.f : 1.f;
-    pdf_ = fmaxf(pdf_, 1e-8f);
-    v[r] = fadd(fmul(fdiv(fsub(u, agg_), pdf_), mask), left_);
-    if (idx_out) idx_out[ray * NF + q] = idx;
-    if (tf_out) tf_out[ray * NF + q] = v[r];
+  for (int r = 0; r < R; ++r) idx[r] = count_below<NC - 1, true>(&s_agg[w][1], u[r]);  // searchsorted(agg[1:-1], u, 'right')
+  float v[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const float agg_ = s_agg[w][idx[r]];
+    const float2 bin = s_bin[w][idx[r]];
+    const float mask = bin.x < 1e-8f ? 0.f : 1.f;
+    const float pdf_ = fmaxf(bin.x, 1e-8f);
+    v[r] = fadd(fmul(fdiv(fsub(u[r], agg_), pdf_), mask), bin.y);
+    key[r] = order_key(__builtin_bit_cast(int, v[r]));
   }
-
-  // ---- bitonic sort of the 128 fine values; element e = lane + 64 r
-  auto stage = [&](auto kc, auto jc) {
-    constexpr int k = decltype(kc)::value, j = decltype(jc)::value;
-    if constexpr (j == 64) {  // partner in the same lane (k == 128: ascending)
-      const float a = v[0], b = v[1];
-      v[0] = fminf(a, b);
-      v[1] = fmaxf(a, b);
-    } else {
-      const bool lower = (lane & j) == 0;
 #pragma unroll
-      for (int r = 0; r < 2; ++r) {
-        const int e = lane + 64 * r;
-        const bool asc = (e & k) == 0;
-        const float o = lane_xor<j>(v[r]);
-        v[r] = (lower == asc) ? fminf(v[r], o) : fmaxf(v[r], o);
-      }
-    }
-  };
-  auto merge = [&](auto kc) {
-    constexpr int k = decltype(kc)::value;
-    if constexpr (k >= 128) stage(kc, std::integral_constant<int, 64>{});
-    if constexpr (k >= 64) stage(kc, std::integral_constant<int, 32>{});
-    if constexpr (k >= 32) stage(kc, std::integral_constant<int, 16>{});
-    if constexpr (k >= 16) stage(kc, std::integral_constant<int, 8>{});
-    if constexpr (k >= 8) stage(kc, std::integral_constant<int, 4>{});
-    if constexpr (k >= 4) stage(kc, std::integral_constant<int, 2>{});
-    stage(kc, std::integral_constant<int, 1>{});
-  };
-  merge(std::integral_constant<int, 2>{});
-  merge(std::integral_constant<int, 4>{});
-  merge(std::integral_constant<int, 8>{});
-  merge(std::integral_constant<int, 16>{});
-  merge(std::integral_constant<int, 32>{});
-  merge(std::integral_constant<int, 64>{});
-  merge(std::integral_constant<int, 128>{});
-  s_sorted[w][lane] = v[0];
-  s_sorted[w][lane + 64] = v[1];
+  for (int r = 0; r < R; ++r) {
+    if (idx_out) (idx_out + ray * NF)[lane + 64 * r] = idx[r];
+    if (tf_out) (tf_out + ray * NF)[lane + 64 * r] = v[r];
+  }
+  wave_sort<R>(key, lane);
+#pragma unroll
+  for (int r = 0; r < R; ++r) s_sorted[w][R * lane + r] = __builtin_bit_cast(float, order_key(key[r]));
   wave_sync();
 
-  // ---- ranks -> row in LDS -> coalesced stores (ray_utils.py:380-398)
-#pragma unroll
-  for (int r = 0; r < 2; ++r) {
-    const int e = lane + 64 * r;
-    s_row[w][e + count_below<NC, true>(&s_tc[w][0], v[r])] = v[r];
-  }
-  if (on) s_row[w][lane + count_below<NF, false>(&s_sorted[w][0], tc)] = tc;
+  // ---- sort(concat(t_coarse, t_fine)) (ray_utils.py:380-398)
+  if (on) s_row[w][lane + count_below<NF, false>(&s_sorted[w][0], tc)] = __builtin_bit_cast(int, tc);
   wave_sync();
   float o3[3] = {0.f, 0.f, 0.f}, d3[3] = {0.f, 0.f, 0.f};
   if (xyz) {
@@ -374,16 +417,27 @@ __global__ __launch_bounds__(256) void fine128_kernel(
       d3[c] = rd[3 * ray + c];
     }
   }
-  float* trow = t_out + ray * S;
-  for (int i = lane; i < S; i += 64) {
-    const float t = s_row[w][i];
-    trow[i] = t;
-    if (xyz) {
-      const int64_t m = ray * S + i;
+  int before = 0;  // coarse values in the places below 64 i
 #pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        xyz[3 * m + c] = fadd(o3[c], fmul(t, d3[c]));
-        dirs[3 * m + c] = d3[c];
+  for (int i = 0; i < Q; ++i) {
+    const int pos = lane + 64 * i;
+    const int c = s_row[w][pos];
+    const uint64_t taken = __ballot(c != kFree);
+    int k = pos - before -
+            (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(taken >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)taken, 0u));
+    before += __popcll(taken);
+    k = k < NF ? k : NF - 1;  // (only where coarse values were not ascending and shared a place)
+    const float f = s_sorted[w][k];
+    const float t = c != kFree ? __builtin_bit_cast(float, c) : f;
+    if (S % 64 == 0 || pos < S) {
+      (t_out + ray * S)[pos] = t;
+      if (xyz) {
+        const int64_t m = ray * S + pos;
+#pragma unroll
+        for (int c3 = 0; c3 < 3; ++c3) {
+          xyz[3 * m + c3] = fadd(o3[c3], fmul(t, d3[c3]));
+          dirs[3 * m + c3] = d3[c3];
+        }
       }
     }
   }
@@ -416,21 +470,24 @@ extern "C" int32_t nerf_create_input_batch_fine(int64_t n_rays, int32_t n_coarse
   const unsigned grid = (unsigned)((n_rays + kWaves - 1) / kWaves);
   hipStream_t s = as_stream(stream);
   const bool comp = cdf_mode == NERF_CDF_COMPENSATED;
-#define NERF_FINE128(NC_, C_)                                                                    \
-  fine128_kernel<NC_, C_><<<grid, 64 * kWaves, 0, s>>>(n_rays, rays_o, rays_d, bin_weights,      \
-                                                      bin_edges, bin_widths, t_vals_coarse,      \
-                                                      u_vals, t_vals, piece_idxs, t_vals_fine,   \
-                                                      xyz_inputs, dir_inputs, cdf)
-  if (n_fine == 128 && n_coarse == 64) {
-    if (comp) NERF_FINE128(64, true); else NERF_FINE128(64, false);
-  } else if (n_fine == 128 && n_coarse == 48) {
-    if (comp) NERF_FINE128(48, true); else NERF_FINE128(48, false);
-  } else {
-    fine_kernel<<<grid, 64 * kWaves, 0, s>>>(
-        n_rays, n_coarse, n_fine, rays_o, rays_d, bin_weights, bin_edges, bin_widths, t_vals_coarse,
-        u_vals, t_vals, piece_idxs, t_vals_fine, xyz_inputs, dir_inputs, comp ? 1 : 0, cdf);
-  }
-#undef NERF_FINE128
+#define NERF_FINE(NC_, NF_)                                                                       \
+  if (n_coarse == NC_ && n_fine == NF_) {                                                         \
+    const auto k = comp ? fine_wave_kernel<NC_, NF_, true> : fine_wave_kernel<NC_, NF_, false>;   \
+    k<<<grid, 64 * kWaves, 0, s>>>(n_rays, rays_o, rays_d, bin_weights, bin_edges, bin_widths,    \
+                                   t_vals_coarse, u_vals, t_vals, piece_idxs, t_vals_fine,        \
+                                   xyz_inputs, dir_inputs, cdf);                                  \
+  } else
+  NERF_FINE(64, 128)
+  NERF_FINE(48, 128)
+  NERF_FINE(32, 128)
+  NERF_FINE(64, 64)
+  NERF_FINE(48, 64)
+  NERF_FINE(32, 64)
+  // other shapes: loops instead of unrolled lanes, a quadratic rank merge
+  fine_kernel<<<grid, 64 * kWaves, 0, s>>>(
+      n_rays, n_coarse, n_fine, rays_o, rays_d, bin_weights, bin_edges, bin_widths, t_vals_coarse,
+      u_vals, t_vals, piece_idxs, t_vals_fine, xyz_inputs, dir_inputs, comp ? 1 : 0, cdf);
+#undef NERF_FINE
   NERF_LAUNCH_CHECK("nerf_create_input_batch_fine");
   return NERF_OK;
 }
