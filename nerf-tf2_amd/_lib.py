@@ -112,8 +112,16 @@ def check(rc: int, name: str) -> None:
         raise RuntimeError(msg or f"{name} failed with {rc}")
 
 
+_fns: dict = {}      # bound entry points of the loaded library
+
+
 def call(name: str, *args) -> None:
-    check(getattr(load(), name)(*args), name)
+    fn = _fns.get(name)
+    if fn is None:
+        fn = _fns[name] = getattr(load(), name)
+    rc = fn(*args)
+    if rc != NERF_OK:
+        check(rc, name)
 
 
 def ptr(t: Optional[torch.Tensor]):
@@ -128,7 +136,12 @@ def ptr(t: Optional[torch.Tensor]):
 
 
 def stream(device: Optional[torch.device] = None):
-    return torch.cuda.current_stream(device).cuda_stream
+    """The calling thread's current stream on `device` (None, or one without an index: the
+    current device), as the raw handle; building a Stream object for it took 4 to 8 us a call."""
+    if device is not None and device.type != "cuda":
+        raise ValueError(f"expected a cuda device, got {device}")
+    index = None if device is None else device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def desc(depth=8, width=256, skip=4, l_xyz=10, l_dir=4) -> NerfMlpDesc:

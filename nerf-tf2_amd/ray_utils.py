@@ -182,6 +182,9 @@ class CompositeFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, sample_rgb, sigma, t_vals, white_bg: bool):
         w, rgb, depth, acc = _composite_fwd(sigma, sample_rgb, t_vals, white_bg)
+        # outputs that no loss reads arrive as None, which the kernel takes, instead of as
+        # zeros filled by a launch each
+        ctx.set_materialize_grads(False)
         ctx.save_for_backward(sample_rgb if sample_rgb is not None else sigma, sigma, t_vals)
         ctx.has_rgb = sample_rgb is not None
         ctx.white_bg = white_bg
@@ -190,6 +193,8 @@ class CompositeFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g_w, g_rgb, g_depth, g_acc):
         sample_rgb, sigma, t_vals = ctx.saved_tensors
+        if g_w is None and g_rgb is None and g_depth is None and g_acc is None:
+            return None, None, None, None
         if not ctx.has_rgb:
             sample_rgb = None
         d_sigma, d_rgb = _composite_bwd(sigma, sample_rgb, t_vals, ctx.white_bg, g_rgb, g_depth, g_acc, g_w)
