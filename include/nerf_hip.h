@@ -230,6 +230,17 @@ int32_t nerf_mlp_weight_grads(const nerf_mlp_desc* desc, int32_t precision, int6
                               int32_t accumulate, void* workspace, int64_t workspace_bytes,
                               void* stream);
 
+/* nerf_mlp_backward and nerf_mlp_weight_grads in one call that writes no dz: for the
+ * descriptions and precisions for which nerf_mlp_has_backward_grads is 1 (the
+ * density-only net of four 64-wide layers in bf16), others are rejected with
+ * NERF_ERR_INVALID_ARG.  The stash, grad_flat, accumulate, the workspace (the same
+ * size) and an empty batch are as there; d_sigma, sigma: (M,1).  No counterpart in the
+ * reference (GradientTape through the model). */
+int32_t nerf_mlp_has_backward_grads(const nerf_mlp_desc* desc, int32_t precision);
+int32_t nerf_mlp_backward_grads(const nerf_mlp_desc* desc, int32_t precision, const void* packed, int64_t M,
+                                const float* d_sigma, const float* sigma, const void* stash, float* grad_flat,
+                                int32_t accumulate, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* nerf_mlp_weight_grads without a workspace and without allocating: no
  * counterpart in the reference; for callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, harnesses that forbid

@@ -767,6 +767,10 @@ int launch_wgrad_bf16(const Wgrad16Args& a, int kb, int nb, hipStream_t s) {
   return -1;
 }
 
+}  // namespace
+#include "mlp_bwd_fused64.h"
+namespace {
+
 // grad[k_off + row(k) * fan_out + n] (+)= sum_s part[s][k][n] for n < n_real;
 // row(k) = row_base + k for hidden inputs, or the encoding slot map (-1 = pad).
 struct ReduceArgs {
@@ -1252,12 +1256,39 @@ static int64_t wgrad_workspace_bytes_for(const nerf_mlp_desc* desc, int64_t M) {
   if (nerf_plan_from_desc(desc, NERF_PREC_BF16, &P16) == 0) {
     const int64_t st = wg16_stacked_floats(P16, M, true);
     if (st > f) f = st;
+    if (fb64::takes(P16) && fb64::groups(M) * fb64::kGroupFloats > f) f = fb64::groups(M) * fb64::kGroupFloats;
   }
   return f * 4 + 256;
 }
 
 extern "C" int64_t nerf_mlp_wgrad_workspace_bytes(const nerf_mlp_desc* desc, int64_t M) {
   return wgrad_workspace_bytes_for(desc, M);
+}
+
+// The reduction of job J's partial tiles jp and bias sums jb over nsplit splits.
+static ReduceArgs reduce_args_for(const MlpPlan& P, const WgradJob& J, const float* jp, const float* jb, int nsplit,
+                                  int32_t accumulate, float* grad_flat) {
+  ReduceArgs r;
+  r.part = jp;
+  r.bpart = jb;
+  r.K = J.K;
+  r.N = J.N;
+  r.n_real = J.n_real;
+  r.splits = nsplit;
+  r.enc_L = J.enc_L;
+  r.enc_KS = J.enc_KS;
+  r.row_base = J.row_base;
+  r.k_off = P.k_off[J.keras];
+  r.b_off = P.b_off[J.keras];
+  r.fan_out = P.fan_out[J.keras];
+  r.accumulate = accumulate;
+  r.grad = grad_flat;
+  return r;
+}
+static int reduce_blocks(const WgradJob& J) {
+  const int64_t tot = (int64_t)J.K * J.N + J.N;
+  const int64_t rb = (tot + 255) / 256;
+  return (int)(rb > 1024 ? 1024 : rb);
 }
 
 // The launches of one weight-gradient call (M > 0) into the partial-tile buffer
@@ -1268,27 +1299,7 @@ static int32_t wgrad_run(const MlpPlan& P, int32_t precision, int64_t M, const v
   WgradJob jobs[2 * NERF_MAX_LAYERS];
   const int nj = wgrad_jobs(P, jobs);
   auto reduce_args = [&](const WgradJob& J, const float* jp, const float* jb, int nsplit) {
-    ReduceArgs r;
-    r.part = jp;
-    r.bpart = jb;
-    r.K = J.K;
-    r.N = J.N;
-    r.n_real = J.n_real;
-    r.splits = nsplit;
-    r.enc_L = J.enc_L;
-    r.enc_KS = J.enc_KS;
-    r.row_base = J.row_base;
-    r.k_off = P.k_off[J.keras];
-    r.b_off = P.b_off[J.keras];
-    r.fan_out = P.fan_out[J.keras];
-    r.accumulate = accumulate;
-    r.grad = grad_flat;
-    return r;
-  };
-  auto reduce_blocks = [](const WgradJob& J) {
-    const int64_t tot = (int64_t)J.K * J.N + J.N;
-    const int64_t rb = (tot + 255) / 256;
-    return (int)(rb > 1024 ? 1024 : rb);
+    return reduce_args_for(P, J, jp, jb, nsplit, accumulate, grad_flat);
   };
   if (precision == NERF_PREC_BF16) {
     Wg16Group groups[2 * NERF_MAX_LAYERS];
@@ -1476,4 +1487,58 @@ extern "C" int32_t nerf_mlp_weight_grads(const nerf_mlp_desc* desc, int32_t prec
                  (long long)wgrad_workspace_bytes_for(desc, M), (long long)M);
   return wgrad_run(P, precision, M, stash, dz, grad_flat, accumulate,
                    reinterpret_cast<float*>(workspace), workspace_bytes / 4, s);
+}
+
+extern "C" int32_t nerf_mlp_has_backward_grads(const nerf_mlp_desc* desc, int32_t precision) {
+  MlpPlan P;
+  return nerf_plan_from_desc(desc, precision, &P) == 0 && fb64::takes(P) ? 1 : 0;
+}
+
+extern "C" int32_t nerf_mlp_backward_grads(const nerf_mlp_desc* desc, int32_t precision, const void* packed,
+                                           int64_t M, const float* d_sigma, const float* sigma,
+                                           const void* stash, float* grad_flat, int32_t accumulate,
+                                           void* workspace, int64_t workspace_bytes, void* stream) {
+  MlpPlan P;
+  NERF_CHECK_ARG(nerf_plan_from_desc(desc, precision, &P) == 0 && fb64::takes(P),
+                 "nerf_mlp_backward_grads: not for this MLP description or precision");
+  NERF_CHECK_ARG(M >= 0 && grad_flat, "nerf_mlp_backward_grads: bad arguments");
+  hipStream_t s = as_stream(stream);
+  if (M == 0) return wgrad_empty(P, grad_flat, accumulate, s);
+  NERF_CHECK_ARG(packed && d_sigma && sigma && stash && workspace, "nerf_mlp_backward_grads: null pointer");
+  const int64_t ng = fb64::groups(M), need = ng * fb64::kGroupFloats * 4;
+  NERF_CHECK_ARG(workspace_bytes >= need,
+                 "nerf_mlp_backward_grads: workspace of %lld bytes, this call needs %lld "
+                 "(nerf_mlp_wgrad_workspace_bytes gives %lld for M = %lld)",
+                 (long long)workspace_bytes, (long long)need, (long long)wgrad_workspace_bytes_for(desc, M),
+                 (long long)M);
+  WgradJob jobs[2 * NERF_MAX_LAYERS];
+  const int nj = wgrad_jobs(P, jobs);
+  NERF_CHECK_ARG(nj == fb64::kD + 1, "nerf_mlp_backward_grads: unexpected layers");
+  fb64::Args a;
+  a.pk = reinterpret_cast<const char*>(packed);
+  for (int l = 0; l < fb64::kD; ++l) a.p_bwd[l] = P.p_bwd[l];
+  a.p_sigma = P.p_head_sigma;
+  a.M = M;
+  a.ld = P.stash_per_sample;
+  for (int k = 0; k < fb64::kD; ++k) a.chunk0[k] = (int)(P.st_h[fb64::kD - 1 - k] / 8);
+  a.chunk0[fb64::kD] = (int)(P.st_encx / 8);
+  a.stash = reinterpret_cast<const __bf16*>(stash);
+  a.d_sigma = d_sigma;
+  a.sigma = sigma;
+  ReduceBatch rb;
+  rb.njobs = nj;
+  rb.first[0] = 0;
+  float* part = reinterpret_cast<float*>(workspace);
+  for (int t = 0; t < nj; ++t) {  // dense_0 .. dense_3, sigma
+    const int64_t tile = (int64_t)jobs[t].K * jobs[t].N;
+    a.part[t] = part;
+    a.bpart[t] = part + ng * tile;
+    part += ng * (tile + jobs[t].N);
+    rb.job[t] = reduce_args_for(P, jobs[t], a.part[t], a.bpart[t], (int)ng, accumulate, grad_flat);
+    rb.first[t + 1] = rb.first[t] + reduce_blocks(jobs[t]);
+  }
+  fb64::mlp_bwd_fused64_kernel<<<(unsigned)ng, 512, 0, s>>>(a);
+  wgrad_reduce_batch_kernel<true><<<(unsigned)rb.first[nj], 256, 0, s>>>(rb);
+  NERF_LAUNCH_CHECK("nerf_mlp_backward_grads");
+  return NERF_OK;
 }

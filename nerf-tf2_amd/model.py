@@ -193,6 +193,8 @@ class NerfMLP:
         self.dz_per_sample = int(lib.nerf_mlp_dz_floats_per_sample(ctypes_ref(self._desc)))
         # samples per block of the stash / dz layout: batch splits of the weight gradients fall on its multiples
         self.sample_block = int(lib.nerf_mlp_sample_block(ctypes_ref(self._desc), self.prec))
+        # a backward kernel that goes from the stash to the weight gradients without dz
+        self._one_backward = bool(lib.nerf_mlp_has_backward_grads(ctypes_ref(self._desc), self.prec))
         self.recompute_chunk: Optional[int] = None  # rays per recomputation chunk (None: stash all)
         self.repack()
 
@@ -268,18 +270,22 @@ class NerfMLP:
 
     # -- backward ----------------------------------------------------------
     def _backward_into(self, M, g_rgb, g_sigma, rgb, sigma, stash, grad, accumulate, work=None):
-        dz = torch.empty((M, self.dz_per_sample), dtype=torch.float32 if self.precision == "fp32" else torch.bfloat16,
-                         device=self.device)
         c = lambda t: None if t is None else t.contiguous()
         if g_sigma is None:
             g_sigma = torch.zeros((M, 1), dtype=torch.float32, device=self.device)
         if self.config.l_dir and g_rgb is None:
             g_rgb = torch.zeros((M, 3), dtype=torch.float32, device=self.device)
-        call("nerf_mlp_backward", ctypes_ref(self._desc), self.prec, ptr(self.packed), M, ptr(c(g_rgb)),
-             ptr(c(g_sigma)), ptr(c(rgb)), ptr(c(sigma)), ptr(stash), ptr(dz), stream(self.device))
         if work is None:
             ws = int(_lib.load().nerf_mlp_wgrad_workspace_bytes(ctypes_ref(self._desc), M))
             work = torch.empty(max(ws, 1), dtype=torch.uint8, device=self.device)
+        if self._one_backward:
+            call("nerf_mlp_backward_grads", ctypes_ref(self._desc), self.prec, ptr(self.packed), M, ptr(c(g_sigma)),
+                 ptr(c(sigma)), ptr(stash), ptr(grad), int(accumulate), ptr(work), work.numel(), stream(self.device))
+            return
+        dz = torch.empty((M, self.dz_per_sample), dtype=torch.float32 if self.precision == "fp32" else torch.bfloat16,
+                         device=self.device)
+        call("nerf_mlp_backward", ctypes_ref(self._desc), self.prec, ptr(self.packed), M, ptr(c(g_rgb)),
+             ptr(c(g_sigma)), ptr(c(rgb)), ptr(c(sigma)), ptr(stash), ptr(dz), stream(self.device))
         call("nerf_mlp_weight_grads", ctypes_ref(self._desc), self.prec, M, ptr(stash), ptr(dz), ptr(grad),
              int(accumulate), ptr(work), work.numel(), stream(self.device))
 
