@@ -49,42 +49,61 @@ struct PackSegs {
   unsigned char kind[kMaxSegs], layer[kMaxSegs];
 };
 
-// Forward A operands of MFMA layer m: thread u writes the 16 bytes of lane u % 64 of
-// (k-step or k-step group, output block) u / 64.
-__device__ void pack_fwd(const MlpPlan& P, const float* __restrict__ flat, char* __restrict__ out, int m, int u) {
+// Forward A operands of MFMA layer m: a wave writes unit w = (k-step or k-step group,
+// output block), 16 bytes per lane.  The unit's number is wave-uniform and a hidden
+// k-step's rows are two runs of four, so that what each lane computes is little more
+// than eight addresses (the divisions by block and model sizes per thread were most of
+// this kernel: 10.7 -> 7.9 us for the two BF16 8x256 models).
+__device__ void pack_fwd(const MlpPlan& P, const float* __restrict__ flat, char* __restrict__ out, int m, int w) {
   const int kl = P.keras_of[m], NBo = P.nb_out[m];
-  const int lane = u & 63, j = lane & 31, g = lane >> 5, nb = (u >> 6) % NBo, t = (u >> 6) / NBo;
+  const int lane = threadIdx.x & 63, j = lane & 31, g = lane >> 5, nb = w % NBo, t = w / NBo;
+  const int col = 32 * nb + j, FO = P.fan_out[kl];
+  const float* k = flat + P.k_off[kl] + col;
+  const bool in = col < FO;
   if (P.prec == 0) {
     if (t >= (P.ks_hid[m] + P.ks_enc[m]) / 4) return;
     floatx4 v;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = kernel_at(P, flat, kl, fwd_row_f32(P, m, 4 * t + r, g), 32 * nb + j);
-    reinterpret_cast<floatx4*>(out + P.p_fwd[m])[u] = v;
+    for (int r = 0; r < 4; ++r) v[r] = kernel_at(P, flat, kl, fwd_row_f32(P, m, 4 * t + r, g), col);
+    reinterpret_cast<floatx4*>(out + P.p_fwd[m])[w * 64 + lane] = v;
   } else {
-    const int ke16 = P.ks_enc[m] == 0 ? 0 : (P.enc_L[m] == P.LX ? P.KX16 : P.KD16);
-    if (t >= P.ks_hid[m] / 8 + ke16) return;
+    const int th = P.ks_hid[m] / 8, ke16 = P.ks_enc[m] == 0 ? 0 : (P.enc_L[m] == P.LX ? P.KX16 : P.KD16);
+    if (t >= th + ke16) return;
+    float f[8];
+    if (t < th) {  // cfeat(t / 2, 8 (t % 2) + r, g)
+      const float* q = k + (int64_t)(16 * t + 4 * g) * FO;
+#pragma unroll
+      for (int r = 0; r < 8; ++r) f[r] = in ? q[(r < 4 ? r : r + 4) * FO] : 0.f;
+    } else {
+#pragma unroll
+      for (int r = 0; r < 8; ++r) f[r] = kernel_at(P, flat, kl, fwd_row_bf16(P, m, t, r, g), col);
+    }
     ushortx8 v;
 #pragma unroll
-    for (int r = 0; r < 8; ++r) v[r] = f2bf(kernel_at(P, flat, kl, fwd_row_bf16(P, m, t, r, g), 32 * nb + j));
-    reinterpret_cast<ushortx8*>(out + P.p_fwd[m])[u] = v;
+    for (int r = 0; r < 8; ++r) v[r] = f2bf(f[r]);
+    reinterpret_cast<ushortx8*>(out + P.p_fwd[m])[w * 64 + lane] = v;
   }
 }
 
-// Backward (transposed) A operands: A[n = input hidden feature 32 nb + j][k = output feature].
-__device__ void pack_bwd(const MlpPlan& P, const float* __restrict__ flat, char* __restrict__ out, int m, int u) {
-  const int kl = P.keras_of[m], lane = u & 63, j = lane & 31, g = lane >> 5, nb = (u >> 6) % P.NB, t = (u >> 6) / P.NB;
+// Backward (transposed) A operands: A[n = input hidden feature 32 nb + j][k = output feature],
+// a unit per wave as above; a lane's outputs are one or two runs of four consecutive weights.
+__device__ void pack_bwd(const MlpPlan& P, const float* __restrict__ flat, char* __restrict__ out, int m, int w) {
+  const int kl = P.keras_of[m], lane = threadIdx.x & 63, j = lane & 31, g = lane >> 5, nb = w % P.NB, t = w / P.NB;
+  const int FO = P.fan_out[kl];
+  const float* k = flat + P.k_off[kl] + (int64_t)(32 * nb + j) * FO;
+  auto run = [&](int c) -> floatx4 {  // (FO is a multiple of 4: a run is inside or outside)
+    return c < FO ? (floatx4)*reinterpret_cast<const floatx4_a4*>(k + c) : floatx4{0.f, 0.f, 0.f, 0.f};
+  };
   if (P.prec == 0) {
     if (t >= 4 * P.nb_out[m]) return;
-    floatx4 v;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = kernel_at(P, flat, kl, 32 * nb + j, cfeat((4 * t + r) / 16, (4 * t + r) % 16, g));
-    reinterpret_cast<floatx4*>(out + P.p_bwd[m])[u] = v;
+    reinterpret_cast<floatx4*>(out + P.p_bwd[m])[w * 64 + lane] = run(cfeat(t / 4, 4 * (t % 4), g));
   } else {
     if (t >= 2 * P.nb_out[m]) return;
+    const floatx4 lo = run(16 * t + 4 * g), hi = run(16 * t + 4 * g + 8);  // cfeat(t / 2, 8 (t % 2) + r, g)
     ushortx8 v;
 #pragma unroll
-    for (int r = 0; r < 8; ++r) v[r] = f2bf(kernel_at(P, flat, kl, 32 * nb + j, cfeat(t / 2, 8 * (t % 2) + r, g)));
-    reinterpret_cast<ushortx8*>(out + P.p_bwd[m])[u] = v;
+    for (int r = 0; r < 8; ++r) v[r] = f2bf(r < 4 ? lo[r & 3] : hi[r & 3]);
+    reinterpret_cast<ushortx8*>(out + P.p_bwd[m])[w * 64 + lane] = v;
   }
 }
 
@@ -192,20 +211,23 @@ __device__ void pack_split_bwd(const MlpPlan& P, const float* __restrict__ flat,
 }
 
 // blockIdx.y: the model (all of one plan).  The first thread of the last launch of an optimizer
-// step also closes the step (state; null otherwise).
+// step also closes the step (state; null otherwise).  SPLIT: plans with split operands, whose
+// 40 KB of LDS would keep the others at four workgroups a CU, two rounds of them.
+template <bool SPLIT>
 __global__ __launch_bounds__(256) void pack_kernel(MlpPlan P, PackSegs S, PackModels A, StepState* state,
                                                    StepEnd end) {
   const float* __restrict__ flat = A.flat[blockIdx.y];
   char* __restrict__ out = A.packed[blockIdx.y];
   if (state && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) step_end(state, end);
-  __shared__ floatx4 s_w[kSplitRows * 8];
+  __shared__ floatx4 s_w[SPLIT ? kSplitRows * 8 : 1];
   __shared__ float s_m[4];
   int seg = 0;
   while (seg + 1 < S.n && (int)blockIdx.x >= S.first[seg + 1]) ++seg;
   const int blk = blockIdx.x - S.first[seg], m = S.layer[seg], u = 256 * blk + threadIdx.x;
+  const int unit = 4 * blk + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   switch (S.kind[seg]) {
-    case kFwd: return pack_fwd(P, flat, out, m, u);
-    case kBwd: return pack_bwd(P, flat, out, m, u);
+    case kFwd: return pack_fwd(P, flat, out, m, unit);
+    case kBwd: return pack_bwd(P, flat, out, m, unit);
     case kBias: {
       const int kl = P.keras_of[m];
       if (u < 32 * P.nb_out[m])
@@ -213,8 +235,12 @@ __global__ __launch_bounds__(256) void pack_kernel(MlpPlan P, PackSegs S, PackMo
       return;
     }
     case kHeads: return pack_heads(P, flat, out);
-    case kSplitFwd: return pack_split(P, flat, out, m, blk, reinterpret_cast<float*>(s_w), s_m);
-    case kSplitBwd: return pack_split_bwd(P, flat, out, m, blk, reinterpret_cast<float*>(s_w), s_m);
+    case kSplitFwd:
+      if constexpr (SPLIT) pack_split(P, flat, out, m, blk, reinterpret_cast<float*>(s_w), s_m);
+      return;
+    case kSplitBwd:
+      if constexpr (SPLIT) pack_split_bwd(P, flat, out, m, blk, reinterpret_cast<float*>(s_w), s_m);
+      return;
   }
 }
 
@@ -255,7 +281,8 @@ void pack_models(const MlpPlan& P, int n, const float* const* flat, void* const*
     A.flat[i] = flat[i];
     A.packed[i] = reinterpret_cast<char*>(packed[i]);
   }
-  pack_kernel<<<dim3((unsigned)S.first[S.n], (unsigned)n), 256, 0, s>>>(P, S, A, state, end);
+  const auto k = P.fs_bytes + P.bs_bytes > 0 ? pack_kernel<true> : pack_kernel<false>;
+  k<<<dim3((unsigned)S.first[S.n], (unsigned)n), 256, 0, s>>>(P, S, A, state, end);
 }
 
 int nerf_plan_from_desc(const nerf_mlp_desc* d, int prec, MlpPlan* p) {

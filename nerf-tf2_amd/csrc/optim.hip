@@ -255,7 +255,7 @@ extern "C" int32_t nerf_check_finite(int64_t n, const float* x, int32_t* flag, v
 
 // What bounds it: launches.  The two 8x256 models' step moves 38 MB (7 us at the rate of a
 // copy); as separate launches (open, a check per model, Adam and packing per model, close) it
-// took 48.5 us (BF16), most of it the eight calls and launches, and takes 21.1 here: one check of every gradient, one
+// took 48.5 us (BF16), most of it the eight calls and launches, and takes 18 here: one check of every gradient, one
 // Adam over every model, one packing launch per plan, the first opening and the last closing
 // the step; without a check the Adam launch opens it.
 extern "C" int32_t nerf_optimizer_step(int32_t n_models, const nerf_opt_model* models, float lr0, int32_t decay_steps,
