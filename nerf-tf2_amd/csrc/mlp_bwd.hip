@@ -783,6 +783,7 @@ struct ReduceArgs {
   int64_t k_off, b_off;
   int fan_out;
   int accumulate;
+  int wide;        // eight threads per element (reduce_job)
   float* grad;
 };
 
@@ -844,31 +845,60 @@ __device__ __forceinline__ float sum_splits_tree(const float* __restrict__ p, in
   return s;
 }
 
+// Where element e of a job's K x N tile (or of the bias row behind it) goes; null: nowhere.
+__device__ __forceinline__ float* reduce_dst(const ReduceArgs& a, int64_t n_el, int64_t e) {
+  if (e < n_el) {
+    const int k = (int)(e / a.N), n = (int)(e % a.N);
+    if (n >= a.n_real) return nullptr;
+    int row = k;
+    if (a.enc_L) {
+      const int g = k / a.enc_KS, s = k % a.enc_KS;
+      row = enc_feat(g, s, a.enc_L);
+      if (row < 0) return nullptr;
+    }
+    return a.grad + a.k_off + (int64_t)(a.row_base + row) * a.fan_out + n;
+  }
+  const int n = (int)(e - n_el);
+  return a.bpart && n < a.n_real ? a.grad + a.b_off + n : nullptr;
+}
+
 // Blocks blk (of nblk) of the reduction of one job: element e of the K x N tile
-// (and of the bias row) summed over the splits into the flat gradient.
+// (and of the bias row) summed over the splits into the flat gradient, by one
+// thread, or in a wide job (few elements, many splits: a thread's serial loads
+// would be the whole launch's time) by eight, each an eighth of the splits.
+constexpr int kWideLanes = 8, kWideEls = 256 / kWideLanes;
 template <bool TREE>
 __device__ __forceinline__ void reduce_job(const ReduceArgs& a, int64_t blk, int64_t nblk) {
   const int64_t n_el = (int64_t)a.K * a.N;
-  for (int64_t e = blk * blockDim.x + threadIdx.x; e < n_el + a.N; e += nblk * blockDim.x) {
-    if (e < n_el) {
-      const int k = (int)(e / a.N), n = (int)(e % a.N);
-      if (n >= a.n_real) continue;
-      int row = k;
-      if (a.enc_L) {
-        const int g = k / a.enc_KS, s = k % a.enc_KS;
-        row = enc_feat(g, s, a.enc_L);
-        if (row < 0) continue;
-      }
-      const float s = TREE ? sum_splits_tree(a.part + e, n_el, a.splits) : sum_splits(a.part + e, n_el, a.splits);
-      float* dst = a.grad + a.k_off + (int64_t)(a.row_base + row) * a.fan_out + n;
-      *dst = a.accumulate ? *dst + s : s;
-    } else if (a.bpart) {
-      const int n = (int)(e - n_el);
-      if (n >= a.n_real) continue;
-      const float s = TREE ? sum_splits_tree(a.bpart + n, a.N, a.splits) : sum_splits(a.bpart + n, a.N, a.splits);
-      float* dst = a.grad + a.b_off + n;
+  auto sum = [&](int64_t e, int first, int n) {
+    const float* p = e < n_el ? a.part + e : a.bpart + (e - n_el);
+    const int64_t stride = e < n_el ? n_el : a.N;
+    p += first * stride;
+    return TREE ? sum_splits_tree(p, stride, n) : sum_splits(p, stride, n);
+  };
+  if (a.wide) {
+    __shared__ float red[kWideLanes][kWideEls];
+    const int i = threadIdx.x % kWideEls, q = threadIdx.x / kWideEls;
+    const int64_t e = blk * kWideEls + i;
+    float* dst = e < n_el + a.N ? reduce_dst(a, n_el, e) : nullptr;
+    const int per = (a.splits + kWideLanes - 1) / kWideLanes, first = q * per;
+    const int n = a.splits - first < per ? a.splits - first : per;
+    red[q][i] = dst && n > 0 ? sum(e, first, n) : 0.f;
+    __syncthreads();
+    if (q == 0 && dst) {
+      float v[kWideLanes];
+#pragma unroll
+      for (int j = 0; j < kWideLanes; ++j) v[j] = red[j][i];
+      const float s = tree_sum(v);
       *dst = a.accumulate ? *dst + s : s;
     }
+    return;
+  }
+  for (int64_t e = blk * blockDim.x + threadIdx.x; e < n_el + a.N; e += nblk * blockDim.x) {
+    float* dst = reduce_dst(a, n_el, e);
+    if (!dst) continue;
+    const float s = sum(e, 0, a.splits);
+    *dst = a.accumulate ? *dst + s : s;
   }
 }
 
@@ -1026,10 +1056,10 @@ extern "C" int32_t nerf_mlp_backward(const nerf_mlp_desc* desc, int32_t precisio
   return NERF_OK;
 }
 
-// The fp32 launches: one for the heads (at most 4 columns, by VALU), one for all other jobs,
+// The fp32 launches: one for the heads (1 or 3 columns, by VALU), one for all other jobs,
 // with the smallest tile that holds each of them (mlp_wgrad_f32s.h).
 enum { kWgTile, kWgHead, kWg32Classes };
-static int wg32_class(const WgradJob& J) { return J.N <= 4 ? kWgHead : kWgTile; }
+static int wg32_class(const WgradJob& J) { return J.N == 1 || J.N == 3 ? kWgHead : kWgTile; }
 static int64_t wg32_job_floats(const WgradJob& J) { return (int64_t)J.K * J.N + (J.bias ? J.N : 0); }
 // Time per sample of a job (measured in the 8 x 8 tile, clocks per chunk: K = 256 7,500 and 7,200
 // with N = 256 and 128, K = 64 and 32 6,000): splitting takes all waves, whatever the layer has.
@@ -1051,7 +1081,7 @@ static int wg32_shape(const WgradJob* jobs, int nj) {
 // cost 7.1 ms where one takes 4.5: 786,432 samples of the 8x256 net); but at least 128 samples per split, and more rounds so that no split
 // sums over more than 8,192 samples (the rounding of one long sum), as far as the partial
 // tiles stay within the allocation-free entry point's static scratch; never so few that a
-// split's rows pass 2^31 bytes.  Heads: 512, of at least 64 samples.
+// split's rows pass 2^31 bytes.  Heads: 1,024, of at least 64 samples.
 static void wg32_splits(const MlpPlan& P, int64_t M, const WgradJob* jobs, int nj, int64_t* sp) {
   static const int per_cu[3] = {1, 1, 3};
   const int64_t least =
@@ -1073,7 +1103,7 @@ static void wg32_splits(const MlpPlan& P, int64_t M, const WgradJob* jobs, int n
   for (int t = 0; t < nj; ++t) {
     const bool head = wg32_class(jobs[t]) == kWgHead;
     const int64_t cap = (M + (head ? 63 : 127)) / (head ? 64 : 128);
-    int64_t s = head ? 512 : groups * wg32_job_cost(jobs[t]) / blocks;
+    int64_t s = head ? 1024 : groups * wg32_job_cost(jobs[t]) / blocks;
     if (s > cap) s = cap;
     if (s < least) s = least;
     sp[t] = s < 1 ? 1 : s;
@@ -1185,10 +1215,10 @@ static int wg16_groups(const MlpPlan& P, int64_t M, const WgradJob* jobs, int nj
   // Where the generic kernel fits several workgroups per CU, a group gets that
   // many times the splits, as far as its partial tiles stay within the largest
   // group's or the allocation-free entry point's static scratch, whichever is
-  // larger (so that entry point takes every batch it took before), and its tiles
-  // are large enough (16,384 floats per split) for the split sums to run wide:
-  // the sums over the splits of a narrow tile (one thread per output) cost more
-  // than the extra workgroups gain.
+  // larger (so that entry point takes every batch it took before).  Narrow tiles
+  // too: one workgroup's loads do not fill a CU's share of the bandwidth (720,896
+  // samples, 32 x 128 52 -> 43 us, 128 x 3 51 -> 38 us), and the sums over more splits
+  // take eight threads an element there (reduce_wide).
   int64_t most = (int64_t)NERF_WGRAD_STATIC_SCRATCH_BYTES / 4;
   for (int i = 0; i < ng; ++i) {
     const int64_t f = wg16_group_floats(groups[i], jobs);
@@ -1200,7 +1230,6 @@ static int wg16_groups(const MlpPlan& P, int64_t M, const WgradJob* jobs, int nj
     if (g.kb == 8 && g.nb == 8) continue;
     int64_t per = 0;  // floats per split
     for (int k = 0; k < g.n; ++k) per += jobs[g.members[k]].K * (int64_t)jobs[g.members[k]].N + jobs[g.members[k]].N;
-    if (per < 16384) continue;
     const int pc = bound ? 3 : wg16_per_cu(g.kb, g.nb);
     int64_t sg = (256 * pc + g.n - 1) / g.n;
     if (sg > cap) sg = cap;
@@ -1265,6 +1294,11 @@ extern "C" int64_t nerf_mlp_wgrad_workspace_bytes(const nerf_mlp_desc* desc, int
   return wgrad_workspace_bytes_for(desc, M);
 }
 
+// Eight threads per element up to 8,192 elements (256 blocks) over 64 splits and more: the
+// sums of the FP32 8x256 net's step 32 -> 15 us, of the proposal net's 8.8 -> 4.9 us.
+static bool reduce_wide(const WgradJob& J, int nsplit) {
+  return (int64_t)J.K * J.N + J.N <= 8192 && nsplit >= 64;
+}
 // The reduction of job J's partial tiles jp and bias sums jb over nsplit splits.
 static ReduceArgs reduce_args_for(const MlpPlan& P, const WgradJob& J, const float* jp, const float* jb, int nsplit,
                                   int32_t accumulate, float* grad_flat) {
@@ -1282,12 +1316,13 @@ static ReduceArgs reduce_args_for(const MlpPlan& P, const WgradJob& J, const flo
   r.b_off = P.b_off[J.keras];
   r.fan_out = P.fan_out[J.keras];
   r.accumulate = accumulate;
+  r.wide = reduce_wide(J, nsplit);
   r.grad = grad_flat;
   return r;
 }
-static int reduce_blocks(const WgradJob& J) {
+static int reduce_blocks(const WgradJob& J, int nsplit) {
   const int64_t tot = (int64_t)J.K * J.N + J.N;
-  const int64_t rb = (tot + 255) / 256;
+  const int64_t rb = reduce_wide(J, nsplit) ? (tot + kWideEls - 1) / kWideEls : (tot + 255) / 256;
   return (int)(rb > 1024 ? 1024 : rb);
 }
 
@@ -1351,7 +1386,7 @@ static int32_t wgrad_run(const MlpPlan& P, int32_t precision, int64_t M, const v
       for (int i = 0; i < n; ++i) {
         const int k = rbt.njobs++;
         rbt.job[k] = reduce_args(jobs[G.members[i]], b.job[i].part, b.job[i].bpart, (int)sg);
-        rbt.first[k + 1] = rbt.first[k] + reduce_blocks(jobs[G.members[i]]);
+        rbt.first[k + 1] = rbt.first[k] + reduce_blocks(jobs[G.members[i]], (int)sg);
       }
       if (!stack) wgrad_reduce_batch_kernel<false><<<(unsigned)rbt.first[rbt.njobs], 256, 0, s>>>(rbt);
     }
@@ -1394,7 +1429,7 @@ static int32_t wgrad_run(const MlpPlan& P, int32_t precision, int64_t M, const v
           const int64_t sj = sp[members[i]];
           const int k = rb.njobs++;
           rb.job[k] = reduce_args(J, base, J.bias ? base + sj * J.K * J.N : nullptr, (int)sj);
-          rb.first[k + 1] = rb.first[k] + reduce_blocks(J);
+          rb.first[k + 1] = rb.first[k] + reduce_blocks(J, (int)sj);
           base += sj * wg32_job_floats(J);
         }
         if (!stack) flush();
@@ -1535,7 +1570,7 @@ extern "C" int32_t nerf_mlp_backward_grads(const nerf_mlp_desc* desc, int32_t pr
     a.bpart[t] = part + ng * tile;
     part += ng * (tile + jobs[t].N);
     rb.job[t] = reduce_args_for(P, jobs[t], a.part[t], a.bpart[t], (int)ng, accumulate, grad_flat);
-    rb.first[t + 1] = rb.first[t] + reduce_blocks(jobs[t]);
+    rb.first[t + 1] = rb.first[t] + reduce_blocks(jobs[t], (int)ng);
   }
   fb64::mlp_bwd_fused64_kernel<<<(unsigned)ng, 512, 0, s>>>(a);
   wgrad_reduce_batch_kernel<true><<<(unsigned)rb.first[nj], 256, 0, s>>>(rb);

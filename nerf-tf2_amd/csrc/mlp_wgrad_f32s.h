@@ -311,65 +311,78 @@ __global__ __launch_bounds__(64 * (KB / RK) * (NB / RN)) void wgrad_f32s_kernel(
   }
 }
 
-// Heads (at most 4 output columns): dW[k][c] = sum_m X[m][k] dz[m][c].  Thread k of a
-// workgroup owns feature k (two or more row groups where K < 256): FP32 FMAs, bounded
-// by reading X once.  The bias, a single sum that may cancel, is summed with compensation
-// by one wave of each row group.
-__global__ __launch_bounds__(256) void wgrad_head_kernel(Args a) {
-  __shared__ float red[256][4];
-  const Tile T = a.tile[tile_of(a, blockIdx.x)];
-  const int split = blockIdx.x - T.first;
-  const int64_t mb = (int64_t)split * T.m_per_split;
-  const int64_t me = mb + T.m_per_split < a.M ? mb + T.m_per_split : a.M;
-  const int KP = T.K > 128 ? 256 : (T.K > 64 ? 128 : 64), R = 256 / KP;  // threads per row group, row groups
-  const int k = threadIdx.x % KP, rg = threadIdx.x / KP;                  // rg is wave-uniform
-  const float* x = a.X + T.xoff + (k < T.K ? k : 0);
-  const float* z = a.Z + T.zoff;
-  float s[4] = {0.f, 0.f, 0.f, 0.f}, b[4] = {0.f, 0.f, 0.f, 0.f}, bl[4] = {0.f, 0.f, 0.f, 0.f};
-  const bool sums = T.bpart && k < 64;  // wave-uniform
+// Rows m, m + R, .. of this split (up to me) into a head's sums s (FP32 FMAs in row order) and,
+// where `sums`, the bias sums b + bl; N columns, B rows in flight.  Everything but column xk of X
+// is wave-uniform: dz comes through scalar loads.
+template <int N, int B>
+__device__ __forceinline__ void head_rows(const float* __restrict__ x, int xk, const float* __restrict__ z, int64_t ldx,
+                                          int64_t ldz, int64_t m, int64_t me, int R, bool sums, float (&s)[3],
+                                          float (&b)[3], float (&bl)[3]) {
+  const int64_t sx = R * ldx, sz = R * ldz;
+  x += m * ldx;
+  z += m * ldz;
   auto add_bias = [&](int c, float zc) {
     float e;
     two_sum(b[c], zc, b[c], e);
     bl[c] += e;
   };
-  constexpr int B = 16;  // rows in flight
-  int64_t m = mb + rg;
   for (; m + (int64_t)(B - 1) * R < me; m += B * R) {
-    float xv[B], zv[B][4];
+    float xv[B], zv[B][N];
 #pragma unroll
-    for (int e = 0; e < B; ++e) xv[e] = x[(m + e * R) * a.ldx];
+    for (int e = 0; e < B; ++e, x += sx) xv[e] = x[xk];
+#pragma unroll
+    for (int e = 0; e < B; ++e, z += sz)
+#pragma unroll
+      for (int c = 0; c < N; ++c) zv[e][c] = z[c];
 #pragma unroll
     for (int e = 0; e < B; ++e)
 #pragma unroll
-      for (int c = 0; c < 4; ++c) zv[e][c] = c < T.N ? z[(m + e * R) * a.ldz + c] : 0.f;
-#pragma unroll
-    for (int e = 0; e < B; ++e)
-#pragma unroll
-      for (int c = 0; c < 4; ++c) s[c] = __builtin_fmaf(xv[e], zv[e][c], s[c]);
+      for (int c = 0; c < N; ++c) s[c] = __builtin_fmaf(xv[e], zv[e][c], s[c]);
     if (sums)
 #pragma unroll
       for (int e = 0; e < B; ++e)
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-          if (c < T.N) add_bias(c, zv[e][c]);
+        for (int c = 0; c < N; ++c) add_bias(c, zv[e][c]);
   }
-  for (; m < me; m += R)
+  for (; m < me; m += R, x += sx, z += sz)
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const float zc = c < T.N ? z[m * a.ldz + c] : 0.f;
-      s[c] = __builtin_fmaf(x[m * a.ldx], zc, s[c]);
-      if (sums) add_bias(c, zc);
+    for (int c = 0; c < N; ++c) {
+      s[c] = __builtin_fmaf(x[xk], z[c], s[c]);
+      if (sums) add_bias(c, z[c]);
     }
+}
+
+// Heads (1 or 3 output columns): dW[k][c] = sum_m X[m][k] dz[m][c].  Thread k of a
+// workgroup owns feature k (two or more row groups where K < 256): FP32 FMAs, bounded
+// by reading X once, so by how many rows are in flight: the single column has a loop of its
+// own, for the registers and so the waves (786,432 samples, both heads: 430 -> 255 us, 5.5 TB/s).
+// The bias, a single sum that may cancel, is summed with compensation
+// by one wave of each row group.
+__global__ __launch_bounds__(256) void wgrad_head_kernel(Args a) {
+  __shared__ float red[256][3];
+  const Tile T = a.tile[tile_of(a, blockIdx.x)];
+  const int split = blockIdx.x - T.first;
+  const int64_t mb = (int64_t)split * T.m_per_split;
+  const int64_t me = mb + T.m_per_split < a.M ? mb + T.m_per_split : a.M;
+  const int KP = T.K > 128 ? 256 : (T.K > 64 ? 128 : 64), R = 256 / KP;  // threads per row group, row groups
+  const int k = threadIdx.x % KP, rg = __builtin_amdgcn_readfirstlane(threadIdx.x / KP);  // rg is wave-uniform
+  const int xk = k < T.K ? k : 0;
+  const float* x = a.X + T.xoff;
+  const float* z = a.Z + T.zoff;
+  float s[3] = {0.f, 0.f, 0.f}, b[3] = {0.f, 0.f, 0.f}, bl[3] = {0.f, 0.f, 0.f};
+  const bool sums = T.bpart && k < 64;  // wave-uniform
+  if (T.N == 1) head_rows<1, 16>(x, xk, z, a.ldx, a.ldz, mb + rg, me, R, sums, s, b, bl);
+  else head_rows<3, 16>(x, xk, z, a.ldx, a.ldz, mb + rg, me, R, sums, s, b, bl);
 #pragma unroll
-  for (int c = 0; c < 4; ++c) b[c] += bl[c];
-  auto combine = [&](float (&q)[4]) {  // over the row groups, in order
+  for (int c = 0; c < 3; ++c) b[c] += bl[c];
+  auto combine = [&](float (&q)[3]) {  // over the row groups, in order
 #pragma unroll
-    for (int c = 0; c < 4; ++c) red[threadIdx.x][c] = q[c];
+    for (int c = 0; c < 3; ++c) red[threadIdx.x][c] = q[c];
     __syncthreads();
     if (rg == 0)
       for (int i = 1; i < R; ++i)
 #pragma unroll
-        for (int c = 0; c < 4; ++c) q[c] += red[k + i * KP][c];
+        for (int c = 0; c < 3; ++c) q[c] += red[k + i * KP][c];
     __syncthreads();
   };
   combine(s);
