@@ -145,9 +145,9 @@ __global__ __launch_bounds__(512) void mlp_bwd_bf16ws8_kernel(
   {
     lds_b8* const in_l = ws::lds_lane(s_act[0], 0, lane);
     lds_b8* const out_l = ws::lds_lane(s_act[1], 2 * nb0 * 64, lane);
-    ws8::run_steps<0, KR / 2, true, false>(acc, wlo, zero, in_l, in_l, [](int) {});
+    ws8::run_steps<kBlocks, 0, KR / 2, true, false>(acc, wlo, zero, in_l, in_l, [](int) {});
     ws8::load_w1<kT / 2, 0>(wlo, rs, P.p_bwd[D], C::NB, nb0, lane_off);
-    ws8::run_steps<KR / 2, KR / 2, false, true>(acc, whi, zero, in_l, in_l, [&](int sb) {
+    ws8::run_steps<kBlocks, KR / 2, KR / 2, false, true>(acc, whi, zero, in_l, in_l, [&](int sb) {
       epilogue(std::false_type{}, std::true_type{}, out_l, 0u, P.dz_bott, sb);
     });
     ws8::load_w1<kT / 2, kT / 2>(whi, rs, P.p_bwd[D], C::NB, nb0, lane_off);
@@ -195,12 +195,12 @@ __global__ __launch_bounds__(512) void mlp_bwd_bf16ws8_kernel(
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[sb][e] = hsv[e] * dzs;
       }
-      ws8::run_steps<0, H, false, false>(acc, wlo, zero, in_l, in_l, [](int) {});
+      ws8::run_steps<kBlocks, 0, H, false, false>(acc, wlo, zero, in_l, in_l, [](int) {});
     } else {
-      ws8::run_steps<0, H, true, false>(acc, wlo, zero, in_l, in_l, [](int) {});
+      ws8::run_steps<kBlocks, 0, H, true, false>(acc, wlo, zero, in_l, in_l, [](int) {});
     }
     if constexpr (layer > 1) ws8::load_w1<H, 0>(wlo, rs, P.p_bwd[layer - 1], C::NB, nb0, lane_off);
-    ws8::run_steps<H, H, false, true>(acc, whi, zero, in_l, in_l, [&](int sb) {
+    ws8::run_steps<kBlocks, H, H, false, true>(acc, whi, zero, in_l, in_l, [&](int sb) {
       epilogue(std::true_type{}, std::integral_constant<bool, (layer > 1)>{}, out_l, mbits[sb], P.dz_h[layer - 1],
                sb);
     });

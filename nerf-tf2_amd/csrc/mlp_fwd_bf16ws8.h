@@ -34,7 +34,6 @@
 
 namespace ws8 {
 
-using ws::kBlocks;
 using ws::kHalf;
 using ws::kRing;
 using ws::kSlab;
@@ -52,20 +51,20 @@ __device__ __forceinline__ void load_w1(bf16x8 (&w)[kHalf], __amdgpu_buffer_rsrc
   for (int t = 0; t < N; ++t) w[t] = ws::ldw(r, lane_off, p_layer + (int64_t)((OFF + t) * NBo + nb) * 1024);
 }
 
-// acc[sb] (+)= sum over k-steps T0 .. T0+H-1 of w[k - T0] * B(sb, k) for the four
-// sample blocks.  Without an epilogue step s runs block s % 4, k-step s / 4;
+// acc[sb] (+)= sum over k-steps T0 .. T0+H-1 of w[k - T0] * B(sb, k) for the N
+// sample blocks.  Without an epilogue step s runs block s % N, k-step s / N;
 // with one, blocks {0, 1} run interleaved over all H k-steps, then {2, 3}, and
 // epi(sb) follows each block's last MFMA.
-template <int T0, int H, bool INIT, bool EPI, typename Epi>
-__device__ __forceinline__ void run_steps(floatx16 (&acc)[kBlocks], const bf16x8 (&w)[kHalf], const floatx16& cb,
+template <int N, int T0, int H, bool INIT, bool EPI, typename Epi>
+__device__ __forceinline__ void run_steps(floatx16 (&acc)[N], const bf16x8 (&w)[kHalf], const floatx16& cb,
                                           const lds_b8* in, const lds_b8* ex, Epi&& epi) {
-  constexpr int S = kBlocks * H;
-  auto blk = [](int s) { return EPI ? 2 * (s / (2 * H)) + (s & 1) : s % kBlocks; };
-  auto kst = [](int s) { return EPI ? (s >> 1) % H : s / kBlocks; };
+  constexpr int S = N * H, P = EPI ? (N < 2 ? 1 : 2) : N;  // blocks run interleaved
+  auto blk = [](int s) { return P * (s / (P * H)) + s % P; };
+  auto kst = [](int s) { return s / P % H; };
   constexpr int R = kRing;
   bf16x8 b[R];
 #pragma unroll
-  for (int s = 0; s < R - 1; ++s) b[s] = ws::b_operand(in, ex, blk(s), T0 + kst(s));
+  for (int s = 0; s < R - 1 && s < S; ++s) b[s] = ws::b_operand(in, ex, blk(s), T0 + kst(s));
 #pragma unroll
   for (int s = 0; s < S; ++s) {
     if (s + R - 1 < S) b[(s + R - 1) % R] = ws::b_operand(in, ex, blk(s + R - 1), T0 + kst(s + R - 1));
@@ -77,7 +76,8 @@ __device__ __forceinline__ void run_steps(floatx16 (&acc)[kBlocks], const bf16x8
 
 }  // namespace ws8
 
-template <int W, int D, int SKIP, int LX, int LD, bool STASH>
+// N sample blocks of 32 per workgroup: 4, or fewer where that many would leave CUs idle.
+template <int W, int D, int SKIP, int LX, int LD, int N, bool STASH>
 __global__ __launch_bounds__(512) void mlp_fwd_bf16ws8_kernel(
     MlpPlan P, const char* __restrict__ pk, int64_t M, const float* __restrict__ xyz,
     const float* __restrict__ dirs, const float* __restrict__ ro, const float* __restrict__ rd,
@@ -88,18 +88,18 @@ __global__ __launch_bounds__(512) void mlp_fwd_bf16ws8_kernel(
   static_assert(W == 256 && LX == 10 && LD == 4 && SKIP >= 0 && SKIP + 1 < D,
                 "weight-stationary kernel is for the 8x256 NeRF MLP");
   static_assert(D == 8, "ReLU bit words: (2 nb + g) D is one chunk per lane half, four layers per store");
-  __shared__ bf16x8 s_act[2][kBlocks * kSlab];  // 2 x 64 KB
-  __shared__ bf16x8 s_ex[kBlocks * kTX * 64];   // 16 KB
-  __shared__ bf16x8 s_ed[kBlocks * kTD * 64];   // 8 KB
-  __shared__ float s_red[4][3][kBlocks * 32];   // rgb-head partials of waves 0-3, 6 KB
+  __shared__ bf16x8 s_act[2][N * kSlab];  // 2 x 64 KB
+  __shared__ bf16x8 s_ex[N * kTX * 64];   // 16 KB
+  __shared__ bf16x8 s_ed[N * kTD * 64];   // 8 KB
+  __shared__ float s_red[4][3][N * 32];   // rgb-head partials of waves 0-3, 6 KB
   const int lane = threadIdx.x & 63, j = lane & 31, g = lane >> 5;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform, 0 .. 7
-  const int64_t base = (int64_t)blockIdx.x * (kBlocks * 32);
+  const int64_t base = (int64_t)blockIdx.x * (N * 32);
   const int nb0 = wv;  // this wave's output block of a 256-wide layer
   const uint32_t lane_off = 16u * (uint32_t)lane, g_off = 16u * (uint32_t)g;
   const __amdgpu_buffer_rsrc_t rs = ws::packed_rsrc(pk, P.packed_bytes);
   // the stash rows of this workgroup as a buffer resource (rows past M fall outside)
-  const int64_t wg_rows = M - base < kBlocks * 32 ? M - base : kBlocks * 32;
+  const int64_t wg_rows = M - base < N * 32 ? M - base : N * 32;
   const __amdgpu_buffer_rsrc_t rst =
       STASH ? __builtin_amdgcn_make_buffer_rsrc(stash + base * P.stash_per_sample, 0,
                                                 (int)(wg_rows * P.stash_per_sample * 2), 0x00020000)
@@ -110,16 +110,16 @@ __global__ __launch_bounds__(512) void mlp_fwd_bf16ws8_kernel(
   // drops the store) plus a uniform part, both in the VGPR offset; the scalar
   // offset of these 8- and 16-byte stores stays 0.
   const int sps = (int)P.stash_per_sample;
-  int nrow[kBlocks];  // rows of each sample block (wave-uniform)
+  int nrow[N];  // rows of each sample block (wave-uniform)
 #pragma unroll
-  for (int sb = 0; sb < kBlocks; ++sb) {
+  for (int sb = 0; sb < N; ++sb) {
     const int64_t left = M - base - 32 * sb;
     nrow[sb] = __builtin_amdgcn_readfirstlane((int)(left < 32 ? (left > 0 ? left : 0) : 32));
   }
   auto rows_in = [&](int sb) { return nrow[sb]; };
-  uint32_t lbase[kBlocks];  // this lane's row start in each sample block; out of range past M
+  uint32_t lbase[N];  // this lane's row start in each sample block; out of range past M
 #pragma unroll
-  for (int sb = 0; sb < kBlocks; ++sb) lbase[sb] = j < nrow[sb] ? (uint32_t)(64 * sb * sps + 16 * j) : 0x80000000u;
+  for (int sb = 0; sb < N; ++sb) lbase[sb] = j < nrow[sb] ? (uint32_t)(64 * sb * sps + 16 * j) : 0x80000000u;
   auto voff = [&](int sb, int ch, int el) -> uint32_t {
     return lbase[sb] + (uint32_t)(16 * rows_in(sb) * ch + 2 * el);
   };
@@ -145,7 +145,7 @@ __global__ __launch_bounds__(512) void mlp_fwd_bf16ws8_kernel(
 
   bf16x8 wlo[kHalf], whi[kHalf];
   floatx16 cb;
-  floatx16 acc[kBlocks];
+  floatx16 acc[N];
 
   // layer 0 weights (4 encoding k-steps) into whi, layer 1's first half into wlo
   load_w1<kTX, 0>(whi, rs, P.p_fwd[0], C::NB, nb0, lane_off);
@@ -157,7 +157,7 @@ __global__ __launch_bounds__(512) void mlp_fwd_bf16ws8_kernel(
   // length counts: with six k-steps on four waves and a 64-bit division per lane a render launch
   // of 6,291,456 samples took 6.58 ms, now 6.51, one of 120,000 136 us, now 132.
   {
-    const int eb = wv & 3;
+    const int eb = wv % N;
     float x[3], d[3];
     load_sample_of(base, eb * 32 + j, M, xyz, dirs, ro, rd, tv, spr, x, d);
     // half g's slots start K / 8 chunks in (K a multiple of 8)
@@ -183,20 +183,30 @@ __global__ __launch_bounds__(512) void mlp_fwd_bf16ws8_kernel(
       encode_kstep<LD>(d, g, t, v);
       put(v, &s_ed[(eb * kTD + t) * 64], voff(eb, g * (C::KD / 8), 0), P.st_encd + 8 * t);
     };
-    if (wv < 4) {
-      ws::static_for<0, 3>(put_x);
-    } else {
-      put_x(std::integral_constant<int, 3>{});
-      ws::static_for<0, 2>(put_d);
+    if constexpr (N == 4) {
+      if (wv < 4) {
+        ws::static_for<0, 3>(put_x);
+      } else {
+        put_x(std::integral_constant<int, 3>{});
+        ws::static_for<0, 2>(put_d);
+      }
+    } else {  // k-steps wv / N and on, 8 / N apart, of block wv % N
+      ws::static_for<0, kTX + kTD>([&](auto uc) {
+        constexpr int u = decltype(uc)::value;
+        if (u % (8 / N) == wv / N) {
+          if constexpr (u < kTX) put_x(uc);
+          else put_d(std::integral_constant<int, u - kTX>{});
+        }
+      });
     }
   }
 
   // ReLU bit words of this wave's block for four trunk layers per sample block:
   // layer 4 q + t in half t % 2 of mw[sb][t / 2]
-  uint32_t mw[kBlocks][2];
+  uint32_t mw[N][2];
   auto store_masks = [&](int q) {
 #pragma unroll
-    for (int sb = 0; sb < kBlocks; ++sb) {
+    for (int sb = 0; sb < N; ++sb) {
       const ws::u32x2 v = {mw[sb][0], mw[sb][1]};
       // (2 nb0 + g) D = 16 nb0 + 8 g: lane half g one chunk on
       __builtin_amdgcn_raw_buffer_store_b64(
@@ -234,7 +244,7 @@ __global__ __launch_bounds__(512) void mlp_fwd_bf16ws8_kernel(
   lds_b8* const ex_l = ws::lds_lane(s_ex, 0, lane);
   {
     lds_b8* const out_l = ws::lds_lane(s_act[0], 2 * nb0 * 64, lane);
-    run_steps<kT, kTX, true, true>(acc, whi, cb, nullptr, ex_l,
+    run_steps<N, kT, kTX, true, true>(acc, whi, cb, nullptr, ex_l,
                                    [&](int sb) { epilogue(out_l, true, P.st_h[0], std::true_type{}, 0, sb); });
   }
   load_half(whi, 1, SKIP == 0, true);  // layer 1's second half and bias
@@ -250,7 +260,7 @@ __global__ __launch_bounds__(512) void mlp_fwd_bf16ws8_kernel(
     lds_b8* const out_l = ws::lds_lane(s_act[cur ^ 1], 2 * nb0 * 64, lane);
     if constexpr (l == D) {
       // sigma head on h_{D-1} (the input of this layer): wave w < 4 handles sample block w
-      if (wv < kBlocks) {
+      if (wv < N) {
         const uint32_t hs_off = 4u * (uint32_t)(g * C::KH);
         float zs = 0.f;
 #pragma unroll
@@ -272,7 +282,7 @@ __global__ __launch_bounds__(512) void mlp_fwd_bf16ws8_kernel(
     }
     constexpr bool enc = l == SKIP + 1;
     constexpr int H = enc ? (kT + kTX) / 2 : kT / 2;
-    run_steps<0, H, true, false>(acc, wlo, cb, in_l, ex_l, [](int) {});
+    run_steps<N, 0, H, true, false>(acc, wlo, cb, in_l, ex_l, [](int) {});
     // wlo is free: the next layer's first half and bias (after the bottleneck: the
     // rgb branch's first 10 k-steps of output block w, waves 0-3)
     if constexpr (l < D) {
@@ -282,7 +292,7 @@ __global__ __launch_bounds__(512) void mlp_fwd_bf16ws8_kernel(
       if (wv < 4) load_w1<kHalf, 0>(wlo, rs, P.p_fwd[D + 1], C::NBR, wv, lane_off);
     }
     const int64_t st_off = l < D ? P.st_h[l] : P.st_bott;
-    run_steps<H, H, false, true>(acc, whi, cb, in_l, ex_l, [&](int sb) {
+    run_steps<N, H, H, false, true>(acc, whi, cb, in_l, ex_l, [&](int sb) {
       epilogue(out_l, l < D, st_off, std::integral_constant<bool, (l < D)>{}, l, sb);
     });
     if constexpr (STASH && l < D && (l & 3) == 3) store_masks(l >> 2);
@@ -305,7 +315,7 @@ __global__ __launch_bounds__(512) void mlp_fwd_bf16ws8_kernel(
     lds_b8* const ed_l = ws::lds_lane(s_ed, 0, lane);
     auto wk = [&](int t) { return t < kHalf ? wlo[t] : whi[t - kHalf]; };
 #pragma unroll
-    for (int sb = 0; sb < kBlocks; ++sb) {
+    for (int sb = 0; sb < N; ++sb) {
       floatx16 a = cb;
 #pragma unroll
       for (int t = 0; t < kT; ++t) a = mfma_bf16(wk(t), in_l[sb * kSlab + t * 64], a);
@@ -344,7 +354,7 @@ __global__ __launch_bounds__(512) void mlp_fwd_bf16ws8_kernel(
   }
   __syncthreads();
   // wave w < 4 finishes the colours of sample block w
-  if (wv < kBlocks) {
+  if (wv < N) {
     const float* bias3 = reinterpret_cast<const float*>(hr4 + 2 * 16 * C::NBR);
     const int64_t m = base + wv * 32 + j;
     if (g == 0 && m < M) {
@@ -362,12 +372,19 @@ template <int W, int D, int SKIP, int LX, int LD>
 void launch_fwd_bf16ws8(const MlpPlan& P, const void* packed, int64_t M, const float* xyz, const float* dirs,
                         const float* ro, const float* rd, const float* tv, int spr, float* rgb, float* sigma,
                         void* stash, hipStream_t s) {
-  const int64_t nwg = (M + 127) / 128;
-  if (stash)
-    mlp_fwd_bf16ws8_kernel<W, D, SKIP, LX, LD, true><<<(unsigned)nwg, 512, 0, s>>>(
-        P, reinterpret_cast<const char*>(packed), M, xyz, dirs, ro, rd, tv, spr, rgb, sigma,
-        reinterpret_cast<__bf16*>(stash));
-  else
-    mlp_fwd_bf16ws8_kernel<W, D, SKIP, LX, LD, false><<<(unsigned)nwg, 512, 0, s>>>(
-        P, reinterpret_cast<const char*>(packed), M, xyz, dirs, ro, rd, tv, spr, rgb, sigma, nullptr);
+  auto go = [&](auto Nc, auto St) {
+    constexpr int N = decltype(Nc)::value;
+    mlp_fwd_bf16ws8_kernel<W, D, SKIP, LX, LD, N, decltype(St)::value>
+        <<<(unsigned)((M + 32 * N - 1) / (32 * N)), 512, 0, s>>>(P, reinterpret_cast<const char*>(packed), M, xyz,
+                                                                 dirs, ro, rd, tv, spr, rgb, sigma,
+                                                                 reinterpret_cast<__bf16*>(stash));
+  };
+  // Fewer blocks a workgroup while that still gives every workgroup a CU of its own: a layer
+  // then takes the time of its weights' stream from L2 rather than of four blocks' MFMAs:
+  // M = 1,000 30.1 -> 17.9 us, 8,192 31.4 -> 20.0 (N = 1), 16,384 32.1 -> 24.7 (N = 2).
+  const int64_t cus = nerf_num_cus();
+  if (stash) go(std::integral_constant<int, 4>{}, std::true_type{});
+  else if (M <= 32 * cus) go(std::integral_constant<int, 1>{}, std::false_type{});
+  else if (M <= 64 * cus) go(std::integral_constant<int, 2>{}, std::false_type{});
+  else go(std::integral_constant<int, 4>{}, std::false_type{});
 }
