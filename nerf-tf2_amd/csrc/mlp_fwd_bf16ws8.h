@@ -152,14 +152,16 @@ __global__ __launch_bounds__(512) void mlp_fwd_bf16ws8_kernel(
   load_half(wlo, 1, SKIP == 0, false);
   cb = ws::bias_acc(rs, P.p_bias[0], nb0, g_off);
 
-  // ---- encodings of sample block w % 4: waves 0-3 the first three k-steps of xyz, waves 4-7
-  // the fourth and the direction's two.  Nothing runs beside this (one workgroup a CU), so its
-  // length counts: with six k-steps on four waves and a 64-bit division per lane a render launch
-  // of 6,291,456 samples took 6.58 ms, now 6.51, one of 120,000 136 us, now 132.
+  // ---- encodings of sample block w % N; with four blocks, waves 0-3 the first three k-steps of
+  // xyz, waves 4-7 the fourth and the direction's two.  Nothing runs beside this (one workgroup a
+  // CU), so its length counts: against six k-steps on four waves a render launch of 6,291,456
+  // samples takes 6.52 instead of 6.62 ms, one of 120,000 135 instead of 141 us.  (A 32-bit division
+  // for the ray behind a uniform one, instead of load_sample's, measured 0.5 % slower.)
   {
     const int eb = wv % N;
     float x[3], d[3];
-    load_sample_of(base, eb * 32 + j, M, xyz, dirs, ro, rd, tv, spr, x, d);
+    const int64_t em = base + eb * 32 + j;
+    load_sample(em < M ? em : M - 1, xyz, dirs, ro, rd, tv, spr, x, d);
     // half g's slots start K / 8 chunks in (K a multiple of 8)
     static_assert(C::KX == 32 && C::KD == 16, "four and two k-steps of encoding");
     auto put = [&](const float (&v)[8], bf16x8* to, uint32_t vo, int64_t st) {

@@ -82,23 +82,6 @@ __device__ __forceinline__ void load_sample(int64_t m, const float* __restrict__
   d[2] = d2;
 }
 
-// load_sample of sample base + i (base wave-uniform, below M; clamped to M - 1): the ray's index
-// by a 32-bit division behind one that is uniform, instead of a 64-bit division per lane.
-__device__ __forceinline__ void load_sample_of(int64_t base, int i, int64_t M, const float* __restrict__ xyz,
-                                               const float* __restrict__ dirs, const float* __restrict__ ro,
-                                               const float* __restrict__ rd, const float* __restrict__ tv, int spr,
-                                               float (&x)[3], float (&d)[3]) {
-  const int64_t left = M - 1 - base;
-  if (left < i) i = (int)left;
-  if (ro) {
-    const int64_t r0 = base / spr;
-    const uint32_t at = (uint32_t)(base - r0 * spr) + (uint32_t)i, dr = at / (uint32_t)spr;
-    load_sample(0, nullptr, nullptr, ro + 3 * (r0 + dr), rd + 3 * (r0 + dr), tv + base + i, 1, x, d);
-  } else {
-    load_sample(base + i, xyz, dirs, nullptr, nullptr, nullptr, 1, x, d);
-  }
-}
-
 // Positional encoding (model.py:309-330) directly in the lane-half slots of
 // mlp_plan.h.  Argument = fl32(x_c * (2^l * fl32(pi))), exact power-of-two
 // scaling of fl32(pi) as in the reference; sin/cos are full-range accurate.
