@@ -33,8 +33,9 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 METRIC = "rays/sec render & train (64+128 samples), learned vs plain at ≤0.1 dB PSNR"
-FP32_PEAK_TFLOPS = 157.3
 BF16_PEAK_TFLOPS = 2500.0
+# the FP32 form's products are three FP16 matrix products each (the FP32 matrix instruction: 157.3)
+FP32_PEAK_TFLOPS = 2500.0 / 3
 HBM_PEAK_GBS = 8000.0
 MLP_FLOP_PER_SAMPLE = 2 * 593408          # both dense stacks of one model, per sample
 RENDER_FLOP_PER_RAY = (64 + 192) * MLP_FLOP_PER_SAMPLE
@@ -42,9 +43,9 @@ RENDER_FLOP_PER_RAY = (64 + 192) * MLP_FLOP_PER_SAMPLE
 
 # HBM bytes per fine-model MLP launch (FETCH_SIZE + WRITE_SIZE, each scaled by the
 # same counter on a 1 GiB device copy), from the rocprofv3 --pmc runs whose commands
-# and figures are in profiles/mlp_fwd_f32r_render800.md and
+# and figures are in profiles/mlp_fwd_f32s_render800.md and
 # profiles/mlp_fwd_bf16ws8_render800.md.
-TRAFFIC_BYTES_PER_LAUNCH = {"fp32": 153.8e6, "bf16": 142.5e6}
+TRAFFIC_BYTES_PER_LAUNCH = {"fp32": 152.1e6, "bf16": 142.5e6}
 
 
 def parse():
@@ -184,7 +185,7 @@ def main():
         "render_tflops": round(head["render_rays_per_s"] * RENDER_FLOP_PER_RAY / 1e12, 2),
         "roofline": None if "mlp_tflops" not in head else {
             "bound": "mfma", "kernel": "mlp_fwd (fine model, 32,768 rays x 192 samples per launch)",
-            "achieved": head["mlp_tflops"], "peak": peak, "unit": "TFLOP/s",
+            "achieved": head["mlp_tflops"], "peak": round(peak, 1), "unit": "TFLOP/s",
             "frac": round(head["mlp_tflops"] / peak, 4), "traffic": TRAFFIC_BYTES_PER_LAUNCH[prec],
             "avg_launch_ms": head["mlp_avg_launch_ms"], "flop_per_launch": head["mlp_flop_per_launch"]},
         "cpu_baseline": cpu,
@@ -422,10 +423,10 @@ def measure_hbm_kernels(nerf, dev, n=32768, reps=20):
         "coarse_kernel (Nc=64)": (8 + 16 * Nc + 4, lambda: call(
             "nerf_create_input_batch_coarse", n, Nc, 1, 1, ptr(ro), ptr(rd), ptr(near), ptr(far), ptr(u_c),
             ptr(edges), ptr(widths), ptr(t_c), None, None, st)),
-        "fine128_kernel (Nc=64, Nf=128)": (4 * (3 * Nc + (Nc + 1) + Nf + S), lambda: call(
+        "fine_wave_kernel (Nc=64, Nf=128)": (4 * (3 * Nc + (Nc + 1) + Nf + S), lambda: call(
             "nerf_create_input_batch_fine", n, Nc, Nf, ptr(ro), ptr(rd), ptr(w_c), ptr(edges), ptr(widths),
             ptr(t_c), ptr(u_f), ptr(t), None, None, None, None, 0, None, st)),
-        "fine128_kernel compensated (Nc=64, Nf=128)": (4 * (3 * Nc + (Nc + 1) + Nf + S), lambda: call(
+        "fine_wave_kernel compensated (Nc=64, Nf=128)": (4 * (3 * Nc + (Nc + 1) + Nf + S), lambda: call(
             "nerf_create_input_batch_fine", n, Nc, Nf, ptr(ro), ptr(rd), ptr(w_c), ptr(edges), ptr(widths),
             ptr(t_c), ptr(u_f), ptr(t), None, None, None, None, 1, None, st)),
         "composite_fwd_kernel (S=192)": (24 * S + 20, lambda: call(
