@@ -21,6 +21,7 @@
 
 #include "mlp_fwd_bf16.h"
 #include "mlp_fwd_bf16ws.h"
+#include "mlp_fwd_bf16res.h"
 #include "mlp_fwd_f32s.h"
 #include "mlp_fwd_bf16ws8.h"
 
@@ -185,8 +186,14 @@ int nerf_dispatch_fwd(const MlpPlan& P, const void* packed, int64_t M, const flo
       return 0;                                                                               \
     }                                                                                         \
     if (P.sblk != 32) return -1;                                                              \
-    return launch_fwd_bf16<W_, D_, S_, LX_, LD_>(P, packed, M, xyz, dirs, ro, rd, tv, spr,    \
-                                                 rgb, sigma, stash, s);                       \
+    if constexpr (W_ == 64 && LD_ == 0 && S_ < 0) {                                           \
+      launch_fwd_bf16res<W_, D_, S_, LX_, LD_>(P, packed, M, xyz, dirs, ro, rd, tv, spr,      \
+                                               sigma, stash, s);                              \
+      return 0;                                                                               \
+    } else {                                                                                  \
+      return launch_fwd_bf16<W_, D_, S_, LX_, LD_>(P, packed, M, xyz, dirs, ro, rd, tv, spr,  \
+                                                   rgb, sigma, stash, s);                     \
+    }                                                                                         \
   }
   NERF_MLP_INSTANCES(NERF_FWD_INST)
 #undef NERF_FWD_INST
