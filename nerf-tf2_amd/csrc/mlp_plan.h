@@ -68,7 +68,7 @@ struct MlpPlan {
   // packed byte offsets
   int64_t p_fwd[NERF_MAX_LAYERS], p_bwd[NERF_MAX_LAYERS], p_bias[NERF_MAX_LAYERS];
   int64_t p_head_sigma, p_head_rgb, packed_bytes;
-  // fp32, W = 256 with an rgb branch only (-1 otherwise): A operands of the forward
+  // fp32, the reference topology only (-1 otherwise): A operands of the forward
   // on the FP16 matrix cores, each weight split into two fp16 planes.  Per layer
   // units [output block of 32][k-step of 16][plane][lane][8], the k-steps and their
   // order as in the bf16 form; the layers follow each other without gaps (fs_bytes
@@ -185,8 +185,11 @@ inline int mlp_make_plan(int D, int W, int skip, int LX, int LD, int prec, MlpPl
     ++m;
   }
   P.n_mfma = m;
-  // packed layout (p_fwd, p_bwd: not for the split form, whose kernels read p_fs and p_bs)
-  const bool split = prec == 0 && W == 256 && P.rgb && P.NBR == 4;
+  // packed layout (p_fwd, p_bwd: not for the split form, whose kernels read p_fs and p_bs).  The
+  // split form is that of the one topology with kernels for it: other descriptions of the same
+  // width have other numbers of inputs (l_xyz or l_dir from 12 on more than its packing holds)
+  // and are packed as any other net.
+  const bool split = prec == 0 && D == 8 && W == 256 && skip == 4 && LX == 10 && LD == 4;
   int64_t b = 0;
   auto align = [&](int64_t a) { b = (b + a - 1) / a * a; };
   for (int i = 0; i < P.n_mfma; ++i) {
