@@ -1,7 +1,7 @@
 // Fused positional-encoding + MLP forward (model.py:289-394) on MFMA.
 //
 // The reference topology (8 x 256 with the rgb branch) runs the kernel of
-// mlp_fwd_f32s.h in fp32 (split products on the FP16 matrix cores) and the
+// mlp_fwd_f32s.h in fp32 (split products on the BF16 matrix cores) and the
 // eight-wave weight-stationary kernel of mlp_fwd_bf16ws8.h in bf16.  The fp32
 // kernel below serves the other topologies (the proposal and finite-difference
 // nets).  One wave owns 32 samples and

@@ -1,55 +1,47 @@
 // FP32 forward of the reference topology (W = 256 with the rgb branch), with or
-// without the training stash, on the FP16 matrix cores (mlp_f32s.h).
+// without the training stash, on the BF16 matrix cores (mlp_split3.h).
 //
 // A workgroup of eight waves carries 32 N samples through every layer.  Wave w
 // owns output block w (32 features); a layer's input sits in LDS as split B
-// operands (32 KB per sample block), the weights, split when they are packed,
-// stream from L2 as 1 KB loads two k-steps ahead.  A layer ends with the bias and
-// the ReLU, the exchange of each sample's largest value (its scale for the next
-// layer) and, behind that barrier, the split values' stores over the old tile.
-// With N = 2 the kernel keeps to 80 KB and 128 registers, so two workgroups share
-// a CU, four waves a SIMD: one workgroup's epilogues, encodings and barriers
-// overlap the other's MFMAs.  The encoding of the skip layer and of the rgb
-// branch is computed a second time into the tile once the hidden input has been
-// read, instead of holding 24 KB of it throughout.
+// operands (48 KB per sample block), the encodings beside it, the weights, split
+// when they are packed, stream from L2 as 1 KB loads three k-steps ahead.  A layer
+// ends with the bias, the ReLU and, behind a barrier, the split values' stores
+// over the old tile.  One workgroup fills a CU with N = 2.
 //
-// What bounds it: power.  The matrix cores are busy 0.69 of the time at a clock
-// that falls to 1.57 GHz; with random operands three FP16 products a step, their
-// LDS reads and 2 KB of weights per six MFMAs from L2, and nothing else, ran at
-// 1,139 TFLOP/s of FP16 work, this kernel at 1,190.  Measured at 6,291,456 samples:
-// 51.0 -> 18.7 ms (147 -> 399 TFLOP/s of FP32 work) against the register-resident
-// v_mfma_f32_16x16x4f32 kernel it replaced, which kept the FP32 matrix cores 0.94
-// busy; one workgroup of 128 samples per CU (half the weight traffic, but its
-// epilogues exposed) took 19.1 ms.  Three exact bf16 planes and six products
-// took 31.6 ms.
+// What bounds it: power.  At 6,291,456 samples it takes 33.3 ms (224 TFLOP/s of FP32 work,
+// 1,345 of BF16 work, where a bare stream of the six products with random operands, LDS and
+// L2 reads runs at 1,250 to 1,450), against 51.0 ms of the register-resident
+// v_mfma_f32_16x16x4f32 kernel that it replaced.  (Two FP16 parts and three products took
+// 18.7 ms, without FP32's range: mlp_split3.h.)  Error against 64 bits there 2.0e-7 (two FP16
+// parts 3.2e-7).
 //
-// N = 1 halves a workgroup's serial time where the samples do not fill the chip:
-// M = 1,000 189 -> 34 us a call; N = 1 / 2: 28.7 / 45.0 us at M = 4,096, 34.5 / 45.0
-// at 8,192, 52.5 / 46.5 at 12,000, 62.5 / 54.6 at 16,384, so N = 1 up to 32 samples
-// per CU.
+// N = 1 halves a workgroup's serial time where the samples do not fill the chip, and doubles
+// the weights' traffic: M = 1,000 189 us (FP32 instruction) -> 37.8; N = 1 / 2: 38.3 / 70.9 us
+// at M = 4,096, 51.2 / 71.3 at 8,192, 87.4 / 74.9 at 12,000, 100.7 / 89.3 at 16,384, and with
+// the stash 59.7 / 82.0 at 8,192, 103.5 / 88.4 at 12,000, so N = 1 up to 32 samples per CU.
 #pragma once
-#include "mlp_f32s.h"
+#include "mlp_split3.h"
 
 // N sample blocks of 32 per workgroup.
 template <int W, int D, int SKIP, int LX, int LD, int N, bool STASH>
-__global__ __launch_bounds__(512, 4) void mlp_fwd_f32s_kernel(
+__global__ __launch_bounds__(512, 2) void mlp_fwd_f32s_kernel(
     MlpPlan P, const char* __restrict__ pk, int64_t M, const float* __restrict__ xyz,
     const float* __restrict__ dirs, const float* __restrict__ ro, const float* __restrict__ rd,
     const float* __restrict__ tv, int spr, float* __restrict__ rgb_out, float* __restrict__ sig_out,
     float* __restrict__ stash) {
-  using namespace f32s;
+  using namespace split3;
   using C = NetC<W, D, SKIP, LX, LD>;
   static_assert(W == 256 && C::KX == 32 && C::KD == 16 && D % 2 == 0 && SKIP >= 0 && SKIP + 1 < D,
                 "split kernel is for the 8x256 NeRF MLP");
   static_assert(N == 1 || N == 2, "the rgb branch's 4 N output blocks go to waves 0 .. 4 N - 1");
   constexpr int TX = C::KX / 8, TD = C::KD / 8;
-  // weight units and k-steps of B operands in registers: one workgroup's two waves a SIMD
-  // (N = 1) wait for L2 and LDS themselves, two workgroups' four for each other
-  constexpr int AR = N == 1 ? 4 : 3, BR = N == 1 ? 2 : 1;
+  // weight units and k-steps of B operands in registers
+  constexpr int AR = N == 1 ? 6 : 4, BR = 2;
   constexpr int NBIAS = (D + 1) * C::NB + C::NBR;
-  __shared__ half8 s_tile[N][kTH * 128];         // 32 KB per sample block: a layer's input
+  __shared__ bf16x8 s_tile[N][kTH * kStep];      // 48 KB per sample block: a layer's input
+  __shared__ bf16x8 s_ex[N][TX * kStep];         // 12 KB: the xyz encoding
+  __shared__ bf16x8 s_ed[N][TD * kStep];         // 6 KB: the direction encoding
   __shared__ floatx4 s_bias[NBIAS * 8];          // 9.5 KB: [block][lane half][16]
-  __shared__ float s_max[N][kWaves * 32];        // a layer's largest values per block and sample
   __shared__ float s_sig[N][kWaves * 32];        // sigma-head partials per block and sample
   __shared__ float s_pt[N][6][32];               // sample points and directions
   const int lane = threadIdx.x & 63, j = lane & 31, g = lane >> 5;
@@ -57,7 +49,6 @@ __global__ __launch_bounds__(512, 4) void mlp_fwd_f32s_kernel(
   const int64_t base = (int64_t)blockIdx.x * (32 * N);
   const __amdgpu_buffer_rsrc_t rs = ws::packed_rsrc(pk + P.p_fs[0], P.fs_bytes);
   const uint32_t lane_off = 16u * (uint32_t)lane;
-  const int* wexp = reinterpret_cast<const int*>(pk + P.p_fse);  // weight scales [layer][block]
   // this wave's units of layer l start here (rgb branch: output block wv % 4)
   auto unit0 = [&](int l) -> int64_t {
     const int T = l == 0 ? TX : (l == SKIP + 1 ? kTH + TX : (l <= D ? kTH : kTH + TD));
@@ -65,7 +56,8 @@ __global__ __launch_bounds__(512, 4) void mlp_fwd_f32s_kernel(
   };
   Planes a[AR];
 #pragma unroll
-  for (int t = 0; t < AR - 1; ++t) a[t] = load_unit(rs, lane_off, unit0(0) + t * kUnit);
+  for (int t = 0; t < AR - 1; ++t)
+    a[t] = load_unit(rs, lane_off, t < TX ? unit0(0) + t * kUnit : unit0(1) + (t - TX) * kUnit);
 
   // the stash rows of this workgroup as a buffer resource (rows past M fall outside it)
   const int64_t w_rows = M - base < 32 * N ? M - base : 32 * N;
@@ -88,27 +80,16 @@ __global__ __launch_bounds__(512, 4) void mlp_fwd_f32s_kernel(
       s_pt[threadIdx.x >> 5][3 + c][threadIdx.x & 31] = d[c];
     }
   }
-  // Scale of this lane's sample in block n for an encoding (c0: 0 xyz, 3 direction): no value
-  // exceeds the largest component, or 1, the bound of the sines.
-  auto enc_scale = [&](int n, int c0) {
-    return scale_exp(fmaxf(fmaxf(fabsf(s_pt[n][c0][j]), fabsf(s_pt[n][c0 + 1][j])), fmaxf(fabsf(s_pt[n][c0 + 2][j]), 1.f)));
-  };
-  // Encoding of L frequencies (K slots per lane half) as the first K / 8 k-steps of the tile:
-  // unit u (wave u % 8) is k-step u % (K / 8) of sample block u / (K / 8).
-  auto encode = [&](auto Lc, int c0, int64_t st_off, bool first) {
-    constexpr int L = decltype(Lc)::value, K = L == LX ? C::KX : C::KD, T = K / 8;
-    for (int u = wv; u < T * N; u += kWaves) {
-      const int n = u / T, t = u % T;
-      const float x[3] = {s_pt[n][c0][j], s_pt[n][c0 + 1][j], s_pt[n][c0 + 2][j]};
-      float v[8];
-      encode_kstep<L>(x, g, t, v);
-      const Planes p = split8(v, pow2(enc_scale(n, c0)));
-      s_tile[n][t * 128 + lane] = p.h;
-      s_tile[n][t * 128 + 64 + lane] = p.l;
-      if (STASH && first) {
-        st4(floatx4{v[0], v[1], v[2], v[3]}, n, st_off + g * K + 8 * t);
-        st4(floatx4{v[4], v[5], v[6], v[7]}, n, st_off + g * K + 8 * t + 4);
-      }
+  // k-step t of an encoding of L frequencies (K slots per lane half) of sample block n
+  auto encode = [&](auto Lc, int c0, int n, int t, bf16x8* to, int64_t st_off) {
+    constexpr int L = decltype(Lc)::value, K = L == LX ? C::KX : C::KD;
+    const float x[3] = {s_pt[n][c0][j], s_pt[n][c0 + 1][j], s_pt[n][c0 + 2][j]};
+    float v[8];
+    encode_kstep<L>(x, g, t, v);
+    put_step((lds_b8*)to + lane, split8(v));
+    if constexpr (STASH) {
+      st4(floatx4{v[0], v[1], v[2], v[3]}, n, st_off + g * K + 8 * t);
+      st4(floatx4{v[4], v[5], v[6], v[7]}, n, st_off + g * K + 8 * t + 4);
     }
   };
   // biases of every layer in accumulator order (element 4 a + r of half g: feature 8 a + 4 g + r)
@@ -120,17 +101,25 @@ __global__ __launch_bounds__(512, 4) void mlp_fwd_f32s_kernel(
       s_bias[e] = ws::ldf4(rp, 4u * (uint32_t)(32 * (blk - C::NB * l) + 8 * q + 4 * h) + (uint32_t)P.p_bias[l], 0);
     }
   }
-  lds_h8* tile[N];
+  lds_b8 *tile[N], *ex[N], *ed[N];
 #pragma unroll
-  for (int n = 0; n < N; ++n) tile[n] = lds_lane(s_tile[n], lane);
+  for (int n = 0; n < N; ++n) {
+    tile[n] = ws::lds_lane(s_tile[n], 0, lane);
+    ex[n] = ws::lds_lane(s_ex[n], 0, lane);
+    ed[n] = ws::lds_lane(s_ed[n], 0, lane);
+  }
   const lds_f4* bias = (const lds_f4*)&s_bias[8 * wv + 4 * g];
-  floatx16 hi[N], lo[N];
-  int se[N];  // scale of this lane's sample in the tile
+  Acc acc[N];
   uint32_t mw[N];
   lds_barrier();
-  encode(std::integral_constant<int, LX>{}, 0, P.st_encx, true);
-#pragma unroll
-  for (int n = 0; n < N; ++n) se[n] = enc_scale(n, 0);
+  // the encodings, a k-step of a sample block at a time (wave u % 8)
+  for (int u = wv; u < (TX + TD) * N; u += kWaves) {
+    if (u < TX * N)
+      encode(std::integral_constant<int, LX>{}, 0, u / TX, u % TX, &s_ex[u / TX][u % TX * kStep], P.st_encx);
+    else
+      encode(std::integral_constant<int, LD>{}, 3, (u - TX * N) / TD, u % TD, &s_ed[(u - TX * N) / TD][u % TD * kStep],
+             P.st_encd);
+  }
   lds_barrier();
 
   // ring position of layer l's first weight unit
@@ -141,55 +130,29 @@ __global__ __launch_bounds__(512, 4) void mlp_fwd_f32s_kernel(
   };
   ws::static_for<0, D + 1>([&](auto Lc) {
     constexpr int l = decltype(Lc)::value, R = ring0(l);
-    const int we = wexp[l * C::NB + wv];
-    zero(hi);
-    zero(lo);
-    if constexpr (l == 0) {
-      steps<N, TX, R, AR, BR>(a, hi, lo, tile, rs, lane_off, unit0(0), unit0(1));
-    } else if constexpr (l == SKIP + 1) {
-      steps<N, kTH, R, AR, BR>(a, hi, lo, tile, rs, lane_off, unit0(l), unit0(l) + kTH * kUnit);
-      lds_barrier();
-      encode(std::integral_constant<int, LX>{}, 0, 0, false);
-      // the sums so far go to the encoding's scale
 #pragma unroll
-      for (int n = 0; n < N; ++n) {
-        const int s1 = enc_scale(n, 0);
-        const float f = pow2(s1 - se[n]);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          hi[n][i] = hi[n][i] * f;
-          lo[n][i] = lo[n][i] * f;
-        }
-        se[n] = s1;
-      }
-      lds_barrier();
-      steps<N, TX, (R + kTH) % AR, AR, BR>(a, hi, lo, tile, rs, lane_off, unit0(l) + kTH * kUnit, unit0(l + 1));
-    } else {
-      steps<N, kTH, R, AR, BR>(a, hi, lo, tile, rs, lane_off, unit0(l), unit0(l + 1));
-    }
+    for (int n = 0; n < N; ++n) zero(acc[n]);
+    constexpr int TH = l == 0 ? 0 : kTH, T = TH + (l == 0 || l == SKIP + 1 ? TX : 0);
+    steps<N, T, TH, R, AR, BR>(a, acc, tile, ex, rs, lane_off, unit0(l), unit0(l + 1));
     const int64_t st_off = (l < D ? P.st_h[l] : P.st_bott) + 32 * wv;
 #pragma unroll
     for (int n = 0; n < N; ++n) {
-      const float f = inv_scale(se[n], we);
-      float mx = 0.f;
+      floatx16& v = acc[n].h;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const floatx4 b = bias[8 * C::NB * l + q];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int i = 4 * q + r;
-          float v = __builtin_fmaf(hi[n][i] + lo[n][i], f, b[r]);
-          if constexpr (l < D) v = v > 0.f ? v : 0.f;
-          hi[n][i] = v;
-          mx = fmaxf(mx, l < D ? v : fabsf(v));
+          v[i] = sum(acc[n], i) + b[r];
+          if constexpr (l < D) v[i] = v[i] > 0.f ? v[i] : 0.f;
         }
       }
-      put_max((lds_f*)s_max[n], wv, j, g, mx);
       if constexpr (STASH && l < D) {
         // ReLU words of this block and lane half, two layers per store
         uint32_t w = 0u;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) w |= (hi[n][i] > 0.f ? 1u : 0u) << i;
+        for (int i = 0; i < 16; ++i) w |= (v[i] > 0.f ? 1u : 0u) << i;
         if constexpr ((l & 1) == 0)
           mw[n] = w;
         else
@@ -204,28 +167,24 @@ __global__ __launch_bounds__(512, 4) void mlp_fwd_f32s_kernel(
         for (int q = 0; q < 4; ++q) {
           const floatx4 w = hs[q];
 #pragma unroll
-          for (int r = 0; r < 4; ++r) z = z + hi[n][4 * q + r] * w[r];
+          for (int r = 0; r < 4; ++r) z = z + v[4 * q + r] * w[r];
         }
         z = z + shfl_xor(z, 32);
         if (g == 0) s_sig[n][wv * 32 + j] = z;
       }
     }
-    lds_barrier();  // every wave has read the tile; the largest values are there
+    lds_barrier();  // every wave has read the tile
 #pragma unroll
     for (int n = 0; n < N; ++n) {
-      se[n] = scale_exp(get_max((const lds_f*)s_max[n], j));
-      const float sc = pow2(se[n]);
-      if constexpr (STASH)
-        store_rows(hi[n], tile[n] + 2 * wv * 128, lane, rst, n * blk_row + (uint32_t)(4 * st_off), row_bytes);
+      const floatx16& u = acc[n].h;
+      lds_b8* o = tile[n] + 2 * wv * kStep;
+      if constexpr (STASH) store_rows(u, o, lane, rst, n * blk_row + (uint32_t)(4 * st_off), row_bytes);
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         float v[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = hi[n][8 * h + i];
-        const Planes p = split8(v, sc);
-        lds_h8* o = tile[n] + (2 * wv + h) * 128;
-        o[0] = p.h;
-        o[64] = p.l;
+        for (int i = 0; i < 8; ++i) v[i] = u[8 * h + i];
+        put_step(o + h * kStep, split8(v));
       }
     }
     lds_barrier();
@@ -236,27 +195,17 @@ __global__ __launch_bounds__(512, 4) void mlp_fwd_f32s_kernel(
   constexpr int RR = ring0(D + 1);
   const bool own = wv < 4 * N;
   const int n = N == 1 ? 0 : wv >> 2, nb = wv & 3;
-  floatx16 h1[1], l1[1];
-  lds_h8* t1[1];
+  Acc c1[1];
+  lds_b8* t1[1];
+  lds_b8* e1[1];
   t1[0] = n ? tile[N - 1] : tile[0];
-  zero(h1);
-  zero(l1);
-  if (own) steps<1, kTH, RR, AR, BR>(a, h1, l1, t1, rs, lane_off, unit0(D + 1), unit0(D + 1) + kTH * kUnit);
-  lds_barrier();
-  encode(std::integral_constant<int, LD>{}, 3, P.st_encd, true);
-  lds_barrier();
+  e1[0] = n ? ed[N - 1] : ed[0];
+  zero(c1[0]);
   float p0 = 0.f, p1 = 0.f, p2 = 0.f;
   if (own) {
-    const int s1 = enc_scale(n, 3);
-    const float f1 = pow2(s1 - (n ? se[N - 1] : se[0]));
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      h1[0][i] = h1[0][i] * f1;
-      l1[0][i] = l1[0][i] * f1;
-    }
-    steps<1, TD, (RR + kTH) % AR, AR, BR>(a, h1, l1, t1, rs, lane_off, unit0(D + 1) + kTH * kUnit, unit0(D + 1));
-    const float f = inv_scale(s1, wexp[(D + 1) * C::NB + nb]);
+    steps<1, kTH + TD, kTH, RR, AR, BR>(a, c1, t1, e1, rs, lane_off, unit0(D + 1), unit0(D + 1));
     const floatx4* hr4 = reinterpret_cast<const floatx4*>(pk + P.p_head_rgb) + g * 16 * C::NBR + 16 * nb;
+    floatx16& v = c1[0].h;
     const lds_f4* br = (const lds_f4*)&s_bias[8 * (C::NB * (D + 1) + nb) + 4 * g];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -264,21 +213,21 @@ __global__ __launch_bounds__(512, 4) void mlp_fwd_f32s_kernel(
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int i = 4 * q + r;
-        const float v = __builtin_fmaf(h1[0][i] + l1[0][i], f, b[r]);
-        h1[0][i] = v > 0.f ? v : 0.f;
+        const float z = sum(c1[0], i) + b[r];
+        v[i] = z > 0.f ? z : 0.f;
         const floatx4 w = hr4[i];  // rgb head (model.py:386-387)
-        p0 = p0 + h1[0][i] * w[0];
-        p1 = p1 + h1[0][i] * w[1];
-        p2 = p2 + h1[0][i] * w[2];
+        p0 = p0 + v[i] * w[0];
+        p1 = p1 + v[i] * w[1];
+        p2 = p2 + v[i] * w[2];
       }
       if constexpr (STASH)
-        st4(floatx4{h1[0][4 * q], h1[0][4 * q + 1], h1[0][4 * q + 2], h1[0][4 * q + 3]}, n,
+        st4(floatx4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]}, n,
             P.st_rbr + 32 * nb + 8 * q + 4 * g);
     }
     if constexpr (STASH) {
       uint32_t w = 0u;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) w |= (h1[0][i] > 0.f ? 1u : 0u) << i;
+      for (int i = 0; i < 16; ++i) w |= (v[i] > 0.f ? 1u : 0u) << i;
       __builtin_amdgcn_raw_buffer_store_b16((unsigned short)w, rst,
                                             row + n * blk_row + (uint32_t)(4 * P.st_mask + 2 * (16 * D + 2 * nb + g)), 0, 0);
     }
@@ -322,7 +271,7 @@ void launch_fwd_f32s(const MlpPlan& P, const void* packed, int64_t M, const floa
   auto go = [&](auto Nc, auto St) {
     constexpr int N = decltype(Nc)::value;
     mlp_fwd_f32s_kernel<W, D, SKIP, LX, LD, N, decltype(St)::value>
-        <<<(unsigned)((M + 32 * N - 1) / (32 * N)), 64 * f32s::kWaves, 0, s>>>(
+        <<<(unsigned)((M + 32 * N - 1) / (32 * N)), 64 * split3::kWaves, 0, s>>>(
             P, reinterpret_cast<const char*>(packed), M, xyz, dirs, ro, rd, tv, spr, rgb, sigma,
             reinterpret_cast<float*>(stash));
   };

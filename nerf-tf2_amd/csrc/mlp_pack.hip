@@ -3,13 +3,14 @@
 #include "common.h"
 #include "mlp_plan.h"
 #include "mlp_f32s.h"
+#include "mlp_split3.h"
 #include "optim.h"
 
 namespace {
 
 typedef float floatx4_a4 __attribute__((ext_vector_type(4), aligned(4)));  // the caller's weights: any float alignment
 
-constexpr int kSplitRows = 320;  // rows of the widest split layer (the skip layer's 256 + 63 inputs), padded
+constexpr int kSplitFloats = 32 * 257;  // a block of the widest split layer (256 outputs)
 
 // Input row (of the Keras kernel) fed by fp32 k-step s on lane half g of MFMA layer m.
 __device__ int fwd_row_f32(const MlpPlan& P, int m, int s, int g) {
@@ -41,7 +42,7 @@ struct PackModels {
   const float* flat[kOptModels];
   char* packed[kOptModels];
 };
-enum PackKind : int { kFwd, kBwd, kBias, kHeads, kSplitFwd, kSplitBwd };
+enum PackKind : int { kFwd, kBwd, kBias, kHeads, kSplitBwd };
 constexpr int kMaxSegs = 3 * NERF_MAX_LAYERS + 1;
 struct PackSegs {
   int n;
@@ -50,25 +51,27 @@ struct PackSegs {
 };
 
 // Forward A operands of MFMA layer m: a wave writes unit w = (k-step or k-step group,
-// output block), 16 bytes per lane.  The unit's number is wave-uniform and a hidden
-// k-step's rows are two runs of four, so that what each lane computes is little more
-// than eight addresses (the divisions by block and model sizes per thread were most of
-// this kernel: 10.7 -> 7.9 us for the two BF16 8x256 models).
+// output block; the split form: output block, k-step), 16 bytes per lane and plane.  The
+// unit's number is wave-uniform and a hidden k-step's rows are two runs of four, so that what
+// each lane computes is little more than eight addresses (the divisions by block and model
+// sizes per thread were most of this kernel: 10.7 -> 7.9 us for the two BF16 8x256 models).
 __device__ void pack_fwd(const MlpPlan& P, const float* __restrict__ flat, char* __restrict__ out, int m, int w) {
-  const int kl = P.keras_of[m], NBo = P.nb_out[m];
-  const int lane = threadIdx.x & 63, j = lane & 31, g = lane >> 5, nb = w % NBo, t = w / NBo;
+  const int kl = P.keras_of[m], NBo = P.nb_out[m], T = (P.ks_hid[m] + P.ks_enc[m]) / 8;
+  const bool split = P.p_fs[m] >= 0;
+  const int lane = threadIdx.x & 63, j = lane & 31, g = lane >> 5;
+  const int nb = split ? w / T : w % NBo, t = split ? w % T : w / NBo;
   const int col = 32 * nb + j, FO = P.fan_out[kl];
   const float* k = flat + P.k_off[kl] + col;
   const bool in = col < FO;
-  if (P.prec == 0) {
-    if (t >= (P.ks_hid[m] + P.ks_enc[m]) / 4) return;
+  if (P.prec == 0 && !split) {
+    if (t >= 2 * T) return;
     floatx4 v;
 #pragma unroll
     for (int r = 0; r < 4; ++r) v[r] = kernel_at(P, flat, kl, fwd_row_f32(P, m, 4 * t + r, g), col);
     reinterpret_cast<floatx4*>(out + P.p_fwd[m])[w * 64 + lane] = v;
   } else {
-    const int th = P.ks_hid[m] / 8, ke16 = P.ks_enc[m] == 0 ? 0 : (P.enc_L[m] == P.LX ? P.KX16 : P.KD16);
-    if (t >= th + ke16) return;
+    const int th = P.ks_hid[m] / 8;
+    if (nb >= NBo || t >= T) return;
     float f[8];
     if (t < th) {  // cfeat(t / 2, 8 (t % 2) + r, g)
       const float* q = k + (int64_t)(16 * t + 4 * g) * FO;
@@ -77,6 +80,14 @@ __device__ void pack_fwd(const MlpPlan& P, const float* __restrict__ flat, char*
     } else {
 #pragma unroll
       for (int r = 0; r < 8; ++r) f[r] = kernel_at(P, flat, kl, fwd_row_bf16(P, m, t, r, g), col);
+    }
+    if (split) {
+      bf16x8* o = reinterpret_cast<bf16x8*>(out + P.p_fs[m]) + w * split3::kStep + lane;
+      const split3::Planes p = split3::split8(f);
+      o[0] = p.h;
+      o[64] = p.m;
+      o[128] = p.l;
+      return;
     }
     ushortx8 v;
 #pragma unroll
@@ -135,47 +146,11 @@ __device__ int split_scale(float mx, float* s_m) {
   return f32s::scale_exp(fmaxf(fmaxf(s_m[0], s_m[1]), fmaxf(s_m[2], s_m[3])), 60);
 }
 
-// Split forward operands of layer m, one workgroup per output block nb: its 32 columns go to
-// LDS (one read of the weights, all loads in flight together), the largest gives the block's
-// scale, and each thread writes 16-byte chunks: the 8 slots of lane (j, g) of k-step t in unit
-// nb T + t, planes 1 KB apart.
-__device__ void pack_split(const MlpPlan& P, const float* __restrict__ flat, char* __restrict__ out, int m, int nb,
-                           float* s_w, float* s_m) {
-  const int kl = P.keras_of[m], T = (P.ks_hid[m] + P.ks_enc[m]) / 8, rows = P.fan_in[kl];
-  const float* w = flat + P.k_off[kl] + 32 * nb + 4 * (threadIdx.x & 7);
-  floatx4 v4[kSplitRows / 32];
-#pragma unroll
-  for (int i = 0; i < kSplitRows / 32; ++i) {
-    const int row = 32 * i + (threadIdx.x >> 3);
-    v4[i] = row < rows ? (floatx4)*reinterpret_cast<const floatx4_a4*>(w + (int64_t)row * P.fan_out[kl]) : floatx4{0.f, 0.f, 0.f, 0.f};
-  }
-  float mx = 0.f;
-#pragma unroll
-  for (int i = 0; i < kSplitRows / 32; ++i) {
-    reinterpret_cast<floatx4*>(s_w)[i * 256 + threadIdx.x] = v4[i];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) mx = fmaxf(mx, fabsf(v4[i][r]));
-  }
-  const int s = split_scale(mx, s_m);
-  if (threadIdx.x == 0) reinterpret_cast<int*>(out + P.p_fse)[m * P.NB + nb] = s;
-  const float sc = f32s::pow2(s);
-  const int j = threadIdx.x & 31, g = (threadIdx.x >> 5) & 1;
-  f32s::half8* o = reinterpret_cast<f32s::half8*>(out + P.p_fs[m]) + (int64_t)nb * T * 128 + (threadIdx.x & 63);
-  for (int t = threadIdx.x >> 6; t < T; t += 4) {
-    float v[8];
-#pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      const int row = fwd_row_bf16(P, m, t, r, g);
-      v[r] = row < 0 ? 0.f : s_w[row * 32 + j];
-    }
-    const f32s::Planes p = f32s::split8(v, sc);
-    o[t * 128] = p.h;
-    o[t * 128 + 64] = p.l;
-  }
-}
-
-// The same for the dX chain: input block nb, 32 rows of fan_out (128 or 256) weights each, kept
-// in LDS one float apart so that 32 lanes read 32 rows without bank conflicts.
+// Split operands of the dX chain, one workgroup per input block nb: its 32 rows of fan_out (128 or
+// 256) weights go to LDS (one read of the weights, all loads in flight together) one float apart,
+// so that 32 lanes read 32 rows without bank conflicts; the largest gives the block's scale, and
+// each thread writes 16-byte chunks: the 8 slots of lane (j, g) of k-step t in unit nb T + t, planes
+// 1 KB apart.
 __device__ void pack_split_bwd(const MlpPlan& P, const float* __restrict__ flat, char* __restrict__ out, int m,
                                int nb, float* s_w, float* s_m) {
   const int kl = P.keras_of[m], T = 2 * P.nb_out[m], FO = P.fan_out[kl], V = FO / 128;  // float4s per thread and 4 rows
@@ -212,14 +187,14 @@ __device__ void pack_split_bwd(const MlpPlan& P, const float* __restrict__ flat,
 
 // blockIdx.y: the model (all of one plan).  The first thread of the last launch of an optimizer
 // step also closes the step (state; null otherwise).  SPLIT: plans with split operands, whose
-// 40 KB of LDS would keep the others at four workgroups a CU, two rounds of them.
+// 33 KB of LDS would keep the others at four workgroups a CU, two rounds of them.
 template <bool SPLIT>
 __global__ __launch_bounds__(256) void pack_kernel(MlpPlan P, PackSegs S, PackModels A, StepState* state,
                                                    StepEnd end) {
   const float* __restrict__ flat = A.flat[blockIdx.y];
   char* __restrict__ out = A.packed[blockIdx.y];
   if (state && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) step_end(state, end);
-  __shared__ floatx4 s_w[SPLIT ? kSplitRows * 8 : 1];
+  __shared__ float s_w[SPLIT ? kSplitFloats : 1];
   __shared__ float s_m[4];
   int seg = 0;
   while (seg + 1 < S.n && (int)blockIdx.x >= S.first[seg + 1]) ++seg;
@@ -235,11 +210,8 @@ __global__ __launch_bounds__(256) void pack_kernel(MlpPlan P, PackSegs S, PackMo
       return;
     }
     case kHeads: return pack_heads(P, flat, out);
-    case kSplitFwd:
-      if constexpr (SPLIT) pack_split(P, flat, out, m, blk, reinterpret_cast<float*>(s_w), s_m);
-      return;
     case kSplitBwd:
-      if constexpr (SPLIT) pack_split_bwd(P, flat, out, m, blk, reinterpret_cast<float*>(s_w), s_m);
+      if constexpr (SPLIT) pack_split_bwd(P, flat, out, m, blk, s_w, s_m);
       return;
   }
 }
@@ -255,14 +227,11 @@ PackSegs pack_segs(const MlpPlan& P) {
   };
   auto blocks16 = [](int64_t bytes) { return (bytes + 4095) / 4096; };  // 16 bytes per thread
   for (int m = 0; m < P.n_mfma; ++m) {
-    if (P.p_fs[m] >= 0) add(kSplitFwd, m, P.nb_out[m]);
     if (P.p_bs[m] >= 0) add(kSplitBwd, m, P.NB);
   }
   for (int m = 0; m < P.n_mfma; ++m) {
-    const int ks = P.ks_hid[m] + P.ks_enc[m];
-    const int ke16 = P.ks_enc[m] == 0 ? 0 : (P.enc_L[m] == P.LX ? P.KX16 : P.KD16);
-    if (P.p_fwd[m] >= 0)
-      add(kFwd, m, blocks16((int64_t)P.nb_out[m] * 64 * 16 * (P.prec == 0 ? ks / 4 : P.ks_hid[m] / 8 + ke16)));
+    const int T = (P.ks_hid[m] + P.ks_enc[m]) / 8;
+    add(kFwd, m, blocks16((int64_t)P.nb_out[m] * 64 * 16 * (P.p_fwd[m] >= 0 && P.prec == 0 ? 2 * T : T)));
     if (P.p_bwd[m] >= 0) add(kBwd, m, blocks16((int64_t)P.nb_out[m] * (P.prec == 0 ? 4 : 2) * P.NB * 64 * 16));
   }
   for (int m = 0; m < P.n_mfma; ++m) add(kBias, m, (32 * P.nb_out[m] + 255) / 256);

@@ -68,15 +68,15 @@ struct MlpPlan {
   // packed byte offsets
   int64_t p_fwd[NERF_MAX_LAYERS], p_bwd[NERF_MAX_LAYERS], p_bias[NERF_MAX_LAYERS];
   int64_t p_head_sigma, p_head_rgb, packed_bytes;
-  // fp32, the reference topology only (-1 otherwise): A operands of the forward
-  // on the FP16 matrix cores, each weight split into two fp16 planes.  Per layer
+  // fp32, the reference topology only (-1 otherwise): A operands of the forward on the
+  // BF16 matrix cores, each weight in three bf16 planes (mlp_split3.h).  Per layer
   // units [output block of 32][k-step of 16][plane][lane][8], the k-steps and their
   // order as in the bf16 form; the layers follow each other without gaps (fs_bytes
-  // from p_fs[0] on).  p_fse: int32 per layer and output block (NB apart), the
-  // power of two its weights are scaled by
-  int64_t p_fs[NERF_MAX_LAYERS], fs_bytes, p_fse;
-  // the same for the dX chain, layers m >= 1: A[n = input hidden feature][k = output
-  // feature], units [input block of 32][k-step of 16], bs_bytes from p_bs[1] on
+  // from p_fs[0] on)
+  int64_t p_fs[NERF_MAX_LAYERS], fs_bytes;
+  // for the dX chain, layers m >= 1: A[n = input hidden feature][k = output feature] in two
+  // fp16 planes, units [input block of 32][k-step of 16], bs_bytes from p_bs[1] on; p_bse:
+  // int32 per layer and block (NB apart), the power of two its weights are scaled by
   int64_t p_bs[NERF_MAX_LAYERS], bs_bytes, p_bse;
   int prec;
   // stash (elements per sample; fp32 or bf16 elements) and dz (floats per sample)
@@ -231,12 +231,9 @@ inline int mlp_make_plan(int D, int W, int skip, int LX, int LD, int prec, MlpPl
   const int64_t fs0 = b;
   for (int i = 0; i < P.n_mfma; ++i) {
     P.p_fs[i] = split ? b : -1;
-    if (split) b += (int64_t)((P.ks_hid[i] + P.ks_enc[i]) / 8) * P.nb_out[i] * 2 * 1024;
+    if (split) b += (int64_t)((P.ks_hid[i] + P.ks_enc[i]) / 8) * P.nb_out[i] * 3 * 1024;
   }
   P.fs_bytes = b - fs0;
-  align(256);
-  P.p_fse = split ? b : -1;
-  if (split) b += (int64_t)P.n_mfma * P.NB * 4;
   align(4096);
   const int64_t bs0 = b;
   for (int i = 0; i < P.n_mfma; ++i) {
