@@ -983,7 +983,6 @@ int launch_bwd_f32(const MlpPlan& P, const void* packed, int64_t M, const float*
                    const float* d_sigma, const float* rgb, const float* sigma, const void* stash,
                    void* dz, hipStream_t s) {
   if constexpr (W == 256 && LD > 0 && SKIP >= 0 && SKIP + 1 < D) {
-    // the reference topology: the register-resident chain (16 samples per wave)
     launch_bwd_f32s<W, D, SKIP, LX, LD>(P, packed, M, d_rgb, d_sigma, rgb, sigma, stash, dz, s);
   } else {
     const int64_t nblk = (M + 31) / 32;

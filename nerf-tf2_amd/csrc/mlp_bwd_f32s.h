@@ -1,45 +1,44 @@
-// FP32 dX chain of the reference topology (W = 256 with the rgb branch) on the FP16
-// matrix cores (mlp_f32s.h): the backward twin of mlp_fwd_f32s.h.
+// FP32 dX chain of the reference topology (W = 256 with the rgb branch) on the BF16
+// matrix cores (mlp_split3.h): the backward twin of mlp_fwd_f32s.h.
 //
 // dh_{l-1} = W_l[:W] dz_l: wave w of a workgroup owns input block w (32 features)
 // of every layer, the k-steps run over the layer's outputs, dz_l sits in LDS as
-// split B operands under each sample's own scale (gradients differ by many powers
-// of two from sample to sample), the transposed weights stream from L2.  The ReLU
-// masks are the forward's 16-bit words, one 16-byte load per lane and sample block
-// for the whole trunk; every dz row is written in FP32 for the weight GEMMs through
-// a buffer resource over the workgroup's rows (rows past M fall outside it).  Two
-// workgroups share a CU (N = 2); N = 1 where the samples do not fill the chip, the
-// forward's rule.
+// split B operands, the transposed weights stream from L2.  The ReLU masks are the
+// forward's 16-bit words, one 16-byte load per lane and sample block for the whole
+// trunk; every dz row is written in FP32 for the weight GEMMs through a buffer
+// resource over the workgroup's rows (rows past M fall outside it).  One workgroup
+// fills a CU with N = 2; N = 1 where the samples do not fill the chip, the forward's
+// rule.
 //
-// Bound by power and by the dz stores (9.9 KB a sample, 2.7 TB/s of them at the time
-// below).  Against the register-resident v_mfma_f32_16x16x4f32 kernel it replaced:
-// 6,570 -> 2,850 us at 786,432 samples, 1,665 -> 680 at 192,064, 188 -> 40 at 8,192, 142
-// -> 31 at 1,000; the dz rows' error against 64 bits 6.3e-7 -> 3.9e-7 of their norm at
-// the last layer (h0), 3.1e-7 -> 1.7e-7 at the first of 256 inputs.
+// Bound by power and by the dz stores (9.9 KB a sample).  Against the register-resident
+// v_mfma_f32_16x16x4f32 kernel that it replaced: 6,570 -> 4,580 us at 786,432 samples
+// (1,150 TFLOP/s of BF16 work), 1,665 -> 1,110 at 192,064, 188 -> 53 at 8,192, 142 -> 39 at
+// 1,000; the dz rows' error against 64 bits 5.5e-7 -> 1.8e-7 of their norm at the last layer
+// (h0), 1.6e-7 -> 0.8e-7 at the first of 256 inputs.  (Two FP16 parts under a scale per sample
+// took 2,800 us and were at 3.5e-7; cotangents below 2^-93 came out too large, and features
+// of unlike size lost the small ones.)
 //   rgb = sigmoid(z):  dz_rgb = d_rgb * rgb (1 - rgb)
 //   sigma = relu(z):   dz_sigma = d_sigma * [sigma > 0]
 //   dz = dh * [h > 0] for the ReLU layers; the bottleneck is linear.
 #pragma once
-#include "mlp_f32s.h"
+#include "mlp_split3.h"
 
 template <int W, int D, int SKIP, int LX, int LD, int N>
-__global__ __launch_bounds__(512, 4) void mlp_bwd_f32s_kernel(
+__global__ __launch_bounds__(512, 2) void mlp_bwd_f32s_kernel(
     MlpPlan P, const char* __restrict__ pk, int64_t M, const float* __restrict__ d_rgb,
     const float* __restrict__ d_sigma, const float* __restrict__ rgb, const float* __restrict__ sigma,
     const float* __restrict__ stash, float* __restrict__ dz) {
-  using namespace f32s;
+  using namespace split3;
   using C = NetC<W, D, SKIP, LX, LD>;
   static_assert(W == 256 && D == 8 && C::NBR == 4 && (N == 1 || N == 2), "split kernel is for the 8x256 NeRF MLP");
-  constexpr int AR = N == 1 ? 4 : 3, BR = N == 1 ? 2 : 1;  // as in the forward
+  constexpr int AR = N == 1 ? 6 : 4, BR = 2;               // as in the forward
   constexpr int TR = 2 * C::NBR;                           // k-steps over the rgb branch's outputs
-  __shared__ half8 s_tile[N][kTH * 128];    // 32 KB per sample block: dz of the layer above
-  __shared__ float s_max[N][kWaves * 32];   // its largest magnitudes per block and sample
+  __shared__ bf16x8 s_tile[N][kTH * kStep];  // 48 KB per sample block: dz of the layer above
   const int lane = threadIdx.x & 63, j = lane & 31, g = lane >> 5;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t base = (int64_t)blockIdx.x * (32 * N);
   const __amdgpu_buffer_rsrc_t rs = ws::packed_rsrc(pk + P.p_bs[1], P.bs_bytes);
   const uint32_t lane_off = 16u * (uint32_t)lane;
-  const int* wexp = reinterpret_cast<const int*>(pk + P.p_bse);  // weight scales [layer][input block]
   auto unit0 = [&](int l) -> int64_t { return P.p_bs[l] - P.p_bs[1] + (int64_t)wv * (l == D + 1 ? TR : kTH) * kUnit; };
   Planes a[AR];
 #pragma unroll
@@ -68,39 +67,29 @@ __global__ __launch_bounds__(512, 4) void mlp_bwd_f32s_kernel(
     const int64_t m = base + 32 * n + j;
     dzs[n] = m < M && sigma[m] > 0.f ? d_sigma[m] : 0.f;
   }
-  lds_h8* tile[N];
+  lds_b8* tile[N];
 #pragma unroll
-  for (int n = 0; n < N; ++n) tile[n] = lds_lane(s_tile[n], lane);
-  floatx16 hi[N], lo[N];
-  int se[N];
+  for (int n = 0; n < N; ++n) tile[n] = ws::lds_lane(s_tile[n], 0, lane);
+  Acc acc[N];
 
-  // v = this wave's block of dz for sample block n: k-steps 2 blk, 2 blk + 1 of the tile
-  auto put_tile = [&](const floatx16& v, int n, int blk, float sc) {
+  // v = this wave's block of dz for a sample block: k-steps 2 blk, 2 blk + 1 of its tile
+  auto put_tile = [&](const floatx16& v, lds_b8* to, int blk) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       float x[8];
 #pragma unroll
       for (int i = 0; i < 8; ++i) x[i] = v[8 * h + i];
-      const Planes p = split8(x, sc);
-      lds_h8* o = tile[n] + (2 * blk + h) * 128;
-      o[0] = p.h;
-      o[64] = p.l;
+      put_step(to + (2 * blk + h) * kStep, split8(x));
     }
-  };
-  auto max_abs = [](const floatx16& v) {
-    float mx = 0.f;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) mx = fmaxf(mx, fabsf(v[i]));
-    return mx;
   };
 
   // ---- rgb head: dh_rbr[f] = sum_c W_rgb[f][c] dz_rgb[c], masked; wave w does output block
-  // w % 4 of sample block w / 4 (the other blocks' largest values are 0)
+  // w % 4 of sample block w / 4
   {
     const int n = N == 1 ? 0 : wv >> 2, nb = wv & 3;
     const bool own = wv < 4 * N;
-    floatx16 v;
     if (own) {
+      floatx16 v;
       const int64_t m = base + 32 * n + j;
       float dzr[3] = {0.f, 0.f, 0.f};
       if (m < M) {
@@ -128,20 +117,7 @@ __global__ __launch_bounds__(512, 4) void mlp_bwd_f32s_kernel(
         v[i] = (mr >> i) & 1u ? d : 0.f;
       }
       store_block(v, n, P.dz_rbr + 32 * nb);
-      // (a sample block's four waves are w = 4 n .. 4 n + 3: slots nb and 4 + nb of its maxima)
-      const float mx = max_abs(v);
-      put_max((lds_f*)s_max[n], nb, j, g, mx);
-      put_max((lds_f*)s_max[n], 4 + nb, j, g, mx);
-    }
-    lds_barrier();
-#pragma unroll
-    for (int k = 0; k < N; ++k) se[k] = scale_exp(get_max((const lds_f*)s_max[k], j));
-    if (own) {
-      const float sc = pow2(n ? se[N - 1] : se[0]);
-      if (n)
-        put_tile(v, N - 1, nb, sc);
-      else
-        put_tile(v, 0, nb, sc);
+      put_tile(v, n ? tile[N - 1] : tile[0], nb);
     }
     lds_barrier();
   }
@@ -151,42 +127,38 @@ __global__ __launch_bounds__(512, 4) void mlp_bwd_f32s_kernel(
   constexpr auto ring0 = [](int s) { return s == 0 ? 0 : (TR + (s - 1) * kTH) % AR; };
   ws::static_for<0, D + 1>([&](auto Sc) {
     constexpr int s = decltype(Sc)::value, l = D + 1 - s, R = ring0(s);
-    const int we = wexp[l * C::NB + wv];
-    zero(hi);
-    zero(lo);
-    steps<N, s == 0 ? TR : kTH, R, AR, BR>(a, hi, lo, tile, rs, lane_off, unit0(l), unit0(l > 1 ? l - 1 : 1));
+#pragma unroll
+    for (int n = 0; n < N; ++n) zero(acc[n]);
+    constexpr int T = s == 0 ? TR : kTH;
+    steps<N, T, T, R, AR, BR>(a, acc, tile, tile, rs, lane_off, unit0(l), unit0(l > 1 ? l - 1 : 1));
     const int64_t el = (l == D + 1 ? P.dz_bott : P.dz_h[l - 1]) + 32 * wv;
 #pragma unroll
     for (int n = 0; n < N; ++n) {
-      const float f = inv_scale(se[n], we);
+      floatx16& v = acc[n].h;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) hi[n][i] = (hi[n][i] + lo[n][i]) * f;
+      for (int i = 0; i < 16; ++i) v[i] = sum(acc[n], i);
       if constexpr (l == D) {  // + W_sigma dz_sigma
         const floatx4* hs = reinterpret_cast<const floatx4*>(pk + P.p_head_sigma) + (g * C::KH + 16 * wv) / 4;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const floatx4 w = hs[q];
 #pragma unroll
-          for (int r = 0; r < 4; ++r) hi[n][4 * q + r] = hi[n][4 * q + r] + w[r] * dzs[n];
+          for (int r = 0; r < 4; ++r) v[4 * q + r] = v[4 * q + r] + w[r] * dzs[n];
         }
       }
       if constexpr (l <= D) {
         const uint32_t w = mw[n][(l - 1) >> 1];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) hi[n][i] = (w >> (16 * ((l - 1) & 1) + i)) & 1u ? hi[n][i] : 0.f;
+        for (int i = 0; i < 16; ++i) v[i] = (w >> (16 * ((l - 1) & 1) + i)) & 1u ? v[i] : 0.f;
       }
-      if constexpr (l > 1) put_max((lds_f*)s_max[n], wv, j, g, max_abs(hi[n]));
     }
-    lds_barrier();  // every wave has read the tile; the largest values are there
+    lds_barrier();  // every wave has read the tile
 #pragma unroll
     for (int n = 0; n < N; ++n)
-      store_rows(hi[n], tile[n] + 2 * wv * 128, lane, rdz, n * blk_z + (uint32_t)(4 * el), row_bytes);
+      store_rows(acc[n].h, tile[n] + 2 * wv * kStep, lane, rdz, n * blk_z + (uint32_t)(4 * el), row_bytes);
     if constexpr (l > 1) {
 #pragma unroll
-      for (int n = 0; n < N; ++n) {
-        se[n] = scale_exp(get_max((const lds_f*)s_max[n], j));
-        put_tile(hi[n], n, wv, pow2(se[n]));
-      }
+      for (int n = 0; n < N; ++n) put_tile(acc[n].h, tile[n], wv);
       lds_barrier();
     }
   });
@@ -197,7 +169,7 @@ void launch_bwd_f32s(const MlpPlan& P, const void* packed, int64_t M, const floa
                      const float* rgb, const float* sigma, const void* stash, void* dz, hipStream_t s) {
   auto go = [&](auto Nc) {
     constexpr int N = decltype(Nc)::value;
-    mlp_bwd_f32s_kernel<W, D, SKIP, LX, LD, N><<<(unsigned)((M + 32 * N - 1) / (32 * N)), 64 * f32s::kWaves, 0, s>>>(
+    mlp_bwd_f32s_kernel<W, D, SKIP, LX, LD, N><<<(unsigned)((M + 32 * N - 1) / (32 * N)), 64 * split3::kWaves, 0, s>>>(
         P, reinterpret_cast<const char*>(packed), M, d_rgb, d_sigma, rgb, sigma,
         reinterpret_cast<const float*>(stash), reinterpret_cast<float*>(dz));
   };

@@ -2,15 +2,12 @@
 // and the size queries of the MLP entry points.
 #include "common.h"
 #include "mlp_plan.h"
-#include "mlp_f32s.h"
 #include "mlp_split3.h"
 #include "optim.h"
 
 namespace {
 
 typedef float floatx4_a4 __attribute__((ext_vector_type(4), aligned(4)));  // the caller's weights: any float alignment
-
-constexpr int kSplitFloats = 32 * 257;  // a block of the widest split layer (256 outputs)
 
 // Input row (of the Keras kernel) fed by fp32 k-step s on lane half g of MFMA layer m.
 __device__ int fwd_row_f32(const MlpPlan& P, int m, int s, int g) {
@@ -42,13 +39,22 @@ struct PackModels {
   const float* flat[kOptModels];
   char* packed[kOptModels];
 };
-enum PackKind : int { kFwd, kBwd, kBias, kHeads, kSplitBwd };
+enum PackKind : int { kFwd, kBwd, kBias, kHeads };
 constexpr int kMaxSegs = 3 * NERF_MAX_LAYERS + 1;
 struct PackSegs {
   int n;
   int first[kMaxSegs + 1];  // first workgroup of each segment; [n]: their number
   unsigned char kind[kMaxSegs], layer[kMaxSegs];
 };
+
+// This lane's slots of unit w of a layer's split operands.
+__device__ __forceinline__ void put_split(const float (&f)[8], char* to, int w, int lane) {
+  bf16x8* o = reinterpret_cast<bf16x8*>(to) + w * split3::kStep + lane;
+  const split3::Planes p = split3::split8(f);
+  o[0] = p.h;
+  o[64] = p.m;
+  o[128] = p.l;
+}
 
 // Forward A operands of MFMA layer m: a wave writes unit w = (k-step or k-step group,
 // output block; the split form: output block, k-step), 16 bytes per lane and plane.  The
@@ -81,14 +87,7 @@ __device__ void pack_fwd(const MlpPlan& P, const float* __restrict__ flat, char*
 #pragma unroll
       for (int r = 0; r < 8; ++r) f[r] = kernel_at(P, flat, kl, fwd_row_bf16(P, m, t, r, g), col);
     }
-    if (split) {
-      bf16x8* o = reinterpret_cast<bf16x8*>(out + P.p_fs[m]) + w * split3::kStep + lane;
-      const split3::Planes p = split3::split8(f);
-      o[0] = p.h;
-      o[64] = p.m;
-      o[128] = p.l;
-      return;
-    }
+    if (split) return put_split(f, out + P.p_fs[m], w, lane);
     ushortx8 v;
 #pragma unroll
     for (int r = 0; r < 8; ++r) v[r] = f2bf(f[r]);
@@ -99,18 +98,21 @@ __device__ void pack_fwd(const MlpPlan& P, const float* __restrict__ flat, char*
 // Backward (transposed) A operands: A[n = input hidden feature 32 nb + j][k = output feature],
 // a unit per wave as above; a lane's outputs are one or two runs of four consecutive weights.
 __device__ void pack_bwd(const MlpPlan& P, const float* __restrict__ flat, char* __restrict__ out, int m, int w) {
-  const int kl = P.keras_of[m], lane = threadIdx.x & 63, j = lane & 31, g = lane >> 5, nb = w % P.NB, t = w / P.NB;
+  const int kl = P.keras_of[m], lane = threadIdx.x & 63, j = lane & 31, g = lane >> 5, T = 2 * P.nb_out[m];
+  const bool split = P.p_bs[m] >= 0;
+  const int nb = split ? w / T : w % P.NB, t = split ? w % T : w / P.NB;
   const int FO = P.fan_out[kl];
   const float* k = flat + P.k_off[kl] + (int64_t)(32 * nb + j) * FO;
   auto run = [&](int c) -> floatx4 {  // (FO is a multiple of 4: a run is inside or outside)
     return c < FO ? (floatx4)*reinterpret_cast<const floatx4_a4*>(k + c) : floatx4{0.f, 0.f, 0.f, 0.f};
   };
-  if (P.prec == 0) {
-    if (t >= 4 * P.nb_out[m]) return;
+  if (P.prec == 0 && !split) {
+    if (t >= 2 * T) return;
     reinterpret_cast<floatx4*>(out + P.p_bwd[m])[w * 64 + lane] = run(cfeat(t / 4, 4 * (t % 4), g));
   } else {
-    if (t >= 2 * P.nb_out[m]) return;
+    if (nb >= P.NB || t >= T) return;
     const floatx4 lo = run(16 * t + 4 * g), hi = run(16 * t + 4 * g + 8);  // cfeat(t / 2, 8 (t % 2) + r, g)
+    if (split) return put_split({lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]}, out + P.p_bs[m], w, lane);
     ushortx8 v;
 #pragma unroll
     for (int r = 0; r < 8; ++r) v[r] = f2bf(r < 4 ? lo[r & 3] : hi[r & 3]);
@@ -137,65 +139,13 @@ __device__ void pack_heads(const MlpPlan& P, const float* __restrict__ flat, cha
   }
 }
 
-// The scale exponent of a workgroup's weights, mx each thread's largest; orders its LDS writes.
-__device__ int split_scale(float mx, float* s_m) {
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) mx = fmaxf(mx, shfl_xor(mx, d));
-  if ((threadIdx.x & 63) == 0) s_m[threadIdx.x >> 6] = mx;
-  __syncthreads();
-  return f32s::scale_exp(fmaxf(fmaxf(s_m[0], s_m[1]), fmaxf(s_m[2], s_m[3])), 60);
-}
-
-// Split operands of the dX chain, one workgroup per input block nb: its 32 rows of fan_out (128 or
-// 256) weights go to LDS (one read of the weights, all loads in flight together) one float apart,
-// so that 32 lanes read 32 rows without bank conflicts; the largest gives the block's scale, and
-// each thread writes 16-byte chunks: the 8 slots of lane (j, g) of k-step t in unit nb T + t, planes
-// 1 KB apart.
-__device__ void pack_split_bwd(const MlpPlan& P, const float* __restrict__ flat, char* __restrict__ out, int m,
-                               int nb, float* s_w, float* s_m) {
-  const int kl = P.keras_of[m], T = 2 * P.nb_out[m], FO = P.fan_out[kl], V = FO / 128;  // float4s per thread and 4 rows
-  const float* w = flat + P.k_off[kl] + (int64_t)32 * nb * FO;
-  floatx4 v4[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-    v4[i] = i < 4 * V ? (floatx4)*reinterpret_cast<const floatx4_a4*>(w + 4 * (i * 256 + threadIdx.x)) : floatx4{0.f, 0.f, 0.f, 0.f};
-  float mx = 0.f;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    if (i >= 4 * V) break;
-    const int e = 4 * (i * 256 + threadIdx.x);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      s_w[(e / FO) * (FO + 1) + e % FO + r] = v4[i][r];
-      mx = fmaxf(mx, fabsf(v4[i][r]));
-    }
-  }
-  const int s = split_scale(mx, s_m);
-  if (threadIdx.x == 0) reinterpret_cast<int*>(out + P.p_bse)[m * P.NB + nb] = s;
-  const float sc = f32s::pow2(s);
-  const int j = threadIdx.x & 31, g = (threadIdx.x >> 5) & 1;
-  f32s::half8* o = reinterpret_cast<f32s::half8*>(out + P.p_bs[m]) + (int64_t)nb * T * 128 + (threadIdx.x & 63);
-  for (int t = threadIdx.x >> 6; t < T; t += 4) {
-    float v[8];
-#pragma unroll
-    for (int r = 0; r < 8; ++r) v[r] = s_w[j * (FO + 1) + cfeat(t / 2, 8 * (t % 2) + r, g)];
-    const f32s::Planes p = f32s::split8(v, sc);
-    o[t * 128] = p.h;
-    o[t * 128 + 64] = p.l;
-  }
-}
-
 // blockIdx.y: the model (all of one plan).  The first thread of the last launch of an optimizer
-// step also closes the step (state; null otherwise).  SPLIT: plans with split operands, whose
-// 33 KB of LDS would keep the others at four workgroups a CU, two rounds of them.
-template <bool SPLIT>
+// step also closes the step (state; null otherwise).
 __global__ __launch_bounds__(256) void pack_kernel(MlpPlan P, PackSegs S, PackModels A, StepState* state,
                                                    StepEnd end) {
   const float* __restrict__ flat = A.flat[blockIdx.y];
   char* __restrict__ out = A.packed[blockIdx.y];
   if (state && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) step_end(state, end);
-  __shared__ float s_w[SPLIT ? kSplitFloats : 1];
-  __shared__ float s_m[4];
   int seg = 0;
   while (seg + 1 < S.n && (int)blockIdx.x >= S.first[seg + 1]) ++seg;
   const int blk = blockIdx.x - S.first[seg], m = S.layer[seg], u = 256 * blk + threadIdx.x;
@@ -210,9 +160,6 @@ __global__ __launch_bounds__(256) void pack_kernel(MlpPlan P, PackSegs S, PackMo
       return;
     }
     case kHeads: return pack_heads(P, flat, out);
-    case kSplitBwd:
-      if constexpr (SPLIT) pack_split_bwd(P, flat, out, m, blk, s_w, s_m);
-      return;
   }
 }
 
@@ -227,12 +174,9 @@ PackSegs pack_segs(const MlpPlan& P) {
   };
   auto blocks16 = [](int64_t bytes) { return (bytes + 4095) / 4096; };  // 16 bytes per thread
   for (int m = 0; m < P.n_mfma; ++m) {
-    if (P.p_bs[m] >= 0) add(kSplitBwd, m, P.NB);
-  }
-  for (int m = 0; m < P.n_mfma; ++m) {
     const int T = (P.ks_hid[m] + P.ks_enc[m]) / 8;
     add(kFwd, m, blocks16((int64_t)P.nb_out[m] * 64 * 16 * (P.p_fwd[m] >= 0 && P.prec == 0 ? 2 * T : T)));
-    if (P.p_bwd[m] >= 0) add(kBwd, m, blocks16((int64_t)P.nb_out[m] * (P.prec == 0 ? 4 : 2) * P.NB * 64 * 16));
+    if (m > 0) add(kBwd, m, blocks16((int64_t)P.nb_out[m] * (P.p_bwd[m] >= 0 && P.prec == 0 ? 4 : 2) * P.NB * 64 * 16));
   }
   for (int m = 0; m < P.n_mfma; ++m) add(kBias, m, (32 * P.nb_out[m] + 255) / 256);
   add(kHeads, 0, 1);
@@ -250,8 +194,7 @@ void pack_models(const MlpPlan& P, int n, const float* const* flat, void* const*
     A.flat[i] = flat[i];
     A.packed[i] = reinterpret_cast<char*>(packed[i]);
   }
-  const auto k = P.fs_bytes + P.bs_bytes > 0 ? pack_kernel<true> : pack_kernel<false>;
-  k<<<dim3((unsigned)S.first[S.n], (unsigned)n), 256, 0, s>>>(P, S, A, state, end);
+  pack_kernel<<<dim3((unsigned)S.first[S.n], (unsigned)n), 256, 0, s>>>(P, S, A, state, end);
 }
 
 int nerf_plan_from_desc(const nerf_mlp_desc* d, int prec, MlpPlan* p) {

@@ -74,10 +74,9 @@ struct MlpPlan {
   // order as in the bf16 form; the layers follow each other without gaps (fs_bytes
   // from p_fs[0] on)
   int64_t p_fs[NERF_MAX_LAYERS], fs_bytes;
-  // for the dX chain, layers m >= 1: A[n = input hidden feature][k = output feature] in two
-  // fp16 planes, units [input block of 32][k-step of 16], bs_bytes from p_bs[1] on; p_bse:
-  // int32 per layer and block (NB apart), the power of two its weights are scaled by
-  int64_t p_bs[NERF_MAX_LAYERS], bs_bytes, p_bse;
+  // the same for the dX chain, layers m >= 1: A[n = input hidden feature][k = output
+  // feature], units [input block of 32][k-step of 16], bs_bytes from p_bs[1] on
+  int64_t p_bs[NERF_MAX_LAYERS], bs_bytes;
   int prec;
   // stash (elements per sample; fp32 or bf16 elements) and dz (floats per sample)
   int64_t st_encx, st_h[NERF_MAX_LAYERS], st_bott, st_rbr, st_encd, stash_per_sample;
@@ -238,12 +237,9 @@ inline int mlp_make_plan(int D, int W, int skip, int LX, int LD, int prec, MlpPl
   const int64_t bs0 = b;
   for (int i = 0; i < P.n_mfma; ++i) {
     P.p_bs[i] = split && i > 0 ? b : -1;
-    if (split && i > 0) b += (int64_t)P.nb_out[i] * 2 * P.NB * 2 * 1024;
+    if (split && i > 0) b += (int64_t)P.nb_out[i] * 2 * P.NB * 3 * 1024;
   }
   P.bs_bytes = b - bs0;
-  align(256);
-  P.p_bse = split ? b : -1;
-  if (split) b += (int64_t)P.n_mfma * P.NB * 4;
   align(256);
   P.packed_bytes = b;
   // stash (elements per sample)

@@ -84,3 +84,47 @@ def test_values_pass_through_a_permutation(nerf, k):
     _, _, stash = _forward(mlp, w)
     h2, h3 = stash[:, 64 + 512:64 + 768], stash[:, 64 + 768:64 + 1024]
     assert bool((h2 > 0).any()) and torch.equal(h3, h2[:, torch.from_numpy(perm).to(DEV)] * 2.0 ** k)
+
+
+def _dz_rows(nerf, mlp, w, shift=0, m=M):
+    """dz rows of the net for cotangents of ordinary size times 2^shift."""
+    import ctypes
+    L = nerf._lib
+    rgb, sigma, stash = _forward(mlp, w, m)
+    g = torch.Generator(device=DEV).manual_seed(11)
+    g_rgb = torch.randn((m, 3), generator=g, device=DEV) * 2.0 ** shift
+    g_sigma = torch.randn((m, 1), generator=g, device=DEV) * 2.0 ** shift
+    dz = torch.full((m, mlp.dz_per_sample), float("nan"), device=DEV)
+    L.call("nerf_mlp_backward", ctypes.byref(mlp._desc), mlp.prec, L.ptr(mlp.packed), m, L.ptr(g_rgb), L.ptr(g_sigma),
+           L.ptr(rgb), L.ptr(sigma), L.ptr(stash), L.ptr(dz), L.stream())
+    return dz[:, :9 * 256 + 128]
+
+
+DZ = {"plain": 2, "skip": 4, "rgb branch": 8}     # the layer's block of 256 dz columns
+
+
+@pytest.mark.parametrize("layer", list(LAYERS))
+@pytest.mark.parametrize("features", list(FEATURES))
+@pytest.mark.parametrize("k", [-60, -40, -24, 24, 40, 60])
+def test_rescaled_neurons_backward(nerf, layer, features, k):
+    mlp, w = _weights(nerf)
+    want = _dz_rows(nerf, mlp, w).clone()
+    cols = torch.from_numpy(256 * DZ[layer] + np.arange(256)[FEATURES[features]]).to(DEV)
+    want[:, cols] *= 2.0 ** -k
+    assert torch.equal(_dz_rows(nerf, mlp, rescale(w, layer, k, FEATURES[features])), want)
+
+
+@pytest.mark.parametrize("m", [33, 8211])      # one and two sample blocks a workgroup
+@pytest.mark.parametrize("k", [-115, -105, -95, -60, 60, 110])
+def test_backward_is_linear_in_its_cotangents(nerf, k, m):
+    """The same bits for cotangents times 2^k while no value leaves FP32's normal range; where small
+    ones do (k <= -95), rounded at 2^-149 as in FP32, each sample's rows to within a few 2^-24 of
+    their norm (values of 2^-115 to 2^-122: 2^-149 is at most 2^-27 of them)."""
+    mlp, w = _weights(nerf)
+    want = _dz_rows(nerf, mlp, w, 0, m).double()
+    got = _dz_rows(nerf, mlp, w, k, m).double() * 2.0 ** -k
+    if abs(k) <= 60 or k > 0:
+        assert torch.equal(got, want)
+    else:
+        err = (got - want).norm(dim=1)
+        assert bool((err <= 1e-6 * want.norm(dim=1)).all()), float((err / want.norm(dim=1)).max())
