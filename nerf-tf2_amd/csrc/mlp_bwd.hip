@@ -1055,100 +1055,115 @@ extern "C" int32_t nerf_mlp_backward(const nerf_mlp_desc* desc, int32_t precisio
   return NERF_OK;
 }
 
-// The fp32 launches: one for the heads (1 or 3 columns, by VALU), one for all other jobs,
-// with the smallest tile that holds each of them (mlp_wgrad_f32s.h).
-enum { kWgTile, kWgHead, kWg32Classes };
-static int wg32_class(const WgradJob& J) { return J.N == 1 || J.N == 3 ? kWgHead : kWgTile; }
-static int64_t wg32_job_floats(const WgradJob& J) { return (int64_t)J.K * J.N + (J.bias ? J.N : 0); }
-// Time per sample of a job (measured in the 8 x 8 tile, clocks per chunk: K = 256 7,500 and 7,200
-// with N = 256 and 128, K = 64 and 32 6,000): splitting takes all waves, whatever the layer has.
-static int wg32_job_cost(const WgradJob& J) { return 24 + (J.K + 63) / 64 * 2; }
-
-enum { kWg8x8, kWg8x4, kWg2x2 };
-static int wg32_shape(const WgradJob* jobs, int nj) {
-  int shape = kWg2x2;
-  for (int t = 0; t < nj; ++t) {
-    if (wg32_class(jobs[t]) != kWgTile) continue;
-    if (jobs[t].N > 128) return kWg8x8;
-    if (jobs[t].N > 64 || jobs[t].K > 64) shape = kWg8x4;
-  }
-  return shape;
+// The fp32 launches: jobs by tile shape (mlp_wgrad_f32s.h), one launch per shape;
+// the heads (1 or 3 columns) by VALU.
+enum { kWg8x4, kWg2x8, kWg2x4, kWg2x2, kWgHead, kWg32Classes };
+static int wg32_class(const WgradJob& J) {
+  if (J.N == 1 || J.N == 3) return kWgHead;
+  if (J.K > 64) return kWg8x4;
+  if (J.N > 128 || (J.N > 64 && J.K > 32)) return kWg2x8;
+  return J.N > 64 ? kWg2x4 : kWg2x2;
 }
+static int64_t wg32_job_floats(const WgradJob& J) { return (int64_t)J.K * J.N + (J.bias ? J.N : 0); }
+static int wg32_tiles(const WgradJob& J, int cls) { return cls == kWg8x4 ? (J.N + 127) / 128 : 1; }
 
-// Splits of each job, into sp: one round of workgroups (a CU holds 1, 1 or 3 of the shapes by
-// their LDS), shared out so that all take about the same time (a second round, a third full,
-// cost 7.1 ms where one takes 4.5: 786,432 samples of the 8x256 net); but at least 128 samples per split, and more rounds so that no split
-// sums over more than 8,192 samples (the rounding of one long sum), as far as the partial
-// tiles stay within the allocation-free entry point's static scratch; never so few that a
-// split's rows pass 2^31 bytes.  Heads: 1,024, of at least 64 samples.
-static void wg32_splits(const MlpPlan& P, int64_t M, const WgradJob* jobs, int nj, int64_t* sp) {
-  static const int per_cu[3] = {1, 1, 3};
-  const int64_t least =
-      wg16_min_splits(M, 4 * (P.stash_per_sample > P.dz_per_sample ? P.stash_per_sample : P.dz_per_sample));
-  int64_t blocks = 0, widest = 0, weight = 0;
+// Splits per job of a class: one round of workgroups (a CU holds 1, 1, 2 or 3 of the
+// shapes by their LDS), but at least 256 samples per split, and more rounds so that no
+// split sums over more than 8,192 samples (the rounding of one long sum), as far as the
+// class's partial tiles stay within the allocation-free entry point's static scratch; never
+// so few that a split's rows pass 2^31 bytes.  Heads: 1,024, of at least 64 samples.
+static int64_t wg32_splits(const MlpPlan& P, int64_t M, const WgradJob* jobs, int nj, int cls) {
+  static const int per_cu[kWg32Classes] = {1, 1, 2, 3, 0};
+  int64_t tiles = 0, floats = 0;
   for (int t = 0; t < nj; ++t)
-    if (wg32_class(jobs[t]) == kWgTile) {
-      const int64_t b = wg32_job_cost(jobs[t]);
-      blocks += b;
-      weight += b * wg32_job_floats(jobs[t]);
-      if (b > widest) widest = b;
+    if (wg32_class(jobs[t]) == cls) {
+      tiles += wg32_tiles(jobs[t], cls);
+      floats += wg32_job_floats(jobs[t]);
     }
-  int64_t groups = 256 * per_cu[wg32_shape(jobs, nj)];
-  const int64_t most = (int64_t)NERF_WGRAD_STATIC_SCRATCH_BYTES / 4 * blocks / weight;
-  const int64_t rounds = (M * blocks + groups * widest * 8192 - 1) / (groups * widest * 8192);
-  if (rounds * groups <= most) groups *= rounds;
-  else if (most > groups) groups = most / groups * groups;
-  else groups = most;
-  for (int t = 0; t < nj; ++t) {
-    const bool head = wg32_class(jobs[t]) == kWgHead;
-    const int64_t cap = (M + (head ? 63 : 127)) / (head ? 64 : 128);
-    int64_t s = head ? 1024 : groups * wg32_job_cost(jobs[t]) / blocks;
-    if (s > cap) s = cap;
-    if (s < least) s = least;
-    sp[t] = s < 1 ? 1 : s;
-  }
+  if (!tiles) return 1;
+  if (cls == kWgHead) return (M + 63) / 64 < 1024 ? (M + 63) / 64 : 1024;
+  const int64_t cap = (M + 255) / 256;
+  int64_t s = 256 * per_cu[cls] / tiles;
+  if (s < 1) s = 1;
+  const int64_t rounds = (M + s * 8192 - 1) / (s * 8192);
+  if (rounds > 1) s = 256 * per_cu[cls] * rounds / tiles;
+  const int64_t most = (int64_t)NERF_WGRAD_STATIC_SCRATCH_BYTES / 4 / floats;
+  if (s > most) s = most;
+  if (s > cap) s = cap;
+  const int64_t least = wg16_min_splits(M, 4 * (P.stash_per_sample > P.dz_per_sample ? P.stash_per_sample : P.dz_per_sample));
+  if (s < least) s = least;
+  return s < 1 ? 1 : s;
 }
 
 static int64_t wg32_floats(const MlpPlan& P, int64_t M, const WgradJob* jobs, int nj) {
-  int64_t sp[2 * NERF_MAX_LAYERS], f = 0;
-  wg32_splits(P, M, jobs, nj, sp);
-  for (int t = 0; t < nj; ++t) f += sp[t] * wg32_job_floats(jobs[t]);
+  int64_t f = 0;
+  for (int cls = 0; cls < kWg32Classes; ++cls) {
+    const int64_t sp = wg32_splits(P, M, jobs, nj, cls);
+    for (int t = 0; t < nj; ++t)
+      if (wg32_class(jobs[t]) == cls) f += sp * wg32_job_floats(jobs[t]);
+  }
   return f;
 }
 
-// One launch of n jobs of one class with sp[t] splits of job t, partial tiles job after job
-// from `part` on.
+// One launch of n jobs of class cls with sp splits, partial tiles job after job from `part` on.
 static void wg32_launch(const MlpPlan& P, int64_t M, const void* stash, const void* dz, const WgradJob* jobs,
-                        const int* members, int n, int shape, const int64_t* sp, float* part, hipStream_t s) {
-  wg32::Args a;
-  a.X = reinterpret_cast<const float*>(stash);
-  a.Z = reinterpret_cast<const float*>(dz);
-  a.ldx = P.stash_per_sample;
-  a.ldz = P.dz_per_sample;
-  a.M = M;
-  a.tiles = n;
-  const bool head = wg32_class(jobs[members[0]]) == kWgHead;
-  const int unit = head ? 1 : wg32::kChunk;
-  int first = 0;
-  for (int i = 0; i < n; ++i) {
-    const WgradJob& J = jobs[members[i]];
-    const int64_t k = sp[members[i]];
-    wg32::Tile& T = a.tile[i];
+                        const int* members, int n, int cls, int64_t sp, float* part, hipStream_t s) {
+  const float* X = reinterpret_cast<const float*>(stash);
+  const float* Z = reinterpret_cast<const float*>(dz);
+  auto tile = [&](const WgradJob& J, int n0, float* p) {
+    wg32::Tile T;
     T.xoff = (int)J.xoff;
     T.zoff = (int)J.zoff;
     T.K = J.K;
     T.N = J.N;
-    T.first = first;
-    T.m_per_split = (int)(((M + k - 1) / k + unit - 1) / unit * unit);
-    T.part = part;
-    T.bpart = J.bias ? part + k * J.K * J.N : nullptr;
-    part += k * wg32_job_floats(J);
-    first += (int)k;
+    T.n0 = n0;
+    T.part = p;
+    T.bpart = J.bias ? p + sp * J.K * J.N : nullptr;
+    return T;
+  };
+  if (cls == kWgHead) {
+    wg32::HeadArgs h;
+    h.X = X;
+    h.Z = Z;
+    h.ldx = P.stash_per_sample;
+    h.ldz = P.dz_per_sample;
+    h.M = M;
+    h.m_per_split = (int)((M + sp - 1) / sp);
+    h.splits = (int)sp;
+    for (int i = 0; i < n; ++i) {
+      h.tile[i] = tile(jobs[members[i]], 0, part);
+      part += sp * wg32_job_floats(jobs[members[i]]);
+    }
+    wg32::wgrad_head_kernel<<<(unsigned)(sp * n), 256, 0, s>>>(h);
+    return;
   }
-  if (head) wg32::wgrad_head_kernel<<<(unsigned)first, 256, 0, s>>>(a);
-  else if (shape == kWg8x8) wg32::wgrad_f32s_kernel<8, 8, 4, 2, 8, 5><<<(unsigned)first, 512, 0, s>>>(a);
-  else if (shape == kWg8x4) wg32::wgrad_f32s_kernel<8, 4, 2, 2, 16, 4><<<(unsigned)first, 512, 0, s>>>(a);
-  else wg32::wgrad_f32s_kernel<2, 2, 1, 1, 16, 4><<<(unsigned)first, 256, 0, s>>>(a);
+  wg32::Args a;
+  a.X = X;
+  a.Z = Z;
+  a.ldx = P.stash_per_sample;
+  a.ldz = P.dz_per_sample;
+  a.M = M;
+  a.m_per_split = (int)(((M + sp - 1) / sp + wg32::kChunk - 1) / wg32::kChunk * wg32::kChunk);
+  a.splits = (int)sp;
+  a.pairs = a.singles = 0;
+  wg32::Tile single[2 * NERF_MAX_LAYERS];
+  for (int i = 0; i < n; ++i) {
+    const WgradJob& J = jobs[members[i]];
+    if (wg32_tiles(J, cls) == 2) {
+      a.tile[2 * a.pairs] = tile(J, 0, part);
+      a.tile[2 * a.pairs + 1] = tile(J, 128, part);
+      ++a.pairs;
+    } else {
+      single[a.singles++] = tile(J, 0, part);
+    }
+    part += sp * wg32_job_floats(J);
+  }
+  for (int i = 0; i < a.singles; ++i) a.tile[2 * a.pairs + i] = single[i];
+  const unsigned grid = (unsigned)(16 * ((a.pairs * sp + 7) / 8) + a.singles * sp);
+  if (cls == kWg8x4) wg32::wgrad_f32s_kernel<8, 4, 2, 2><<<grid, 512, 0, s>>>(a);
+  else if (cls == kWg2x8) wg32::wgrad_f32s_kernel<2, 8, 2, 1><<<grid, 512, 0, s>>>(a);
+  else if (cls == kWg2x4) wg32::wgrad_f32s_kernel<2, 4, 2, 1><<<grid, 256, 0, s>>>(a);
+  else wg32::wgrad_f32s_kernel<2, 2, 1, 1><<<grid, 256, 0, s>>>(a);
 }
 
 // Partial-tile floats of the weight-gradient workspace: room for `s` tiles of the
@@ -1400,36 +1415,34 @@ static int32_t wgrad_run(const MlpPlan& P, int32_t precision, int64_t M, const v
       rb.njobs = 0;
       base = part;
     };
-    int64_t sp[2 * NERF_MAX_LAYERS];
-    wg32_splits(P, M, jobs, nj, sp);
     for (int cls = 0; cls < kWg32Classes; ++cls) {
+      const int64_t sp0 = wg32_splits(P, M, jobs, nj, cls);
       int t = 0;
       while (t < nj) {
         // the jobs of this class that fit the partial-tile buffer together
         int members[2 * NERF_MAX_LAYERS], n = 0;
-        int64_t used = base - part;
+        int64_t sp = sp0, used = base - part;
         for (; t < nj; ++t) {
           if (wg32_class(jobs[t]) != cls) continue;
           const int64_t f = wg32_job_floats(jobs[t]);
-          if (used + sp[t] * f > part_floats) {
+          if (used + sp * f > part_floats) {
             if (n || used) break;
-            sp[t] = part_floats / f;  // a job that does not fit by itself: fewer splits
+            sp = part_floats / f;  // a job that does not fit by itself: fewer splits
           }
-          used += sp[t] * f;
+          used += sp * f;
           members[n++] = t;
         }
         if (!n) {
           if (t < nj) flush();
           continue;
         }
-        wg32_launch(P, M, stash, dz, jobs, members, n, wg32_shape(jobs, nj), sp, base, s);
+        wg32_launch(P, M, stash, dz, jobs, members, n, cls, sp, base, s);
         for (int i = 0; i < n; ++i) {
           const WgradJob& J = jobs[members[i]];
-          const int64_t sj = sp[members[i]];
           const int k = rb.njobs++;
-          rb.job[k] = reduce_args(J, base, J.bias ? base + sj * J.K * J.N : nullptr, (int)sj);
-          rb.first[k + 1] = rb.first[k] + reduce_blocks(J, (int)sj);
-          base += sj * wg32_job_floats(J);
+          rb.job[k] = reduce_args(J, base, J.bias ? base + sp * J.K * J.N : nullptr, (int)sp);
+          rb.first[k + 1] = rb.first[k] + reduce_blocks(J, (int)sp);
+          base += sp * wg32_job_floats(J);
         }
         if (!stack) flush();
       }

@@ -128,3 +128,41 @@ def test_backward_is_linear_in_its_cotangents(nerf, k, m):
     else:
         err = (got - want).norm(dim=1)
         assert bool((err <= 1e-6 * want.norm(dim=1)).all()), float((err / want.norm(dim=1)).max())
+
+
+# a chunk of 32 samples is summed in FP32, chunks and splits after it: 2^-24 of the sum of |x| |z| each
+# time, a few of them; the six products leave out 2^-24 of a term at most
+TOL_SUM = 1e-6
+
+
+@pytest.mark.parametrize("width", [32, 128, 256])
+@pytest.mark.parametrize("m", [33, 4099])
+@pytest.mark.parametrize("spread", [40, 60, 120])
+def test_weight_grads_of_samples_of_unlike_size(nerf, width, m, spread):
+    """dz of every second sample is 2^-spread of the others', and half of the features are zero in
+    the large samples: their gradients are sums of small terms only, each as good as in FP32."""
+    import ctypes
+    L = nerf._lib
+    cfg = nerf.MLPConfig(depth=3, width=width, skip=-1)
+    mlp = nerf.NerfMLP("fine", cfg, "fp32", seed=1, device=DEV)
+    d = ctypes.byref(mlp._desc)
+    g = torch.Generator(device=DEV).manual_seed(m)
+    stash = torch.randn((m, mlp.stash_per_sample), generator=g, device=DEV).relu()
+    dz = torch.randn((m, mlp.dz_per_sample), generator=g, device=DEV)
+    odd = torch.arange(m, device=DEV)[:, None] % 2
+    dz *= 2.0 ** (spread // 2 - spread * odd)
+    stash[:, ::2] *= odd
+    work = torch.empty(int(L.load().nerf_mlp_wgrad_workspace_bytes(d, m)), dtype=torch.uint8, device=DEV)
+    grad = torch.full((mlp.n_params,), float("nan"), device=DEV)
+    L.call("nerf_mlp_weight_grads", d, 0, m, L.ptr(stash), L.ptr(dz), L.ptr(grad), 0, L.ptr(work), work.numel(),
+           L.stream())
+    enc, off = 2 * ((2 + 3 * cfg.l_xyz + 7) // 8 * 8), 0
+    for j, (name, fi, fo) in enumerate(cfg.layer_shapes()[:3]):
+        k = grad[off:off + fi * fo].view(fi, fo).cpu().double()
+        off += fi * fo + fo
+        if j == 0:
+            continue
+        x = stash[:, enc + (j - 1) * width:enc + j * width].cpu().double()
+        z = dz[:, j * width:(j + 1) * width].cpu().double()
+        err, most = (k - x.T @ z).abs(), x.T @ z.abs()
+        assert bool((err <= TOL_SUM * most).all()), (name, float((err / most).nan_to_num().max()))
