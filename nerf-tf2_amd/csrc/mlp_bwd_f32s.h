@@ -13,7 +13,7 @@
 // Bound by power and by the dz stores (9.9 KB a sample).  Against the register-resident
 // v_mfma_f32_16x16x4f32 kernel that it replaced: 6,570 -> 4,580 us at 786,432 samples
 // (1,150 TFLOP/s of BF16 work), 1,665 -> 1,110 at 192,064, 188 -> 53 at 8,192, 142 -> 39 at
-// 1,000; the dz rows' error against 64 bits 5.5e-7 -> 1.8e-7 of their norm at the last layer
+// 1,000; the dz rows' error against 64 bits 5.5e-7 -> 1.9e-7 of their norm at the last layer
 // (h0), 1.6e-7 -> 0.8e-7 at the first of 256 inputs.  (Two FP16 parts under a scale per sample
 // took 2,800 us and were at 3.5e-7; cotangents below 2^-93 came out too large, and features
 // of unlike size lost the small ones.)

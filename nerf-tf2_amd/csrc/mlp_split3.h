@@ -1,13 +1,15 @@
 // FP32 products on the BF16 matrix cores, for the 8x256 NeRF MLP.
 //
-// An FP32 operand is held exactly, as three bf16 numbers x = h + m / 2^7 + l / 2^14, each the
-// rounded remainder: 24 significant bits.  m and l are stored scaled up, so that all three have
-// about the exponent of x: every finite x of at least 2^-124 in magnitude is exact, whatever
+// An FP32 operand is held exactly, as three bf16 numbers x = h + m / 2^6 + l / 2^12: h the top
+// half of x's bits (so that an infinity stays one and no finite x becomes one), m and l the
+// rounded remainders, 24 significant bits.  m and l are stored scaled up, so that all three have
+// about the exponent of x: every finite x of at least 2^-122 in magnitude is exact, whatever
 // stands beside it (below that the last bits of l reach under bf16's range), and no scale is
 // needed for a sample, a feature or a block.  A product is the six partial products that reach
-// 2^-24 of it, in three FP32 accumulators of one order each, h h; m h + h m; l h + h l + m m,
-// added once per output, the small ones first (the three that are left out are below 2^-24 of
-// the product, 2^-27 on average).  An infinite or NaN operand makes its products NaN.
+// 2^-23 of it, in three FP32 accumulators of one order each, h h; m h + h m; l h + h l + m m,
+// added once per output, the small ones first (the three that are left out are below 2^-22 of
+// the product, 2^-25 on average).  An infinite or NaN operand makes the small sums NaN; the
+// large one alone is then what FP32's sum is.
 //
 // v_mfma_f32_32x32x16_bf16 does 16 times the work per cycle of the FP32 instruction, so the
 // six products take 3/8 of its time; and a sum is rounded once per 16 terms, not once per term.
@@ -28,20 +30,19 @@ constexpr int kWaves = 8;       // waves per workgroup: wave w owns output block
 constexpr int kUnit = 3072;     // bytes of one (output block, k-step): three planes of 1 KB
 constexpr int kStep = 3 * 64;   // bf16x8 of one k-step of a tile
 constexpr int kTH = 16;         // k-steps of a hidden input
-constexpr float kScale = 128.f; // of m against h and of l against m
+constexpr float kScale = 64.f;  // of m against h and of l against m: both stay below h, their sums in its range
 
 struct Planes {  // one k-step of an operand
   bf16x8 h, m, l;
 };
 
-// a and b in three parts.  h is held to the largest finite bf16, so that the few FP32 values
-// above it do not round to infinity.
+// a and b in three parts.
 __device__ __forceinline__ void split2(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
-  const float big = __builtin_bit_cast(float, 0x7F7F0000u);
   auto lo = [](uint32_t p) { return __builtin_bit_cast(float, p << 16); };
   auto up = [](uint32_t p) { return __builtin_bit_cast(float, p & 0xFFFF0000u); };
-  h = pack_bf16x2(__builtin_amdgcn_fmed3f(a, -big, big), __builtin_amdgcn_fmed3f(b, -big, big));
-  const float ra = fmul(fsub(a, lo(h)), kScale), rb = fmul(fsub(b, up(h)), kScale);
+  const uint32_t ua = __builtin_bit_cast(uint32_t, a), ub = __builtin_bit_cast(uint32_t, b);
+  h = __builtin_amdgcn_perm(ub, ua, 0x07060302u);
+  const float ra = fmul(fsub(a, up(ua)), kScale), rb = fmul(fsub(b, up(ub)), kScale);
   m = pack_bf16x2(ra, rb);
   l = pack_bf16x2(fmul(fsub(ra, lo(m)), kScale), fmul(fsub(rb, up(m)), kScale));
 }
@@ -74,9 +75,12 @@ __device__ __forceinline__ void zero(Acc& c) {
   for (int i = 0; i < 16; ++i) c.h[i] = c.m[i] = c.l[i] = 0.f;
 }
 
-__device__ __forceinline__ float sum(const Acc& c, int i) {
+__device__ __forceinline__ float sum_finite(const Acc& c, int i) {  // NaN or infinite where FP32's sum is either
   constexpr float k = 1.f / kScale;
   return __builtin_fmaf(__builtin_fmaf(c.l[i], k, c.m[i]), k, c.h[i]);
+}
+__device__ __forceinline__ float sum(const Acc& c, int i) {
+  return __builtin_fabsf(c.h[i]) < __builtin_inff() ? sum_finite(c, i) : c.h[i];
 }
 
 // Workgroup barrier that orders LDS only (global loads and stores stay in flight).

@@ -174,7 +174,7 @@ __global__ __launch_bounds__(64 * (KB / RK) * (NB / RN)) void wgrad_f32s_kernel(
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[x][y][i] += split3::sum(c, i);
+        for (int i = 0; i < 16; ++i) acc[x][y][i] += split3::sum_finite(c, i);
         asm volatile("" : "+v"(acc[x][y]));  // (added here, not sunk past the next block)
         __builtin_amdgcn_sched_barrier(0);
       }

@@ -166,3 +166,36 @@ def test_weight_grads_of_samples_of_unlike_size(nerf, width, m, spread):
         z = dz[:, j * width:(j + 1) * width].cpu().double()
         err, most = (k - x.T @ z).abs(), x.T @ z.abs()
         assert bool((err <= TOL_SUM * most).all()), (name, float((err / most).nan_to_num().max()))
+
+
+@pytest.mark.parametrize("m", [33, 8211])      # one and two sample blocks a workgroup
+@pytest.mark.parametrize("layer", [1, 4, 6])   # (4: the skip layer's input)
+def test_infinite_hidden_values(nerf, m, layer):
+    """A feature that passes FP32's range is infinite and stays so: the next layer's outputs are
+    infinite or zero by the sign of its weights, as the FP32 product of each of them is."""
+    mlp, w = _weights(nerf)
+    f = 77
+    w[2 * layer][:, f], w[2 * layer + 1][f] = 2.0 ** 127, 3.3e38   # infinite for any input above 0.1
+    w[22] = np.abs(w[22])
+    x, _ = _points(m)
+    _, sigma, stash = _forward(mlp, w, m)
+    h = lambda i: stash[:, 64 + 256 * i:64 + 256 * (i + 1)]
+    assert bool((h(layer)[:, f] == float("inf")).all())
+    sign = torch.from_numpy(np.sign(w[2 * layer + 2][f])).to(DEV)
+    assert bool((h(layer + 1)[:, sign > 0] == float("inf")).all()) and bool((h(layer + 1)[:, sign < 0] == 0).all())
+    if layer == 6:
+        assert bool((sigma == float("inf")).all())
+
+
+@pytest.mark.parametrize("top", [3.3e38, 3.4e38])   # within and above the largest bf16, 3.39e38
+def test_largest_finite_values_forward(nerf, top):
+    """Hidden values up to FP32's largest are finite inputs: the next layer's kernel takes them back."""
+    mlp, w = _weights(nerf)
+    f = 77
+    w[4][:, f], w[5][f] = 0.0, top                       # h2[f] = top for every sample
+    w[6][f] = np.sign(w[6][f]) * np.float32(2.0 ** -127)
+    _, _, stash = _forward(mlp, w)
+    h = lambda i: stash[:, 64 + 256 * i:64 + 256 * (i + 1)].cpu().double()
+    assert bool((h(2)[:, f] == float(np.float32(top))).all())
+    want = torch.relu(h(2) @ torch.from_numpy(w[6]).double() + torch.from_numpy(w[7]).double())
+    assert float((h(3) - want).norm()) <= 1e-6 * float(want.norm())
