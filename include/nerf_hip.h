@@ -321,7 +321,8 @@ int32_t nerf_step_end(nerf_step_state* state, int32_t interval, float factor, fl
 
 /* One optimizer step over any number of models: nerf_step_begin, with `check` nerf_check_finite of every
  * gradient's grad_n values (of the scaled loss), nerf_adam_tf_state and nerf_mlp_pack of every
- * model, nerf_step_end, in a few launches (8 models per launch) with the same results.  `models` is a host
+ * model, nerf_step_end, in a few launches (8 models per launch) with the same results; models that share
+ * parameters or moments are updated in their order, a launch each.  `models` is a host
  * array; reserved[0] of the state belongs to it between its launches. */
 typedef struct nerf_opt_model {
   const nerf_mlp_desc* desc; /* host */

@@ -276,11 +276,26 @@ extern "C" int32_t nerf_optimizer_step(int32_t n_models, const nerf_opt_model* m
   StepState* st = reinterpret_cast<StepState*>(state);
   const StepBegin sb{lr0, (float)decay_steps, decay_rate, b1, b2};
   const StepEnd se{interval, factor, min_scale, 1};
+  // models that share parameters or moments (one net listed twice) are updated one after the other
+  auto shares = [&](int i, int j) {
+    MlpPlan Pi, Pj;
+    nerf_plan_from_desc(models[i].desc, models[i].precision, &Pi);
+    nerf_plan_from_desc(models[j].desc, models[j].precision, &Pj);
+    const float* bi[3] = {models[i].params, models[i].m, models[i].v};
+    const float* bj[3] = {models[j].params, models[j].m, models[j].v};
+    for (const float* x : bi)
+      for (const float* y : bj)
+        if (x < y + Pj.n_params && y < x + Pi.n_params) return true;
+    return false;
+  };
   // models first, first + 1, .. of at most kOptModels per launch
   auto args = [&](int first, OptArgs& a, int& n, unsigned& gx) {
     a = OptArgs{};
     int64_t most = 0;
     for (n = 0; n < kOptModels && first + n < n_models; ++n) {
+      bool apart = true;
+      for (int k = 0; k < n && apart; ++k) apart = !shares(first + k, first + n);
+      if (!apart) break;
       const nerf_opt_model& M = models[first + n];
       nerf_plan_from_desc(M.desc, M.precision, &P);
       a.n[n] = P.n_params;
@@ -300,11 +315,11 @@ extern "C" int32_t nerf_optimizer_step(int32_t n_models, const nerf_opt_model* m
   int n = 0;
   unsigned gx = 1;
   if (check)
-    for (int i = 0; i == 0 || i < n_models; i += kOptModels) {  // (the first launch opens the step)
+    for (int i = 0; i == 0 || i < n_models; i += n ? n : 1) {  // (the first launch opens the step)
       args(i, a, n, gx);
       opt_check_kernel<<<dim3(gx, (unsigned)n + (i == 0)), 256, 0, s>>>(a, n, st, sb);
     }
-  for (int i = 0; i < n_models; i += kOptModels) {
+  for (int i = 0; i < n_models; i += n) {
     args(i, a, n, gx);
     opt_adam_kernel<<<dim3(gx, (unsigned)n), 256, 0, s>>>(a, eps, st, !check, sb);
   }
