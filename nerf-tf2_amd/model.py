@@ -397,6 +397,9 @@ class AdamTF:
             o.desc, o.precision = ctypes.pointer(mm._desc), mm.prec
             o.params, o.m, o.v, o.packed = ptr(mm.params), ptr(m), ptr(v), ptr(mm.packed)
             o.grad, o.grad_n = ptr(g), g.numel()
+        if scaler is not None:
+            for g in grads[len(models):]:                      # gradients of no model are checked all the same
+                call("nerf_check_finite", g.numel(), ptr(g), ptr(self.state) + 36, stream(self.state.device))  # reserved[0]
         end = (self._NEVER, 1.0, 1.0) if scaler is None else (scaler.interval, scaler.factor, scaler.min_scale)
         call("nerf_optimizer_step", len(keep) if scaler is None else min(len(models), len(grads)), models,
              self.initial_lr, self.decay_steps, self.decay_rate, float(self.b1), float(self.b2), float(self.eps),

@@ -38,3 +38,21 @@ def test_a_net_listed_twice_is_updated_twice(nerf, order, scaled):
         net.repack()
         assert torch.equal(net.packed, packed)
     assert all(torch.equal(a, b) for a, b in zip(opt.m + opt.v, ms + vs))
+
+
+@pytest.mark.parametrize("bad", [None, float("inf"), float("nan")])
+def test_gradients_past_the_models_are_checked(nerf, bad):
+    """With a scaler every gradient that is given is checked, those of no model too."""
+    net = nerf.NerfMLP("fine", nerf.MLPConfig(), "bf16", seed=1, device=DEV)
+    opt = nerf.AdamTF([net])
+    scaler = nerf.DynamicLossScaler(opt)
+    extra = torch.ones(1000, device=DEV)
+    if bad is not None:
+        extra[999] = bad
+    before = net.params.clone()
+    for step in (1, 2):
+        opt.apply_gradients([torch.ones(net.n_params, device=DEV), extra], scaler)
+        assert (opt.iterations, scaler.skipped) == ((step, 0) if bad is None else (0, step))
+    assert torch.equal(net.params, before) == (bad is not None)
+    opt.apply_gradients([torch.ones(net.n_params, device=DEV)], scaler)
+    assert opt.iterations == (3 if bad is None else 1)
