@@ -34,8 +34,8 @@ sys.path.insert(0, ROOT)
 
 METRIC = "rays/sec render & train (64+128 samples), learned vs plain at ≤0.1 dB PSNR"
 BF16_PEAK_TFLOPS = 2500.0
-# the FP32 form's products are three FP16 matrix products each (the FP32 matrix instruction: 157.3)
-FP32_PEAK_TFLOPS = 2500.0 / 3
+# the FP32 form's products are six BF16 matrix products each (the FP32 matrix instruction: 157.3)
+FP32_PEAK_TFLOPS = 2500.0 / 6
 HBM_PEAK_GBS = 8000.0
 MLP_FLOP_PER_SAMPLE = 2 * 593408          # both dense stacks of one model, per sample
 RENDER_FLOP_PER_RAY = (64 + 192) * MLP_FLOP_PER_SAMPLE
@@ -45,7 +45,7 @@ RENDER_FLOP_PER_RAY = (64 + 192) * MLP_FLOP_PER_SAMPLE
 # same counter on a 1 GiB device copy), from the rocprofv3 --pmc runs whose commands
 # and figures are in profiles/mlp_fwd_f32s_render800.md and
 # profiles/mlp_fwd_bf16ws8_render800.md.
-TRAFFIC_BYTES_PER_LAUNCH = {"fp32": 152.1e6, "bf16": 142.5e6}
+TRAFFIC_BYTES_PER_LAUNCH = {"fp32": 163.3e6, "bf16": 142.5e6}
 
 
 def parse():

@@ -1231,7 +1231,8 @@ static int wg16_groups(const MlpPlan& P, int64_t M, const WgradJob* jobs, int nj
   // group's or the allocation-free entry point's static scratch, whichever is
   // larger (so that entry point takes every batch it took before).  Narrow tiles
   // too: one workgroup's loads do not fill a CU's share of the bandwidth (720,896
-  // samples, 32 x 128 52 -> 43 us, 128 x 3 51 -> 38 us), and the sums over more splits
+  // samples, 32 x 128 52 -> 43 us, 128 x 3 51 -> 38 us by themselves, no difference in a whole
+  // backward pass), and the sums over more splits
   // take eight threads an element there (reduce_wide).
   int64_t most = (int64_t)NERF_WGRAD_STATIC_SCRATCH_BYTES / 4;
   for (int i = 0; i < ng; ++i) {

@@ -154,9 +154,10 @@ __global__ __launch_bounds__(512) void mlp_fwd_bf16ws8_kernel(
 
   // ---- encodings of sample block w % N; with four blocks, waves 0-3 the first three k-steps of
   // xyz, waves 4-7 the fourth and the direction's two.  Nothing runs beside this (one workgroup a
-  // CU), so its length counts: against six k-steps on four waves a render launch of 6,291,456
-  // samples takes 6.52 instead of 6.62 ms, one of 120,000 135 instead of 141 us.  (A 32-bit division
-  // for the ray behind a uniform one, instead of load_sample's, measured 0.5 % slower.)
+  // CU), so its length counts: against six k-steps on four waves one of 120,000 samples takes 133
+  // instead of 137 us; a render launch of 6,291,456 differs by less than two runs do (6.55 and 6.69
+  // ms, 2 %).  (A 32-bit division for the ray behind a uniform one, instead of load_sample's, measured
+  // 0.5 % slower.)
   {
     const int eb = wv % N;
     float x[3], d[3];

@@ -8,8 +8,9 @@
 // ends with the bias, the ReLU and, behind a barrier, the split values' stores
 // over the old tile.  One workgroup fills a CU with N = 2.
 //
-// What bounds it: power.  At 6,291,456 samples it takes 33.3 ms (224 TFLOP/s of FP32 work,
-// 1,345 of BF16 work, where a bare stream of the six products with random operands, LDS and
+// What bounds it: the matrix cores at the clock that they are held at (0.65 busy at 1.89 GHz).
+// At 6,291,456 samples it takes 32.9 to 34.1 ms (219 to 227 TFLOP/s of FP32 work, 1,310 to 1,360
+// of BF16 work, where a bare stream of the six products with random operands, LDS and
 // L2 reads runs at 1,250 to 1,450), against 51.0 ms of the register-resident
 // v_mfma_f32_16x16x4f32 kernel that it replaced.  (Two FP16 parts and three products took
 // 18.7 ms, without FP32's range: mlp_split3.h.)  Error against 64 bits, of the norm over 4,096
@@ -17,7 +18,7 @@
 // 0.45e-7 (0.73e-7).
 //
 // N = 1 halves a workgroup's serial time where the samples do not fill the chip, and doubles
-// the weights' traffic: M = 1,000 189 us (FP32 instruction) -> 37.8; N = 1 / 2: 38.3 / 70.9 us
+// the weights' traffic: M = 1,000 189 us (FP32 instruction) -> 39.8; N = 1 / 2: 38.3 / 70.9 us
 // at M = 4,096, 51.2 / 71.3 at 8,192, 87.4 / 74.9 at 12,000, 100.7 / 89.3 at 16,384, and with
 // the stash 59.7 / 82.0 at 8,192, 103.5 / 88.4 at 12,000, so N = 1 up to 32 samples per CU.
 #pragma once
